@@ -212,11 +212,12 @@ struct fsg_domain {
   int* counts = nullptr;
   int* offsets = nullptr;
   int* n_fluid = nullptr;
-  int* fluid_index = nullptr;
+  // the Jacobi-CG forms' unknowns (tile order): index per cell, cell per unknown; b per
+  // cell (every form), and per unknown in ap
+  int* index_of = nullptr;
   int* cell_of = nullptr;
-  // true: the last pressure solve compacted the system (fluid_index, and b per unknown
-  // index); false (multigrid form): b holds the reference's b per cell, and the fluid
-  // indices follow from the labels
+  // true: the last pressure solve indexed its unknowns in index_of; false (multigrid
+  // form): the fluid indices follow from the labels
   bool compacted = false;
   float* b = nullptr;
   uint8_t* info = nullptr;
@@ -224,12 +225,13 @@ struct fsg_domain {
   float* ap = nullptr;
   float* xg = nullptr;
   float* pg0 = nullptr;
-  int2* updn = nullptr;
-  float* exch = nullptr;
+  float* exch = nullptr;    // 3 C floats: the one-launch CG's tagged words (2 C of them)
   double* x64 = nullptr;
   double* partials = nullptr;
-  unsigned* bar = nullptr;
+  unsigned* bar = nullptr;  // [1]: a one-launch CG solve abandoned a wait
   CgScalars* sc = nullptr;
+  bool last_dev = false;    // the last solve's statistics are in sc (a one-launch CG form)
+  bool dev_totals = false;  // sc holds totals of such solves (since the last reset)
   HostScalars* hsc = nullptr;  // pinned host memory: the solve loop's readback
   bool mg_finish_pending = false;  // the next pressure update finishes the MG solve
   int max_coop_blocks = 0;  // co-resident 1024-thread blocks of the persistent solver
@@ -767,123 +769,157 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   return FSG_OK;
 }
 
+// The three-kernels-per-iteration form of the plain CG, in batches of check_every
+// iterations between stop-test reads: systems that the one-launch form cannot take.
+int plain_many_launches(fsg_domain* h, int F, const CgParams& cp) {
+  timed(h, "cg_init", [&] {
+    // b per unknown lies in ap until the first iteration writes it
+    launch_cg_init(h->stream, F, cp, h->cell_of, h->info, h->ap, h->r, h->pg0, h->xg, h->partials,
+                   h->sc);
+  });
+  const int check = h->prm.check_every > 0 ? h->prm.check_every : 32;
+  int launched = 0;
+  CgScalars hs{};
+  while (launched < cp.max_iter) {
+    const int n = std::min(check, cp.max_iter - launched);
+    for (int q = 0; q < n; ++q) {
+      const int it = launched + q;
+      timed(h, "cg_iteration", [&] {
+        launch_cg_iteration(h->stream, F, h->g.nx, it, cp, h->cell_of, h->info, h->r, h->ap,
+                            h->pg0, h->xg, h->partials, h->sc);
+      });
+    }
+    launched += n;
+    HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (hs.done) break;
+  }
+  if (cp.max_iter == 0) {
+    HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+  }
+  h->host_stats.cg_iterations = hs.iter;
+  h->host_stats.cg_error = hs.err;
+  h->host_stats.total_unknown_iterations += (int64_t)F * hs.spmv;
+  h->host_stats.total_solves += 1;
+  h->last_dev = false;
+  return FSG_OK;
+}
+
 int solve_pressure(fsg_domain* h) {
   h->mg_solved = false;
+  h->last_dev = false;
   h->host_stats.cg_iterations = 0;
   h->host_stats.cg_error = 0.0;
   h->host_stats.refine_sweeps = 0;
   const int solver = h->prm.solver;
   // the multigrid form's launches do not depend on the number of unknowns (a system
   // without any stops at its first test, and the pressure update reads the count on
-  // the device); it reads the count back with its stop test.  Its set-up forms the
-  // LIQUID count and the reference's b per cell itself: no compaction.
+  // the device); it reads the count back with its stop test.
   h->compacted = solver != FSG_SOLVER_MG;
   if (solver == FSG_SOLVER_MG) return mg_solve(h, -1, nullptr, true);
-  const int nb = (int)((ncell(h) + kScanChunk - 1) / kScanChunk);
-  timed(h, "count_liquid", [&] { launch_count_liquid(h->stream, h->g, h->label, h->counts); });
-  timed(h, "scan_counts", [&] { launch_scan_counts(h->stream, nb, h->counts, h->offsets, h->n_fluid); });
-  timed(h, "compact", [&] {
-    launch_compact(h->stream, h->g, h->label, h->offsets, h->fluid_index, h->cell_of, UF(h), VF(h),
-                   h->b, h->info);
+  timed(h, "pcg_setup", [&] {
+    launch_pcg_count(h->stream, h->g, h->label, h->counts);
+    launch_scan_counts(h->stream, pcg_tiles(h->g), h->counts, h->offsets, h->n_fluid);
+    launch_pcg_fill(h->stream, h->g, h->label, h->offsets, h->index_of, h->cell_of, UF(h), VF(h),
+                    h->ap, h->b, h->info);
   });
-  // the launch geometry of the other forms depends on the number of unknowns
-  int F = 0;
-  HIPCHK(h, hipMemcpyAsync(&F, h->n_fluid, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  h->host_stats.n_fluid = F;
-  h->last_F = F;
-  if (F == 0) return FSG_OK;
-  if (solver == FSG_SOLVER_PLAIN) {
-    const CgParams cp = make_cg_params(h, (float)h->prm.cg_tol);
-    timed(h, "cg_init", [&] {
-      launch_cg_init(h->stream, F, cp, h->cell_of, h->info, h->b, h->r, h->pg0, h->xg, h->partials,
-                     h->sc);
-    });
-    const int check = h->prm.check_every > 0 ? h->prm.check_every : 32;
-    int launched = 0;
-    CgScalars hs{};
-    while (launched < cp.max_iter) {
-      const int n = std::min(check, cp.max_iter - launched);
-      for (int q = 0; q < n; ++q) {
-        const int it = launched + q;
-        timed(h, "cg_iteration", [&] {
-          launch_cg_iteration(h->stream, F, h->g.nx, it, cp, h->cell_of, h->info, h->r, h->ap,
-                              h->pg0, h->xg, h->partials, h->sc);
-        });
-      }
-      launched += n;
-      HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-      if (hs.done) break;
-    }
-    if (cp.max_iter == 0) {
-      HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-    }
-    h->host_stats.cg_iterations = hs.iter;
-    h->host_stats.cg_error = hs.err;
-    h->host_stats.total_unknown_iterations += (int64_t)F * hs.spmv;
-    h->host_stats.total_solves += 1;
-    return FSG_OK;
+  const bool refined = solver == FSG_SOLVER_REFINED, plain = solver == FSG_SOLVER_PLAIN;
+  // Launch shape of the one-launch CG: G blocks of 512 threads, kpt x 1024 unknowns per
+  // block.  One block exchanges nothing and needs no cooperative launch, so it takes
+  // every system that fits its registers (1.0-2.6 us per iteration against 4.0-4.4 for
+  // the fewest blocks).  A grid of no more cells than that needs no count of its unknowns
+  // on the host either: the launch is sized by the cells and the step does not
+  // synchronise.
+  const int one_max = refined ? kPcgOneRefined : kPcgOneUnknowns;
+  const bool fixed = !plain && (h->prm.pcg_kpt > 0 || h->prm.pcg_blocks > 0);
+  const bool no_count = !fixed && ncell(h) <= (size_t)one_max;
+  int F = (int)ncell(h);
+  if (!no_count) {
+    HIPCHK(h, hipMemcpyAsync(&F, h->n_fluid, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->host_stats.n_fluid = F;
+    h->last_F = F;
+    if (F == 0) return FSG_OK;
   }
-  // persistent / refined: one cooperative launch, every iteration on the device
-  // Launch shape: G blocks of 1024 threads, KPT unknowns per thread.  Fewer blocks
-  // make the grid barrier cheaper (measured ~1 us at 32 blocks, ~3.6 us at 256);
-  // more unknowns per thread cost registers and LDS (a window of per + 2 nx values
-  // of three arrays).  The default takes the largest KPT whose LDS window fits;
-  // fsg_params.pcg_kpt / pcg_blocks override.
-  int kpt = 0, grid = 0;
+  // The largest systems: kpt 4 (refined form: 2) on every co-resident block; the
+  // persistent and refined forms also refuse grids whose rows would not leave a block's
+  // unknowns room in an LDS window of the row-major order (pcg_lds_bytes).
   const int gmax = h->max_coop_blocks;
-  const int kfix = h->prm.pcg_kpt;
-  // spill-free register budgets at 1024 threads: KPT <= 4 (FP32 form), KPT <= 2
-  // (refined), the only instances built; measured fastest at 1024^2: KPT 2 for both
-  const bool refined = solver == FSG_SOLVER_REFINED;
-  const std::initializer_list<int> order_plain = {2, 4, 1}, order_ref = {2, 1};
-  for (int k : refined ? order_ref : order_plain) {
-    if (kfix > 0 && k != kfix) continue;
+  const int kfix = plain ? 0 : h->prm.pcg_kpt;
+  auto blocks = [&](int k) {
     const int gneed = (F + 1024 * k - 1) / (1024 * k);
-    if (gneed > gmax) continue;
-    int g = gneed;
-    if (h->prm.pcg_blocks > 0) g = std::min(std::max(gneed, h->prm.pcg_blocks), gmax);
-    if (pcg_lds_bytes(F, g, h->g.nx) > h->pcg_lds_max) continue;
-    kpt = k;
-    grid = g;
-    break;
+    const int want = plain ? 0 : h->prm.pcg_blocks;
+    return want > 0 ? std::min(std::max(gneed, want), std::max(gneed, gmax)) : gneed;
+  };
+  bool fits = no_count;
+  for (int k : {1, 2, 4}) {
+    if (fits || (kfix > 0 && k != kfix) || (refined && k == 4)) continue;
+    fits = blocks(k) <= gmax &&
+           (plain || pcg_lds_bytes(F, std::max(blocks(k), 1), h->g.nx) <= h->pcg_lds_max);
   }
-  if (kpt == 0)
+  // More than one block: the fewest, since a sum costs what the blocks poll of each other
+  // (plain form at 1024^2, 251,000 unknowns: 5.0 / 5.9 / 7.7 us per iteration at kpt
+  // 4 / 2 / 1, 62 / 123 / 245 blocks; 23,000 unknowns: 4.0 / 4.3 / 4.4).
+  // fsg_params.pcg_kpt / pcg_blocks override (not for the plain form).
+  int kpt = 0, grid = 0;
+  if (fits && !fixed && F <= one_max) {
+    grid = kpt = 1;
+  } else if (fits) {
+    kpt = kfix > 0 ? kfix : 4;
+    grid = std::max(blocks(kpt), 2);
+  }
+  if (kpt == 0) {
+    if (plain) return plain_many_launches(h, F, make_cg_params(h, (float)h->prm.cg_tol));
     return fail(h, FSG_E_INVALID,
                 "pressure system too large for the register-resident persistent solver "
                 "(use FSG_SOLVER_PLAIN)");
-  timed(h, "updown", [&] {
-    launch_updown(h->stream, h->g.nx, F, h->n_fluid, h->cell_of, h->info, h->fluid_index, h->updn);
-  });
+  }
   PersistentArgs a{};
   a.nx = h->g.nx;
-  a.F_max = (int)ncell(h);
   a.F_actual = F;
   a.n_fluid = h->n_fluid;
   a.cell_of = h->cell_of;
   a.info = h->info;
-  a.updn = h->updn;
-  a.b = h->b;
+  a.index_of = h->index_of;
+  a.b = h->ap;
   a.xg = h->xg;
-  a.exch = h->exch;
+  a.zx = reinterpret_cast<uint64_t*>(h->exch);
   a.x64 = h->x64;
-  a.partials = h->partials;
-  a.bar = h->bar;
+  a.slots = reinterpret_cast<uint64_t*>(h->partials);
+  a.abort = h->bar + 1;
   a.sc = h->sc;
-  a.refined = solver == FSG_SOLVER_REFINED;
-  a.cp = make_cg_params(h, a.refined ? (float)h->prm.refine_inner_tol : (float)h->prm.cg_tol);
+  a.refined = refined;
+  a.cp = make_cg_params(h, refined ? (float)h->prm.refine_inner_tol : (float)h->prm.cg_tol);
   a.max_outer = h->prm.refine_max_outer;
   a.inner_tol = (float)h->prm.refine_inner_tol;
   a.outer_tol = h->prm.cg_tol;
-  a.warm_start = h->prm.warm_start != 0;
-  timed(h, "zero_barrier", [&] { launch_fill(h->stream, reinterpret_cast<float*>(h->bar), 4, 0.f); });
+  a.warm_start = !plain && h->prm.warm_start != 0;
+  a.min_iter = plain ? 1 : 0;
   hipError_t e = hipSuccess;
-  timed(h, a.refined ? "cg_refined" : "cg_persistent", [&] { e = launch_pcg(h->stream, a, grid, kpt); });
-  HIPCHK(h, e);
+  timed(h, plain ? "cg_plain" : refined ? "cg_refined" : "cg_persistent",
+        [&] { e = launch_pcg(h->stream, a, grid, kpt); });
   h->last_grid = grid;
   h->last_kpt = kpt;
+  h->last_dev = h->dev_totals = true;
+  if (plain && grid > 1) {
+    // a cooperative launch that was refused, or gave up a wait, is solved again the way
+    // that needs no co-resident blocks
+    unsigned gave_up = 0;
+    if (e == hipSuccess) {
+      HIPCHK(h, hipMemcpyAsync(&gave_up, h->bar + 1, sizeof(gave_up), hipMemcpyDeviceToHost,
+                               h->stream));
+      HIPCHK(h, hipStreamSynchronize(h->stream));
+    } else {
+      (void)hipGetLastError();
+    }
+    if (e != hipSuccess || gave_up) {
+      launch_fill(h->stream, reinterpret_cast<float*>(h->bar), 4, 0.f);
+      return plain_many_launches(h, F, a.cp);
+    }
+    return FSG_OK;
+  }
+  HIPCHK(h, e);
   return FSG_OK;
 }
 
@@ -1051,7 +1087,7 @@ int fsg_create(fsg_domain** out, int32_t nx, int32_t ny, float length_x, float l
   h->density = density;
   h->pic_ratio = pic_ratio;     // the constructor stores it unclamped (src/FluidDomain.cpp:54-68)
   const size_t C = (size_t)nx * ny;
-  const int nb = (int)((C + kScanChunk - 1) / kScanChunk);
+  const size_t nb = (size_t)pcg_tiles(h->g);
   bool ok = true;
   ok &= dalloc(h, &h->u[0], C) == hipSuccess;
   ok &= dalloc(h, &h->u[1], C) == hipSuccess;
@@ -1066,10 +1102,10 @@ int fsg_create(fsg_domain** out, int32_t nx, int32_t ny, float length_x, float l
   for (int q = 0; q < 4; ++q) ok &= dalloc(h, &h->mask[q], C) == hipSuccess;
   ok &= dalloc(h, &h->info_u, C) == hipSuccess;
   ok &= dalloc(h, &h->info_v, C) == hipSuccess;
-  ok &= dalloc(h, &h->counts, (size_t)nb) == hipSuccess;
-  ok &= dalloc(h, &h->offsets, (size_t)nb) == hipSuccess;
+  ok &= dalloc(h, &h->counts, nb) == hipSuccess;
+  ok &= dalloc(h, &h->offsets, nb) == hipSuccess;
   ok &= dalloc(h, &h->n_fluid, 4) == hipSuccess;
-  ok &= dalloc(h, &h->fluid_index, C) == hipSuccess;
+  ok &= dalloc(h, &h->index_of, C) == hipSuccess;
   ok &= dalloc(h, &h->cell_of, C) == hipSuccess;
   ok &= dalloc(h, &h->b, C) == hipSuccess;
   ok &= dalloc(h, &h->info, C) == hipSuccess;
@@ -1077,7 +1113,6 @@ int fsg_create(fsg_domain** out, int32_t nx, int32_t ny, float length_x, float l
   ok &= dalloc(h, &h->ap, C) == hipSuccess;
   ok &= dalloc(h, &h->xg, C) == hipSuccess;
   ok &= dalloc(h, &h->pg0, C) == hipSuccess;
-  ok &= dalloc(h, &h->updn, C) == hipSuccess;
   ok &= dalloc(h, &h->exch, 3 * C) == hipSuccess;
   ok &= dalloc(h, &h->x64, C) == hipSuccess;
   ok &= dalloc(h, &h->partials, (size_t)4 * 4096) == hipSuccess;
@@ -1094,7 +1129,7 @@ int fsg_create(fsg_domain** out, int32_t nx, int32_t ny, float length_x, float l
       if (lds == 0 || lds > 160 * 1024) lds = 160 * 1024;
       h->pcg_lds_max = lds - 4096;
       if (pcg_set_lds_limit(h->pcg_lds_max) == hipSuccess)
-        h->max_coop_blocks = std::min(prop.multiProcessorCount, 1024);
+        h->max_coop_blocks = std::min(prop.multiProcessorCount, kPcgMaxBlocks);
     }
   }
   if (hipStreamSynchronize(h->stream) != hipSuccess) return bail(FSG_E_HIP);
@@ -1547,21 +1582,22 @@ int fsg_run_phase(fsg_domain* h, int32_t phase, float dt) {
   return FSG_OK;
 }
 
-// The fluid index of every cell (src/FluidSolver.cpp:331-346): the compaction's, or,
-// where the last solve did not compact (the multigrid form), the row-major running
-// count of the LIQUID cells of the labels, which is what the compaction forms.
+// The fluid index of every cell (src/FluidSolver.cpp:331-346): the row-major running
+// count of the LIQUID cells of the last solve (or, where that did not index them, of the
+// labels).
 static int host_fluid_indices(fsg_domain* h, int32_t* idx) {
   const size_t C = ncell(h);
+  int32_t k = 0;
   if (h->compacted) {
-    HIPCHK(h, hipMemcpyAsync(idx, h->fluid_index, C * sizeof(int), hipMemcpyDeviceToHost,
+    HIPCHK(h, hipMemcpyAsync(idx, h->index_of, C * sizeof(int), hipMemcpyDeviceToHost,
                              h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    for (size_t c = 0; c < C; ++c) idx[c] = idx[c] >= 0 ? k++ : -1;
     return FSG_OK;
   }
   std::vector<uint8_t> lab(C);
   HIPCHK(h, hipMemcpyAsync(lab.data(), h->label, C, hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  int32_t k = 0;
   for (size_t c = 0; c < C; ++c) idx[c] = lab[c] == kLiquid ? k++ : -1;
   return FSG_OK;
 }
@@ -1580,19 +1616,10 @@ int fsg_get_pressure(fsg_domain* h, float* p) {
 
 int fsg_get_rhs(fsg_domain* h, float* bout) {
   if (!h || check_grid_ptr(h, bout)) return FSG_E_INVALID;
-  const size_t C = ncell(h);
-  if (!h->compacted) {  // b per cell, 0 off the LIQUID cells
-    HIPCHK(h, hipMemcpyAsync(bout, h->b, C * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    return FSG_OK;
-  }
-  std::vector<int> idx(C);
-  std::vector<float> bc(C);
-  HIPCHK(h, hipMemcpyAsync(idx.data(), h->fluid_index, C * sizeof(int), hipMemcpyDeviceToHost,
+  // b per cell, 0 off the LIQUID cells
+  HIPCHK(h, hipMemcpyAsync(bout, h->b, ncell(h) * sizeof(float), hipMemcpyDeviceToHost,
                            h->stream));
-  HIPCHK(h, hipMemcpyAsync(bc.data(), h->b, C * sizeof(float), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  for (size_t c = 0; c < C; ++c) bout[c] = idx[c] >= 0 ? bc[(size_t)idx[c]] : 0.f;
   return FSG_OK;
 }
 
@@ -1636,9 +1663,11 @@ int fsg_get_reject_flags(fsg_domain* h, uint8_t* flags) {
 
 int fsg_get_stats(fsg_domain* h, fsg_stats* s) {
   if (!h || !s) return FSG_E_INVALID;
-  // the plain and multigrid forms keep their statistics on the host (read with their
-  // stop tests): no device access, no synchronisation
-  if (h->prm.solver == FSG_SOLVER_PLAIN || h->prm.solver == FSG_SOLVER_MG) {
+  // the multigrid form and the many-launch plain form keep their statistics on the host
+  // (read with their stop tests): no device access, no synchronisation
+  const bool one_launch =
+      h->prm.solver == FSG_SOLVER_PERSISTENT || h->prm.solver == FSG_SOLVER_REFINED;
+  if (!one_launch && !h->last_dev && !h->dev_totals) {
     *s = h->host_stats;
     return FSG_OK;
   }
@@ -1648,11 +1677,16 @@ int fsg_get_stats(fsg_domain* h, fsg_stats* s) {
   HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipMemcpyAsync(&F, h->n_fluid, sizeof(int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  memset(s, 0, sizeof(*s));
-  s->n_fluid = F;
-  s->cg_iterations = hs.iter;
-  s->cg_error = hs.err;
-  s->refine_sweeps = hs.refine_sweeps;
+  if (one_launch)
+    memset(s, 0, sizeof(*s));
+  else
+    *s = h->host_stats;
+  if (one_launch || h->last_dev) {
+    s->n_fluid = F;
+    s->cg_iterations = hs.iter;
+    s->cg_error = hs.err;
+    s->refine_sweeps = hs.refine_sweeps;
+  }
   s->total_unknown_iterations = (int64_t)hs.total_unknown_iters + h->host_stats.total_unknown_iterations;
   s->total_solves = hs.total_solves + h->host_stats.total_solves;
   return FSG_OK;
@@ -1670,6 +1704,7 @@ int fsg_reset_stats(fsg_domain* h) {
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->host_stats.total_unknown_iterations = 0;
   h->host_stats.total_solves = 0;
+  h->dev_totals = false;
   return FSG_OK;
 }
 

@@ -141,8 +141,6 @@ void launch_advect_level_set(hipStream_t s, const Geom& g, const float* phi, flo
                              const float* u, const float* v, float dt);
 
 // ---------------------------------------------------------------- pressure
-constexpr int kScanChunk = 2048;  // cells per block of the liquid count / compaction
-
 // Info bit of the multigrid form's level-0 cells: the cell is an unknown (a LIQUID cell
 // with a non-SOLID neighbour).
 constexpr uint8_t kMgUnknown = 0x80;
@@ -187,13 +185,15 @@ struct CgParams {
   int project_mean;
 };
 
-void launch_count_liquid(hipStream_t s, const Geom& g, const uint8_t* label, int* counts);
+// The unknowns in tile order (kernels_pcg.hip): LIQUID cells per 32 x 32 tile, the scan
+// of the counts into offsets (and *n_fluid), then per unknown its cell, neighbour info
+// byte and b, per cell its unknown (-1) and b (0)
+int pcg_tiles(const Geom& g);
+void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts);
 void launch_scan_counts(hipStream_t s, int nb, const int* counts, int* offsets, int* n_fluid);
-void launch_compact(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
-                    int* fluid_index, int* cell_of, const float* uf, const float* vf, float* b,
-                    uint8_t* info);
-void launch_updown(hipStream_t s, int nx, int F_bound, const int* n_fluid, const int* cell_of,
-                   const uint8_t* info, const int* fluid_index, int2* updn);
+void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
+                     int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
+                     float* rhs, uint8_t* info);
 
 // plain form (partials: >= 12288 doubles)
 void launch_cg_init(hipStream_t s, int F, const CgParams& cp, const int* cell_of,
@@ -203,21 +203,24 @@ void launch_cg_iteration(hipStream_t s, int F, int nx, int it, const CgParams& c
                          const int* cell_of, const uint8_t* info, float* r, float* ap, float* pg,
                          float* xg, double* partials, CgScalars* sc);
 
-// persistent forms (pipelined PCG, optionally inside FP64 refinement)
+// one-launch forms of the Jacobi-PCG, optionally inside FP64 refinement
+// (kernels_pcg.hip)
+constexpr int kPcgOneUnknowns = 8192;  // the most unknowns that one block solves (FP32 form)
+constexpr int kPcgOneRefined = 4096;   // and in the refined form
+constexpr int kPcgMaxBlocks = 256;     // blocks of a solve: four waves read their sums
 struct PersistentArgs {
   int nx;
-  int F_max;             // capacity of the compact arrays
-  int F_actual;          // unknowns of this solve (host copy, sizes the launch)
+  int F_actual;          // unknowns of this solve, or a bound of them (sizes the launch)
   const int* n_fluid;
   const int* cell_of;
   const uint8_t* info;
-  const int2* updn;
+  const int* index_of;   // unknown of a cell
   const float* b;
   float* xg;             // solution, grid layout
-  float* exch;           // 3 x F_max floats: device-coherent z and p (x2) exchange
-  double* x64;           // F_max doubles: FP64 solution exchange (refined form)
-  double* partials;      // 2 x grid x 4 doubles
-  unsigned* bar;         // [0] arrival counter, [1] abort flag
+  uint64_t* zx;          // F_actual words: z crossing blocks, tagged
+  double* x64;           // F_actual doubles: FP64 solution exchange (refined form)
+  uint64_t* slots;       // pcg_slot_words(grid): the blocks' partial sums, tagged
+  unsigned* abort;       // set when a block gave up waiting
   CgScalars* sc;
   CgParams cp;
   int refined;
@@ -225,9 +228,14 @@ struct PersistentArgs {
   float inner_tol;
   double outer_tol;
   int warm_start;        // 1: x0 = previous solution (xg), else x0 = 0
+  int min_iter;          // the solve runs only with cp.max_iter >= min_iter (plain form:
+                         // 1, it takes no iteration at max_iter 0; else 0)
 };
-int pcg_max_kpt();
 size_t pcg_lds_bytes(int F, int grid, int nx);
+size_t pcg_slot_words(int grid);
+// kpt: 1024-unknown units per block.  grid 1: an ordinary launch, F_actual (kpt is not
+// used) at most kPcgOneUnknowns or kPcgOneRefined; more blocks: kpt 1, 2 or 4, a
+// cooperative launch, and the exchange is cleared before it
 hipError_t launch_pcg(hipStream_t s, const PersistentArgs& a, int grid, int kpt);
 hipError_t pcg_set_lds_limit(size_t max_bytes);
 

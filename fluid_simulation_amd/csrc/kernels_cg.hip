@@ -1,26 +1,20 @@
-// kernels_cg.hip -- pressure Poisson system setup and the Jacobi-preconditioned CG
-// solvers that replace Eigen::ConjugateGradient (include/FluidSolver.h:114,
-// src/FluidSolver.cpp:81,362-425).
+// kernels_cg.hip -- the many-launch form of the Jacobi-preconditioned CG that replaces
+// Eigen::ConjugateGradient (include/FluidSolver.h:114, src/FluidSolver.cpp:81,362-425):
+// three kernels per iteration, for systems of more unknowns than the one-launch form
+// (kernels_pcg.hip) holds in registers (about 2^20), and for a plain solve whose
+// co-resident launch was refused or gave up a wait.
 //
-// Unknowns are the LIQUID cells in row-major order, exactly the reference's
-// fluid_indices (src/FluidSolver.cpp:331-346), built by a three-kernel scan.  The
-// operator is applied matrix-free: one info byte per unknown holds the four
-// LIQUID-neighbour bits and the count of non-SOLID neighbours, so A's row is
-// diag_tab[count] at the centre and off = 1/dx^2 at each LIQUID neighbour.  Left
-// and right neighbours of unknown k are k-1 and k+1 (row-major order); the up and
-// down neighbours' indices are stored per unknown.
+// Unknowns are the LIQUID cells in the order of kernels_pcg.hip's set-up.  The operator
+// is applied matrix-free: one info byte per unknown holds the four LIQUID-neighbour bits
+// and the count of non-SOLID neighbours, so A's row is diag_tab[count] at the centre and
+// off = 1/dx^2 at each LIQUID neighbour; x and p are cell grids.
 //
 // Synchronisation on gfx950 (measured): a contended returning atomic costs ~90 ns
 // per block and agent-scope release/acquire fences write back and invalidate L2.
-// So no kernel here uses a last-block ticket or an agent-scope fence:
-//  - the plain form lets every block re-sum the previous kernel's per-block
-//    partials in a fixed order (kernel boundaries order the data);
-//  - the persistent forms use a fence-free grid barrier: data that crosses blocks
-//    (halo values, partial sums) is written with agent-scope atomic stores and read
-//    with agent-scope atomic loads, both of which go to the device coherence point,
-//    and the arrival counter takes one non-returning atomic add per block.
-// Every sum is deterministic (fixed per-thread order, fixed wave/block tree, fixed
-// block order), so every block of a persistent launch derives identical scalars.
+// So no kernel here uses a last-block ticket or an agent-scope fence: every block
+// re-sums the previous kernel's per-block partials in a fixed order (kernel boundaries
+// order the data).  Every sum is deterministic (fixed per-thread order, fixed wave /
+// block tree, fixed block order).
 #include <float.h>
 
 #include "fsg_common.h"
@@ -30,29 +24,7 @@
 namespace fsg {
 
 // ------------------------------------------------------------ system setup
-// Per 2048-cell chunk: number of LIQUID cells (8 cells per thread, 8-byte loads).
-__global__ void __launch_bounds__(256) k_count_liquid(int n, const uint8_t* __restrict__ label,
-                                                      int* __restrict__ counts) {
-  const int base = blockIdx.x * kScanChunk + threadIdx.x * 8;
-  int cnt = 0;
-  if (base + 8 <= n) {
-    const uint2 w = *reinterpret_cast<const uint2*>(label + base);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      cnt += ((w.x >> (8 * q)) & 0xFF) == kLiquid;
-      cnt += ((w.y >> (8 * q)) & 0xFF) == kLiquid;
-    }
-  } else {
-    for (int q = 0; q < 8; ++q)
-      if (base + q < n) cnt += label[base + q] == kLiquid;
-  }
-  double v[1] = {(double)cnt};
-  __shared__ double sm[4];
-  block_sum<1, 256>(v, sm);
-  if (threadIdx.x == 0) counts[blockIdx.x] = (int)v[0];
-}
-
-// Exclusive scan of the chunk counts in one block of 1024 threads.
+// Exclusive scan of the tiles' LIQUID counts in one block of 1024 threads.
 __global__ void __launch_bounds__(1024) k_scan_counts(int nb, const int* __restrict__ counts,
                                                       int* __restrict__ offsets,
                                                       int* __restrict__ n_fluid) {
@@ -70,87 +42,13 @@ __global__ void __launch_bounds__(1024) k_scan_counts(int nb, const int* __restr
     sm[threadIdx.x] += v;
     __syncthreads();
   }
-  int run = sm[threadIdx.x] - s;  // exclusive prefix of this thread's first chunk
+  int run = sm[threadIdx.x] - s;  // exclusive prefix of this thread's first tile
   for (int q = 0; q < per; ++q)
     if (b0 + q < nb) {
       offsets[b0 + q] = run;
       run += counts[b0 + q];
     }
   if (threadIdx.x == 1023) *n_fluid = sm[1023];
-}
-
-// fluid_indices (src/FluidSolver.cpp:331-346), the compact cell list, the
-// divergence right-hand side b = divVelX + divVelY (:413, MacGrid.h:98-111) and the
-// neighbour info byte (:379-410).
-__global__ void __launch_bounds__(256) k_compact(Geom g, const uint8_t* __restrict__ label,
-                                                 const int* __restrict__ offsets,
-                                                 int* __restrict__ fluid_index,
-                                                 int* __restrict__ cell_of,
-                                                 const float* __restrict__ uf,
-                                                 const float* __restrict__ vf,
-                                                 float* __restrict__ b,
-                                                 uint8_t* __restrict__ info) {
-  const int n = g.nx * g.ny, nx = g.nx;
-  const int base = blockIdx.x * kScanChunk + threadIdx.x * 8;
-  uint8_t lab[8];
-#pragma unroll
-  for (int q = 0; q < 8; ++q) lab[q] = (base + q < n) ? label[base + q] : kAir;
-  int cnt = 0;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) cnt += lab[q] == kLiquid;
-  // exclusive scan over the block's 256 threads
-  __shared__ int sm[256];
-  sm[threadIdx.x] = cnt;
-  __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int v = threadIdx.x >= off ? sm[threadIdx.x - off] : 0;
-    __syncthreads();
-    sm[threadIdx.x] += v;
-    __syncthreads();
-  }
-  int k = offsets[blockIdx.x] + sm[threadIdx.x] - cnt;
-#pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int c = base + q;
-    if (c >= n) break;
-    if (lab[q] != kLiquid) {
-      fluid_index[c] = -1;
-      continue;
-    }
-    fluid_index[c] = k;
-    cell_of[k] = c;
-    const int i = c % nx, j = c / nx;
-    // out-of-range neighbours count as SOLID (a SOLID border makes this moot)
-    const uint8_t lxm = i > 0 ? label[c - 1] : kSolid;
-    const uint8_t lxp = i < nx - 1 ? label[c + 1] : kSolid;
-    const uint8_t lym = j > 0 ? label[c - nx] : kSolid;
-    const uint8_t lyp = j < g.ny - 1 ? label[c + nx] : kSolid;
-    const int bits = (lxm == kLiquid) | ((lxp == kLiquid) << 1) | ((lym == kLiquid) << 2) |
-                     ((lyp == kLiquid) << 3);
-    const int nns = (lxm != kSolid) + (lxp != kSolid) + (lym != kSolid) + (lyp != kSolid);
-    info[k] = (uint8_t)(bits | (nns << 4));
-    const float uxp = i < nx - 1 ? uf[c + 1] : 0.f;
-    const float vyp = j < g.ny - 1 ? vf[c + nx] : 0.f;
-    const float dvx = div_x(uxp - uf[c], g);
-    const float dvy = div_y(vyp - vf[c], g);
-    b[k] = dvx + dvy;
-    ++k;
-  }
-}
-
-// Compact indices of the (j-1) and (j+1) neighbours of every unknown (-1 where the
-// neighbour is not LIQUID).  Runs after k_compact has written fluid_index.
-__global__ void __launch_bounds__(256) k_updown(int nx, const int* __restrict__ n_fluid,
-                                                const int* __restrict__ cell_of,
-                                                const uint8_t* __restrict__ info,
-                                                const int* __restrict__ fluid_index,
-                                                int2* __restrict__ updn) {
-  const int F = *n_fluid;
-  for (int k = blockIdx.x * 256 + threadIdx.x; k < F; k += gridDim.x * 256) {
-    const int c = cell_of[k];
-    const uint8_t inf = info[k];
-    updn[k] = make_int2((inf & 4) ? fluid_index[c - nx] : -1, (inf & 8) ? fluid_index[c + nx] : -1);
-  }
 }
 
 // ---------------------------------------------------------------- plain form
@@ -338,26 +236,8 @@ static inline int cg_blocks(int F) {
   return nb;
 }
 
-void launch_count_liquid(hipStream_t s, const Geom& g, const uint8_t* label, int* counts) {
-  const int n = g.nx * g.ny;
-  k_count_liquid<<<(n + kScanChunk - 1) / kScanChunk, 256, 0, s>>>(n, label, counts);
-}
 void launch_scan_counts(hipStream_t s, int nb, const int* counts, int* offsets, int* n_fluid) {
   k_scan_counts<<<1, 1024, 0, s>>>(nb, counts, offsets, n_fluid);
-}
-void launch_compact(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
-                    int* fluid_index, int* cell_of, const float* uf, const float* vf, float* b,
-                    uint8_t* info) {
-  const int n = g.nx * g.ny;
-  k_compact<<<(n + kScanChunk - 1) / kScanChunk, 256, 0, s>>>(g, label, offsets, fluid_index,
-                                                               cell_of, uf, vf, b, info);
-}
-void launch_updown(hipStream_t s, int nx, int F_bound, const int* n_fluid, const int* cell_of,
-                   const uint8_t* info, const int* fluid_index, int2* updn) {
-  int nb = (F_bound + 255) / 256;
-  if (nb > 4096) nb = 4096;
-  if (nb < 1) nb = 1;
-  k_updown<<<nb, 256, 0, s>>>(nx, n_fluid, cell_of, info, fluid_index, updn);
 }
 void launch_cg_init(hipStream_t s, int F, const CgParams& cp, const int* cell_of,
                     const uint8_t* info, const float* b, float* r, float* pg, float* xg,

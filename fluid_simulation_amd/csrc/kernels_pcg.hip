@@ -1,39 +1,52 @@
-// kernels_pcg.hip -- persistent (one launch per solve) Jacobi-preconditioned CG,
-// optionally inside FP64 iterative refinement.  Replaces Eigen::ConjugateGradient
-// (include/FluidSolver.h:114, src/FluidSolver.cpp:81,424-425).
+// kernels_pcg.hip -- Jacobi-preconditioned CG with every iteration of a solve in one
+// launch, optionally inside FP64 iterative refinement, and the set-up of the systems.
+// Replaces Eigen::ConjugateGradient (include/FluidSolver.h:114, src/FluidSolver.cpp:81,
+// 424-425).
 //
-// Launch: G co-resident blocks of 1024 threads (cooperative launch).  Block b owns
-// the contiguous range [k0, k1) = [b*per, (b+1)*per) of unknowns (LIQUID cells in
-// row-major order); a thread owns up to KPT of them (k = k0 + tid + j*1024) and
-// keeps their x, r and Ap in registers.
+// G blocks of 512 threads; block b owns the range [b*per, (b+1)*per) of the unknowns (the
+// LIQUID cells in tile order, k_pcg_fill), a thread up to KPT of them (k = k0 + tid +
+// j*512) whose x, r, z, p and Ap stay in its registers.  The search direction p of the
+// block's unknowns and of their neighbours in other blocks (its halo) is in LDS.
 //
-// Neighbour values.  The SpMV of unknown k reads k-1, k+1 and its up/down
-// neighbours, all within hw = nx of k in the compact order.  Each block keeps an
-// LDS window over [k0 - hw, k1 + hw) of z = M^-1 r and of the search direction p
-// (two buffers, by iteration parity).  Own entries are written by the owning
-// threads; the two halo stripes are staged from device-coherent exchange arrays
-// into which every unknown within hw of its block's ends is published.
+// Iteration (Eigen's PCG, the same float operations per unknown as the kernels of
+// kernels_cg.hip, sums in FP64):
+//   A: p = z + beta p (own unknowns and halo alike); Ap; sum p.Ap
+//      -- alpha = r.z / p.Ap
+//   B: x += alpha p, r -= alpha Ap, z = M^-1 r; sums |r|^2, r.z
+//      -- stop test, beta
+// Only z crosses blocks: a block keeps p on its halo itself, from the halo's z.
 //
-// Iteration (Eigen's PCG, two grid barriers, each also a reduction):
-//   A: stage the halo of z and p_{k-1}; p_k = z_k + beta p_{k-1} for own unknowns
-//      and, in the stencil, for neighbours; publish p_k; Ap; partial p.Ap
-//      -- barrier --  alpha = r.z / p.Ap
-//   B: x += alpha p, r -= alpha Ap, z = M^-1 r (published), partial |r|^2, r.z
-//      -- barrier --  stop test, beta
-// Phase A reads z (published before barrier B) and p_{k-1} (published in the
-// previous phase A, before barrier A) and writes p_k into the other buffer of the
-// pair, so no third barrier is needed.
+// What bounds an iteration is the chain of device-coherent round trips between blocks
+// (0.6 us between two blocks, 1.2-1.3 us for all of 23-123 blocks to have read a word of
+// each), not arithmetic or bytes: 250,000 unknowns are 1 MB per vector, held in
+// registers.  So nothing is ordered by waiting for stores, counting arrivals in a memory
+// location and reading the data afterwards (three to four round trips per sum): every
+// 32-bit value that crosses blocks travels in a 64-bit word together with a tag (the
+// number of the sum it belongs to), and its readers poll the word itself until the tag
+// is the one they wait for.  A sum then costs one store and one successful poll; the
+// halo's z is polled by other waves of the block while the sums of phase B are, so it
+// costs no trip of its own.  Refined form at 250,000 unknowns (1024^2): 15.0 -> 4.9 us
+// per iteration against a counting grid barrier on 123 blocks of 1024 threads.
 //
-// Grid barrier: agent-scope atomic stores for everything that crosses blocks, one
-// non-returning atomic add per block on a monotonic counter, relaxed polling; no
-// agent-scope fences (they write back and invalidate L2 on gfx950).  The wait is
-// bounded: a block that waits too long raises an abort flag, every block leaves at
-// its next barrier, and the host reports the failure.
+// A single block (k_pcg_one) exchanges nothing: its sums go through LDS with one
+// workgroup barrier each.  1.0 us per iteration at 530 unknowns, 1.6 us at 3,800 (bound
+// by VALU issue: 8 unknowns per thread), where three launches per iteration take 15-17.
+//
+// Ordering: words are cleared before the launch (k_pcg_clear) and tags grow, so a tag
+// is never met before its value.  Sum e uses slot set e & 1: a block publishes sum e + 2
+// only after it has read every block's sum e + 1, which each publishes after it has read
+// all of sum e.  A block's z words of iteration k are rewritten in phase B of the next
+// iteration, after the sum of phase A, which every block joins only after it has read
+// its halo.  Waits are bounded: a wave that polls for too long raises an abort flag,
+// every block leaves at its next sum, and the host reports it (or, for the plain form,
+// solves again with the kernels of kernels_cg.hip).
 //
 // Refined form: FP64 iterative refinement around the FP32 solve -- r64 = b - A x64
 // with the SpMV and its reduction in FP64, inner solve of A e = r64 to a relative
 // tolerance, x64 += e -- until |b - A x64| < tol |b| in FP64.
 #include <float.h>
+
+#include <algorithm>
 
 #include "fsg_common.h"
 #include "fsg_device.h"
@@ -41,111 +54,367 @@
 
 namespace fsg {
 
-constexpr int kPcgThreads = 1024;
-constexpr unsigned kSpinLimit = 1u << 22;  // seconds of waiting: treated as a fault
+namespace {
 
-struct BarrierState {
-  unsigned* count;  // monotonic arrival counter
-  unsigned* abort;  // set when a block gives up waiting
-  unsigned epoch;
-  double* slots;    // 2 parity sets x G blocks x 4 values
+constexpr int kPcgThreads = 512;
+constexpr unsigned kSpinLimit = 1u << 22;  // seconds of waiting: treated as a fault
+constexpr int kSlotWords = 4;              // 64-bit words per block and sum: 2 doubles
+
+// DPP move of a double; lanes without a source take 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+// Sum over the first 8 lanes of each 16-lane row, in lane 7 of the row.
+__device__ __forceinline__ double row_sum8(double v) {
+  v += dpp_f64<0x111, 0xF>(v);  // row_shr:1, 2, 4
+  v += dpp_f64<0x112, 0xF>(v);
+  v += dpp_f64<0x114, 0xF>(v);
+  return v;
+}
+// Sums over the wave, in lane 63, the values' steps interleaved (register moves only: a
+// shuffle tree of doubles costs 12 LDS-latency exchanges).
+template <int CTRL, int ROWS, int NV>
+__device__ __forceinline__ void dpp_step(double (&v)[NV]) {
+  double t[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) t[q] = dpp_f64<CTRL, ROWS>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] += t[q];
+}
+template <int NV>
+__device__ __forceinline__ void wave_sums(double (&v)[NV]) {
+  dpp_step<0x111, 0xF>(v);
+  dpp_step<0x112, 0xF>(v);
+  dpp_step<0x114, 0xF>(v);
+  dpp_step<0x118, 0xF>(v);
+  dpp_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  dpp_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+}
+// Lane `from`'s value, in every lane.
+__device__ __forceinline__ double lane_value(double v, int from) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), from),
+                          __builtin_amdgcn_readlane(__double2loint(v), from));
+}
+
+// Halo entries of a block of `per` unknowns in tile order, at most: an unknown on the rim
+// of its 32 x 32 tile has at most two neighbours in other tiles, and the first and the
+// last tile of the range may be shared with another block (33 links each).
+__host__ __device__ constexpr int pcg_halo_cap(int per) { return 2 * per + 66; }
+
+__device__ __forceinline__ uint64_t tagged(uint32_t bits, uint32_t tag) {
+  return ((uint64_t)tag << 32) | bits;
+}
+__device__ __forceinline__ uint32_t tag_of(uint64_t w) { return (uint32_t)(w >> 32); }
+
+struct PcgNet {
+  uint64_t* slots;  // [2][G][kSlotWords]
+  uint64_t* z;      // one word per unknown: z of the unknowns in some block's halo
+  unsigned* abort;
+  uint32_t epoch;   // sums so far; the tag of the last one
 };
 
-// Grid barrier carrying up to 4 partial sums per block; returns the grid totals
-// (identical in every block).  Returns false if the wait was abandoned, in which
-// case the caller leaves the kernel without entering another barrier.
-template <int NV>
-__device__ __forceinline__ bool grid_reduce(BarrierState& bs, double (&v)[NV], double* sm) {
-  static_assert(NV <= 4, "grid_reduce: at most 4 values");
-  block_sum<NV, kPcgThreads>(v, sm);
-  const unsigned G = gridDim.x;
-  double* set = bs.slots + (size_t)(bs.epoch & 1) * G * 4;
-  if (threadIdx.x == 0)
+struct PcgShared {
+  double part[2][2][8];  // the block's wave sums, by epoch parity and value
+  double tot[2][2][8];   // the grid's totals per polling wave; 0 past those
+  int ok;
+  int n_halo;
+};
+
+// Polls a thread's N words until each carries the tag (at(q): word q, null for none);
+// false when the wait was abandoned.  All loads of a round are in flight together.
+template <int N, typename At>
+__device__ __forceinline__ bool poll(At&& at, uint32_t tag, uint64_t (&w)[N], unsigned* abort) {
+  for (unsigned spins = 0;; ++spins) {
+    bool good = true;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) st_dev(&set[blockIdx.x * 4 + q], v[q]);
-  // every wave's device-coherent stores complete before the block arrives
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  bs.epoch += 1;
-  __shared__ int ok;
-  if (threadIdx.x == 0) {
-    __hip_atomic_fetch_add(bs.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned target = bs.epoch * G;
-    unsigned spins = 0;
-    int good = 1;
-    while (ld_dev(bs.count) < target) {
-      __builtin_amdgcn_s_sleep(1);
-      if (++spins > kSpinLimit) {
-        st_dev(bs.abort, 1u);
-        good = 0;
-        break;
-      }
-      if ((spins & 255u) == 0 && ld_dev(bs.abort)) {
-        good = 0;
-        break;
-      }
+    for (int q = 0; q < N; ++q) {
+      const uint64_t* p = at(q);
+      w[q] = p ? ld_dev(p) : tagged(0u, tag);
     }
-    ok = good;
+#pragma unroll
+    for (int q = 0; q < N; ++q) good &= tag_of(w[q]) == tag;
+    if (good) return true;
+    if (spins > kSpinLimit) {
+      st_dev(abort, 1u);
+      return false;
+    }
+    if ((spins & 255u) == 255u && ld_dev(abort)) return false;
+  }
+}
+
+// The sums of NV values over the grid, in every thread (the same fixed order in every
+// block); false when a wait was abandoned: the caller leaves the kernel without
+// another sum.  `side` runs in the waves that do not poll the sums, while those do.
+// DRAIN: the block's device-coherent stores are complete before its sum is published
+// (a reader that has the sum may then read what they wrote).
+// One slot per block, not one per wave (which would save the first barrier): beyond the
+// two trips a sum costs what the blocks poll of each other (62 blocks: 5.5 us per
+// iteration with a slot per block, 6.9 with one per wave; 245 blocks: 8.6 and 17).
+template <int NV, bool ONE, bool DRAIN, typename Side>
+__device__ __forceinline__ bool grid_sum(PcgNet& net, double (&v)[NV], PcgShared& sh,
+                                         Side&& side) {
+  static_assert(NV <= 2, "grid_sum: at most 2 values");
+  constexpr int NW = kPcgThreads / 64;
+  static_assert(NW == 8, "grid_sum: eight waves");
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t e = ++net.epoch;
+  const int par = e & 1;
+  wave_sums(v);
+  if (lane == 63)
+#pragma unroll
+    for (int q = 0; q < NV; ++q) sh.part[par][q][wave] = v[q];
+  if (DRAIN && !ONE) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0);
   }
   __syncthreads();
-  if (!ok) return false;
-  double acc[NV];
+  // value q's total over the waves in lane 16 q + 7
+  auto total = [&](const double (&t)[2][8]) {
+    return row_sum8(t[(lane >> 4) & (NV - 1)][lane & 7]);
+  };
+  if (!ONE) {
+    const int G = gridDim.x, npoll = (G + 63) >> 6;
+    uint64_t* set = net.slots + (size_t)par * G * kSlotWords;
+    bool good = true;
+    if (wave < npoll) {
+      if (wave == 0) {
+        const double s = total(sh.part[par]);
+        if ((lane & 15) == 7 && (lane >> 4) < NV) {
+          uint64_t* dst = set + (size_t)blockIdx.x * kSlotWords + 2 * (lane >> 4);
+          st_dev(dst, tagged((uint32_t)__double2loint(s), e));
+          st_dev(dst + 1, tagged((uint32_t)__double2hiint(s), e));
+        }
+      }
+      const int b = wave * 64 + lane;
+      uint64_t w[2 * NV];
+      good = poll([&](int q) { return b < G ? set + (size_t)b * kSlotWords + q : nullptr; }, e, w,
+                  net.abort);
+      double t[NV];
 #pragma unroll
-  for (int q = 0; q < NV; ++q) acc[q] = 0.0;
-  for (int b = threadIdx.x; b < (int)G; b += kPcgThreads)
+      for (int q = 0; q < NV; ++q)
+        t[q] = __hiloint2double((int)(uint32_t)w[2 * q + 1], (int)(uint32_t)w[2 * q]);
+      wave_sums(t);
+      if (lane == 63)
 #pragma unroll
-    for (int q = 0; q < NV; ++q) acc[q] += ld_dev(&set[b * 4 + q]);
-  block_sum<NV, kPcgThreads>(acc, sm);
+        for (int q = 0; q < NV; ++q) sh.tot[par][q][wave] = t[q];
+    } else {
+      good = side(wave - npoll, NW - npoll);
+    }
+    if (!good) sh.ok = 0;
+    __syncthreads();
+    if (!sh.ok) return false;
+  }
+  // each wave adds the parts itself
+  const double s = total(ONE ? sh.part[par] : sh.tot[par]);
 #pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] = acc[q];
+  for (int q = 0; q < NV; ++q) v[q] = lane_value(s, 16 * q + 7);
   return true;
 }
 
-template <int KPT, bool REFINED>
-__global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
-  extern __shared__ float lds[];
-  __shared__ double sm[4 * (kPcgThreads / 64)];
-  const int F = *a.n_fluid;
-  if (F == 0) return;  // uniform across the grid: no barrier is entered
-  const int G = gridDim.x;
-  const int per = (F + G - 1) / G;
-  const int hw = a.nx;                 // halo width in compact indices
-  const int W = per + 2 * hw;          // LDS window length
-  const int k0 = min(F, (int)blockIdx.x * per);
-  const int k1 = min(F, k0 + per);
-  const int wb = k0 - hw;              // window base: slot = k - wb
-  const int tid = threadIdx.x;
-  float* lz = lds;
-  float* lp0 = lds + W;
-  float* lp1 = lds + 2 * W;
-  float* ez = a.exch;
-  float* ep0 = a.exch + a.F_max;
-  float* ep1 = a.exch + 2 * (size_t)a.F_max;
-  const CgParams& cp = a.cp;
+// ---------------------------------------------------------------- set-up
+// The unknowns (LIQUID cells) in tile order: 32 x 32-cell tiles row by row, a tile's
+// cells row by row.  A block's range of them is then a compact patch: its halo is the
+// patch's rim (320 links for 4 full tiles), where a range of the row-major order has a
+// full row of the grid above and below it (2044 at 1024 columns); the halo is read
+// through device-coherent loads in every iteration (62 blocks: 5.5 -> 5.0 us each).
+__device__ __forceinline__ bool tile_cell(const Geom& g, int tile, int t, int& i, int& j) {
+  const int tiles_x = (g.nx + 31) >> 5;
+  i = (tile % tiles_x) * 32 + (t & 31);
+  j = (tile / tiles_x) * 32 + (t >> 5);
+  return i < g.nx && j < g.ny;
+}
 
-  // unknown j of this thread: k = k0 + tid + j*1024, LDS slot hw + tid + j*1024
-  int su[KPT], sd[KPT];  // LDS slots of the up / down neighbours
-  unsigned valid = 0, infw = 0, nnsw = 0, exported = 0;
+// LIQUID cells per tile (thread t: the four cells 4 t .. 4 t + 3 of the tile).
+__global__ void __launch_bounds__(256) k_pcg_count(Geom g, const uint8_t* __restrict__ label,
+                                                   int* __restrict__ counts) {
+  __shared__ int s_w[4];
+  int n = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    int i, j;
+    if (tile_cell(g, blockIdx.x, 4 * threadIdx.x + e, i, j)) n += label[i + j * g.nx] == kLiquid;
+  }
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
+  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) counts[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+}
+
+// Per unknown: its cell, neighbour info (src/FluidSolver.cpp:379-410) and right-hand side
+// b = divVelX + divVelY (:413, MacGrid.h:98-111); per cell: its unknown's index (-1), and
+// b (0) as fsg_get_rhs returns it.
+__global__ void __launch_bounds__(256) k_pcg_fill(Geom g, const uint8_t* __restrict__ label,
+                                                  const int* __restrict__ offsets,
+                                                  int* __restrict__ index_of,
+                                                  int* __restrict__ cell_of,
+                                                  const float* __restrict__ uf,
+                                                  const float* __restrict__ vf,
+                                                  float* __restrict__ b, float* __restrict__ rhs,
+                                                  uint8_t* __restrict__ info) {
+  __shared__ int s_w[4];
+  const int nx = g.nx, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int c[4], n = 0;
+  bool in[4], liq[4];
+  int ci[4], cj[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    in[e] = tile_cell(g, blockIdx.x, 4 * threadIdx.x + e, ci[e], cj[e]);
+    c[e] = in[e] ? ci[e] + cj[e] * nx : 0;
+    liq[e] = in[e] && label[c[e]] == kLiquid;
+    n += liq[e];
+  }
+  int x = n;  // inclusive scan over the wave
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) s_w[wave] = x;
+  __syncthreads();
+  int k = offsets[blockIdx.x] + x - n;
+  for (int w = 0; w < wave; ++w) k += s_w[w];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (!in[e]) continue;
+    float bf = 0.f;
+    int idx = -1;
+    if (liq[e]) {
+      const int i = ci[e], j = cj[e], q = c[e];
+      // out-of-range neighbours count as SOLID (a SOLID border makes this moot)
+      const uint8_t lxm = i > 0 ? label[q - 1] : kSolid;
+      const uint8_t lxp = i < nx - 1 ? label[q + 1] : kSolid;
+      const uint8_t lym = j > 0 ? label[q - nx] : kSolid;
+      const uint8_t lyp = j < g.ny - 1 ? label[q + nx] : kSolid;
+      const int bits = (lxm == kLiquid) | ((lxp == kLiquid) << 1) | ((lym == kLiquid) << 2) |
+                       ((lyp == kLiquid) << 3);
+      const int nns = (lxm != kSolid) + (lxp != kSolid) + (lym != kSolid) + (lyp != kSolid);
+      const float uxp = i < nx - 1 ? uf[q + 1] : 0.f;
+      const float vyp = j < g.ny - 1 ? vf[q + nx] : 0.f;
+      const float dvx = div_x(uxp - uf[q], g);
+      const float dvy = div_y(vyp - vf[q], g);
+      bf = dvx + dvy;
+      idx = k++;
+      info[idx] = (uint8_t)(bits | (nns << 4));
+      cell_of[idx] = q;
+      b[idx] = bf;
+    }
+    index_of[c[e]] = idx;
+    rhs[c[e]] = bf;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_pcg_clear(uint64_t* __restrict__ z, int64_t n,
+                                                   uint64_t* __restrict__ slots, int n_slots,
+                                                   unsigned* __restrict__ abort) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < n) z[t] = 0;
+  if (t < n_slots) slots[t] = 0;
+  if (t == 0) *abort = 0;
+}
+
+}  // namespace
+
+namespace {
+
+// The solve of F > 0 unknowns (F <= KPT NT gridDim.x).
+template <int KPT, bool REFINED, bool ONE>
+__device__ __forceinline__ void pcg_solve(const PersistentArgs& a, int F, float* lds,
+                                          PcgShared& sh) {
+  constexpr int NT = kPcgThreads;
+  CgScalars* sc = a.sc;
+  const int tid = threadIdx.x;
+  const int G = ONE ? 1 : (int)gridDim.x;
+  const int per = (F + G - 1) / G;
+  const int k0 = ONE ? 0 : min(F, (int)blockIdx.x * per);
+  const int k1 = min(F, k0 + per);
+  // LDS: lds[0] = 0, p of the block's unknowns (room for KPT per thread) and of its halo
+  // (pcg_halo_cap), then the halo's z and unknown indices
+  constexpr int cap = KPT * NT;
+  const int hcap = ONE ? 0 : pcg_halo_cap(per);
+  float* lp = lds + 1;
+  float* lph = lp + cap;
+  float* lzh = lph + hcap;
+  int* lhq = reinterpret_cast<int*>(lzh + hcap);
+  const CgParams& cp = a.cp;
+  if (tid < 32) {
+    (&sh.part[0][0][0])[tid] = 0.0;
+    (&sh.tot[0][0][0])[tid] = 0.0;
+  }
+  if (tid == 0) {
+    sh.ok = 1;
+    sh.n_halo = 0;
+    lds[0] = 0.f;
+  }
+  __syncthreads();
+
+  // unknown j of this thread: k = k0 + tid + j*NT, LDS slot k - k0.  nb: byte offsets in
+  // LDS of its left, right, down and up neighbours' p.  A neighbour that is not an
+  // unknown reads lds[0], so its term is + 0; a thread's j past the block's unknowns hold
+  // zeros and read lds[0]: the iterations run without branches and selects, every LDS
+  // read of a phase in flight at once.  A neighbour in another block gets a halo entry of
+  // its own (a cell may have two), and the unknown itself is in that neighbour's block's
+  // halo.
+  int nb[KPT][4];
+  float diag[KPT], invd[KPT];
+  unsigned exported = 0;
+  int nv = 0;  // valid unknowns: j = 0 .. nv - 1
+#define FSG_VALID(j) ((j) < nv)
+#define FSG_K(j) (k0 + tid + (j) * NT)
+  char* const ldsb = reinterpret_cast<char*>(lds);
+  auto ld_p = [&](int off) { return *reinterpret_cast<const float*>(ldsb + off); };
 #pragma unroll
   for (int j = 0; j < KPT; ++j) {
-    const int k = k0 + tid + j * kPcgThreads;
-    su[j] = sd[j] = 0;
+    const int k = FSG_K(j);
+    nb[j][0] = nb[j][1] = nb[j][2] = nb[j][3] = 0;
+    diag[j] = invd[j] = 0.f;
     if (k >= k1) continue;
-    valid |= 1u << j;
-    const uint8_t f = a.info[k];
-    const int2 ud = a.updn[k];
-    su[j] = ud.x - wb;
-    sd[j] = ud.y - wb;
-    infw |= (unsigned)(f & 15) << (4 * j);
-    nnsw |= (unsigned)((f >> 4) & 7) << (3 * j);
-    if (k - k0 < hw || k1 - 1 - k < hw) exported |= 1u << j;
+    nv = j + 1;
+    const unsigned f = a.info[k];
+    const int c = a.cell_of[k];
+    diag[j] = sel5((int)(f >> 4) & 7, cp.diag_tab);
+    invd[j] = sel5((int)(f >> 4) & 7, cp.invd_tab);
+    const int d[4] = {-1, 1, -a.nx, a.nx};
+    int q[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) q[t] = (f & (1u << t)) ? a.index_of[c + d[t]] : -1;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      if (q[t] < 0) continue;
+      int slot = q[t] - k0;
+      if (!ONE && (q[t] < k0 || q[t] >= k1)) {
+        const int h = atomicAdd(&sh.n_halo, 1);  // < hcap (pcg_halo_cap)
+        lhq[h] = q[t];
+        slot = cap + h;
+        exported |= 1u << j;
+      }
+      nb[j][t] = 4 * (slot + 1);
+    }
   }
-#define FSG_VALID(j) (valid & (1u << (j)))
-#define FSG_K(j) (k0 + tid + (j) * kPcgThreads)
-#define FSG_S(j) (hw + tid + (j) * kPcgThreads)
-  BarrierState bs{a.bar, a.bar + 1, 0u, a.partials};
-  CgScalars* sc = a.sc;
+  __syncthreads();
+  const int nh = ONE ? 0 : sh.n_halo;
+  PcgNet net{a.slots, a.zx, a.abort, 0u};
+  auto idle = [](int, int) { return true; };
+  // z of the halo, published for sum e: four words of a thread in flight at once
+  auto stage_halo = [&](int w, int nw) {
+    constexpr int U = 4;
+    bool good = true;
+    const int n = nw * 64;
+    for (int t0 = w * 64 + (tid & 63); t0 < nh; t0 += U * n) {
+      auto at = [&](int u) -> const uint64_t* {
+        const int t = t0 + u * n;
+        return t < nh ? net.z + lhq[t] : nullptr;
+      };
+      uint64_t v[U];
+      good &= poll(at, net.epoch, v, net.abort);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (t0 + u * n < nh) lzh[t0 + u * n] = __uint_as_float((uint32_t)v[u]);
+    }
+    return good;
+  };
 
   // optional mean removal of b (fully Neumann systems)
   float mean = 0.f;
@@ -154,11 +423,11 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
 #pragma unroll
     for (int j = 0; j < KPT; ++j)
       if (FSG_VALID(j)) v[0] += (double)a.b[FSG_K(j)];
-    if (!grid_reduce<1>(bs, v, sm)) return;
+    if (!grid_sum<1, ONE, false>(net, v, sh, idle)) return;
     mean = (float)v[0] / (float)F;
   }
 
-  float x[KPT], r[KPT], ap[KPT];
+  float x[KPT], r[KPT], z[KPT], p[KPT], ap[KPT];
   int total_it = 0, total_spmv = 0, sweeps = 0;
   double err = 0.0, b2 = 0.0, res2 = 0.0, thr2 = 0.0;
   // Start: x0 = 0 (Eigen's solve()), or with warm_start the previous solution kept
@@ -177,13 +446,12 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
       double x0 = 0.0;
       if (a.warm_start) {
         const int c = a.cell_of[k];
-        const unsigned f = (infw >> (4 * j)) & 15u;
         x0 = (double)a.xg[c];
-        double ax = (double)sel5((nnsw >> (3 * j)) & 7, cp.diag_tab) * x0;
-        if (f & 1u) ax += off * (double)a.xg[c - 1];
-        if (f & 2u) ax += off * (double)a.xg[c + 1];
-        if (f & 4u) ax += off * (double)a.xg[c - a.nx];
-        if (f & 8u) ax += off * (double)a.xg[c + a.nx];
+        double ax = (double)diag[j] * x0;
+        if (nb[j][0]) ax += off * (double)a.xg[c - 1];
+        if (nb[j][1]) ax += off * (double)a.xg[c + 1];
+        if (nb[j][2]) ax += off * (double)a.xg[c - a.nx];
+        if (nb[j][3]) ax += off * (double)a.xg[c + a.nx];
         rk = bk - ax;
       }
       if (REFINED) st_dev(a.x64 + k, x0);
@@ -191,7 +459,7 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
       v[0] += bk * bk;
       v[1] += rk * rk;
     }
-    if (!grid_reduce<2>(bs, v, sm)) return;
+    if (!grid_sum<2, ONE, REFINED>(net, v, sh, idle)) return;
     b2 = v[0];
     res2 = v[1];
     thr2 = a.outer_tol * a.outer_tol * b2;
@@ -201,18 +469,22 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
   while (true) {
     if (REFINED && !(b2 > 0.0 && res2 >= thr2 && sweeps < a.max_outer)) break;
     // ------------- one FP32 Jacobi-PCG solve of A e = r (x0 = 0) -------------
+    // z for the halo of the neighbouring blocks, tagged with the sum that follows
+    auto publish_z = [&](int j) {
+      if (!ONE && (exported & (1u << j)))
+        st_dev(net.z + FSG_K(j), tagged(__float_as_uint(z[j]), net.epoch + 1));
+    };
     double v2[2] = {0.0, 0.0};
 #pragma unroll
     for (int j = 0; j < KPT; ++j) {
-      x[j] = 0.f;
-      if (!FSG_VALID(j)) continue;
-      const float z = sel5((nnsw >> (3 * j)) & 7, cp.invd_tab) * r[j];
-      lz[FSG_S(j)] = z;
-      if (exported & (1u << j)) st_dev(ez + FSG_K(j), z);
+      x[j] = p[j] = 0.f;
+      z[j] = invd[j] * r[j];
+      publish_z(j);
       v2[0] += (double)(r[j] * r[j]);
-      v2[1] += (double)(r[j] * z);
+      v2[1] += (double)(r[j] * z[j]);
     }
-    if (!grid_reduce<2>(bs, v2, sm)) return;
+    for (int t = tid; t < nh; t += NT) lph[t] = 0.f;
+    if (!grid_sum<2, ONE, false>(net, v2, sh, stage_halo)) return;
     const float rhs = (float)v2[0];
     int it = 0, spmv = 0;
     float rr = rhs;
@@ -221,50 +493,32 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
     const float ref = REFINED ? rhs : (float)b2;
     float thr = tol * tol * ref;
     if (thr < FLT_MIN) thr = FLT_MIN;
-    if (ref != 0.f && rhs != 0.f && !(rr < thr)) {
+    if (ref != 0.f && rhs != 0.f && !(rr < thr) && cp.max_iter >= a.min_iter) {
       float abs_new = (float)v2[1];
       float beta = 0.f;
-      int par = 0;  // p_k goes to buffer par, p_{k-1} is read from par ^ 1
       while (true) {
-        const bool first = it == 0;
-        float* lp_new = par ? lp1 : lp0;
-        const float* lp_old = par ? lp0 : lp1;
-        float* ep_new = par ? ep1 : ep0;
-        const float* ep_old = par ? ep0 : ep1;
-        // stage the halo stripes [k0 - hw, k0) and [k1, k1 + hw)
-        for (int t = tid; t < 2 * hw; t += kPcgThreads) {
-          const int q = t < hw ? k0 - hw + t : k1 + (t - hw);
-          if (q < 0 || q >= F) continue;
-          lz[q - wb] = ld_dev(ez + q);
-          if (!first) const_cast<float*>(lp_old)[q - wb] = ld_dev(ep_old + q);
+        // phase A: p on the window (beta = 0 and p = 0 at first), its halo from the halo's z
+#pragma unroll
+        for (int j = 0; j < KPT; ++j) {
+          p[j] = z[j] + beta * p[j];
+          lp[tid + j * NT] = p[j];
         }
+        for (int t = tid; t < nh; t += NT) lph[t] = lzh[t] + beta * lph[t];
         __syncthreads();
-        // phase A: p_k (own, published) and Ap with neighbours' p_k recomputed
         double v1[1] = {0.0};
 #pragma unroll
         for (int j = 0; j < KPT; ++j) {
-          ap[j] = 0.f;
-          if (!FSG_VALID(j)) continue;
-          const int s = FSG_S(j);
-          const float pk = first ? lz[s] : lz[s] + beta * lp_old[s];
-          const unsigned f = (infw >> (4 * j)) & 15u;
-          float acc = sel5((nnsw >> (3 * j)) & 7, cp.diag_tab) * pk;
-          if (f & 1u) acc += cp.off * (first ? lz[s - 1] : lz[s - 1] + beta * lp_old[s - 1]);
-          if (f & 2u) acc += cp.off * (first ? lz[s + 1] : lz[s + 1] + beta * lp_old[s + 1]);
-          if (f & 4u) {
-            const int t2 = su[j];
-            acc += cp.off * (first ? lz[t2] : lz[t2] + beta * lp_old[t2]);
-          }
-          if (f & 8u) {
-            const int t2 = sd[j];
-            acc += cp.off * (first ? lz[t2] : lz[t2] + beta * lp_old[t2]);
-          }
+          const float nl = ld_p(nb[j][0]), nr = ld_p(nb[j][1]);
+          const float nd = ld_p(nb[j][2]), nu = ld_p(nb[j][3]);
+          float acc = diag[j] * p[j];
+          acc += cp.off * nl;
+          acc += cp.off * nr;
+          acc += cp.off * nd;
+          acc += cp.off * nu;
           ap[j] = acc;
-          v1[0] += (double)(pk * acc);
-          lp_new[s] = pk;
-          if (exported & (1u << j)) st_dev(ep_new + FSG_K(j), pk);
+          v1[0] += (double)(p[j] * acc);
         }
-        if (!grid_reduce<1>(bs, v1, sm)) return;
+        if (!grid_sum<1, ONE, false>(net, v1, sh, idle)) return;
         ++spmv;
         const float alpha = abs_new / (float)v1[0];
         // phase B
@@ -272,17 +526,14 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
         v2[1] = 0.0;
 #pragma unroll
         for (int j = 0; j < KPT; ++j) {
-          if (!FSG_VALID(j)) continue;
-          const int s = FSG_S(j);
-          x[j] = x[j] + alpha * lp_new[s];
           r[j] = r[j] - alpha * ap[j];
-          const float z = sel5((nnsw >> (3 * j)) & 7, cp.invd_tab) * r[j];
-          lz[s] = z;
-          if (exported & (1u << j)) st_dev(ez + FSG_K(j), z);
+          z[j] = invd[j] * r[j];
+          publish_z(j);
+          x[j] = x[j] + alpha * p[j];
           v2[0] += (double)(r[j] * r[j]);
-          v2[1] += (double)(r[j] * z);
+          v2[1] += (double)(r[j] * z[j]);
         }
-        if (!grid_reduce<2>(bs, v2, sm)) return;
+        if (!grid_sum<2, ONE, false>(net, v2, sh, stage_halo)) return;
         rr = (float)v2[0];
         if (rr < thr) break;
         const float abs_old = abs_new;
@@ -290,7 +541,6 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
         beta = abs_new / abs_old;
         ++it;
         if (it >= cp.max_iter) break;
-        par ^= 1;
       }
     }
     total_it += it;
@@ -306,7 +556,7 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
         st_dev(a.x64 + k, ld_dev(a.x64 + k) + (double)x[j]);
       }
     double w[1] = {0.0};
-    if (!grid_reduce<1>(bs, w, sm)) return;
+    if (!grid_sum<1, ONE, true>(net, w, sh, idle)) return;
     const double off = (double)cp.off;
     w[0] = 0.0;
 #pragma unroll
@@ -315,19 +565,21 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
         r[j] = 0.f;
         continue;
       }
+      __builtin_amdgcn_sched_barrier(0);  // one unknown's loads at a time: no spills
       const int k = FSG_K(j);
-      const unsigned f = (infw >> (4 * j)) & 15u;
-      double ax = (double)sel5((nnsw >> (3 * j)) & 7, cp.diag_tab) * ld_dev(a.x64 + k);
-      if (f & 1u) ax += off * ld_dev(a.x64 + k - 1);
-      if (f & 2u) ax += off * ld_dev(a.x64 + k + 1);
-      if (f & 4u) ax += off * ld_dev(a.x64 + su[j] + wb);
-      if (f & 8u) ax += off * ld_dev(a.x64 + sd[j] + wb);
+      double ax = (double)diag[j] * ld_dev(a.x64 + k);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (nb[j][t]) {
+          const int slot = nb[j][t] / 4 - 1;
+          ax += off * ld_dev(a.x64 + (slot < cap ? k0 + slot : lhq[slot - cap]));
+        }
       const double bk = (double)(cp.project_mean ? a.b[k] - mean : a.b[k]);
       const double rk = bk - ax;
       r[j] = (float)rk;
       w[0] += rk * rk;
     }
-    if (!grid_reduce<1>(bs, w, sm)) return;
+    if (!grid_sum<1, ONE, false>(net, w, sh, idle)) return;
     res2 = w[0];
     total_spmv += 1;
   }
@@ -345,12 +597,11 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
   }
 #undef FSG_VALID
 #undef FSG_K
-#undef FSG_S
   if (REFINED) err = b2 > 0.0 ? sqrt(res2 / b2) : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->iter = total_it;
     sc->spmv = total_spmv;
-    sc->err = err;
+    sc->err = cp.max_iter >= a.min_iter ? err : 0.0;
     sc->b64_norm2 = b2;
     sc->res64_norm2 = res2;
     sc->refine_sweeps = sweeps;
@@ -359,41 +610,100 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
   }
 }
 
-int pcg_max_kpt() { return 4; }
+// Many blocks, KPT unknowns per thread (F > 0).
+template <int KPT, bool REFINED>
+__global__ void __launch_bounds__(kPcgThreads) k_pcg(PersistentArgs a) {
+  extern __shared__ float lds[];
+  __shared__ PcgShared sh;
+  pcg_solve<KPT, REFINED, false>(a, *a.n_fluid, lds, sh);
+}
+
+// One block.  The launch may be sized by a bound of F, so the unknowns per thread (up to
+// KMAX) are chosen here: an iteration costs instructions for each of them, used or not.
+// 512 threads: 256 take 1.95 us per iteration at 3,800 unknowns against 1.59, and the
+// same at 530.
+template <int KMAX, bool REFINED>
+__global__ void __launch_bounds__(kPcgThreads) k_pcg_one(PersistentArgs a) {
+  constexpr int NT = kPcgThreads;
+  extern __shared__ float lds[];
+  __shared__ PcgShared sh;
+  const int F = *a.n_fluid;
+  if (threadIdx.x == 0) {
+    *a.abort = 0;  // (more blocks: k_pcg_clear)
+    if (F == 0) {
+      a.sc->iter = a.sc->spmv = a.sc->refine_sweeps = 0;
+      a.sc->err = 0.0;
+    }
+  }
+  if (F == 0) return;
+  if (F <= NT) pcg_solve<1, REFINED, true>(a, F, lds, sh);
+  else if (F <= 2 * NT) pcg_solve<2, REFINED, true>(a, F, lds, sh);
+  else if (F <= 4 * NT) pcg_solve<4, REFINED, true>(a, F, lds, sh);
+  else if (F <= 8 * NT) pcg_solve<8, REFINED, true>(a, F, lds, sh);
+  else if constexpr (KMAX >= 16) pcg_solve<16, REFINED, true>(a, F, lds, sh);
+}
+
+}  // namespace
+
+int pcg_tiles(const Geom& g) { return ((g.nx + 31) / 32) * ((g.ny + 31) / 32); }
+void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts) {
+  k_pcg_count<<<pcg_tiles(g), 256, 0, s>>>(g, label, counts);
+}
+void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
+                     int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
+                     float* rhs, uint8_t* info) {
+  k_pcg_fill<<<pcg_tiles(g), 256, 0, s>>>(g, label, offsets, index_of, cell_of, uf, vf, b, rhs,
+                                          info);
+}
 
 size_t pcg_lds_bytes(int F, int grid, int nx) {
   const int per = (F + grid - 1) / grid;
   return (size_t)3 * (per + 2 * nx) * sizeof(float);
 }
+size_t pcg_slot_words(int grid) { return (size_t)2 * grid * kSlotWords; }
+
+namespace {
+template <int KPT>
+const void* pcg_kernel(bool refined) {
+  return refined ? (const void*)k_pcg<KPT, true> : (const void*)k_pcg<KPT, false>;
+}
+}  // namespace
 
 hipError_t launch_pcg(hipStream_t s, const PersistentArgs& a, int grid, int kpt) {
   void* args[] = {(void*)&a};
-  const size_t lds = pcg_lds_bytes(a.F_actual, grid, a.nx);
-  const void* f = nullptr;
   const bool ref = a.refined != 0;
+  const void* f = nullptr;
+  if (grid == 1) {
+    int cap = kPcgThreads;  // the kernel's KPT x threads for any F <= F_actual
+    while (cap < a.F_actual) cap *= 2;
+    const size_t lds = (size_t)(cap + 1) * sizeof(float);
+    if (a.F_actual > (ref ? kPcgOneRefined : kPcgOneUnknowns)) return hipErrorInvalidValue;
+    f = ref ? (const void*)k_pcg_one<8, true> : (const void*)k_pcg_one<16, false>;
+    return hipLaunchKernel(f, dim3(1), dim3(kPcgThreads), args, lds, s);
+  }
+  const int per = (a.F_actual + grid - 1) / grid;
+  if (per > 1024 * kpt) return hipErrorInvalidValue;
+  const size_t lds = (size_t)(1 + 1024 * kpt + 3 * pcg_halo_cap(per)) * sizeof(float);
+  const int n_slots = (int)pcg_slot_words(grid);
+  const int64_t n = std::max<int64_t>(a.F_actual, n_slots);
+  k_pcg_clear<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(a.zx, a.F_actual, a.slots, n_slots,
+                                                          a.abort);
   switch (kpt) {
-    case 1: f = ref ? (const void*)k_pcg<1, true> : (const void*)k_pcg<1, false>; break;
-    case 2: f = ref ? (const void*)k_pcg<2, true> : (const void*)k_pcg<2, false>; break;
-    // 4 unknowns per thread only in the FP32 form: the refined form's FP64 state
-    // exceeds the 128 VGPRs of a 1024-thread block there (it would spill)
-    case 4:
-      if (ref) return hipErrorInvalidValue;
-      f = (const void*)k_pcg<4, false>;
-      break;
+    case 1: f = pcg_kernel<2>(ref); break;
+    case 2: f = pcg_kernel<4>(ref); break;
+    case 4: f = pcg_kernel<8>(ref); break;
     default: return hipErrorInvalidValue;
   }
   return hipLaunchCooperativeKernel(f, dim3(grid), dim3(kPcgThreads), args, lds, s);
 }
 
 hipError_t pcg_set_lds_limit(size_t max_bytes) {
-  const void* fs[] = {(const void*)k_pcg<1, false>, (const void*)k_pcg<2, false>,
-                      (const void*)k_pcg<4, false>, (const void*)k_pcg<1, true>,
-                      (const void*)k_pcg<2, true>};
-  for (const void* f : fs) {
-    hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)max_bytes);
-    if (e != hipSuccess) return e;
-  }
+  for (bool ref : {false, true})
+    for (const void* f : {pcg_kernel<2>(ref), pcg_kernel<4>(ref), pcg_kernel<8>(ref)}) {
+      hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                         (int)max_bytes);
+      if (e != hipSuccess) return e;
+    }
   return hipSuccess;
 }
 

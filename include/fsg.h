@@ -77,8 +77,10 @@ extern "C" {
                         shift of both coordinates its Vec2 form implies) */
 
 /* Pressure solver forms (all replace Eigen::ConjugateGradient, FluidSolver.h:114). */
-#define FSG_SOLVER_PLAIN 0      /* FP32 Jacobi-PCG, 3 kernels per iteration, host loop */
-#define FSG_SOLVER_PERSISTENT 1 /* FP32 Jacobi-PCG in one persistent cooperative kernel */
+#define FSG_SOLVER_PLAIN 0      /* FP32 Jacobi-PCG; one launch per solve up to about 2^20
+                                   unknowns, else 3 kernels per iteration, host loop */
+#define FSG_SOLVER_PERSISTENT 1 /* FP32 Jacobi-PCG in one persistent kernel, with warm
+                                   start and a settable launch shape */
 #define FSG_SOLVER_REFINED 2    /* FP32 PCG inside FP64 iterative refinement, FP64
                                    residual and reductions, persistent kernel */
 #define FSG_SOLVER_MG 3         /* CG preconditioned by a geometric-multigrid V-cycle
@@ -104,12 +106,12 @@ typedef struct fsg_params {
   int32_t integrator;     /* FSG_RK3 */
   int32_t solver;         /* FSG_SOLVER_PLAIN */
   int32_t project_mean;   /* 0: remove the mean of b (fully Neumann systems) */
-  int32_t check_every;    /* plain solver: iterations enqueued between host checks */
+  int32_t check_every;    /* plain solver, many-launch form: iterations between host checks */
   double refine_inner_tol;/* refined solver: relative tolerance of each FP32 inner solve */
   int32_t refine_max_outer;/* refined solver: maximum FP64 refinement sweeps */
   int32_t record_ext_info; /* 1: fsg_step also records the extension sources */
   int32_t pcg_blocks;     /* persistent solvers: blocks (0: automatic) */
-  int32_t pcg_kpt;        /* persistent solvers: unknowns per thread, 1/2/4 (refined form:
+  int32_t pcg_kpt;        /* persistent solvers: 1024s of unknowns per block, 1/2/4 (refined form:
                              1/2), 0: automatic */
   int32_t warm_start;     /* persistent, refined and multigrid solvers: 1 starts CG
                              from the previous solve's pressure (same stopping test
