@@ -56,7 +56,14 @@ namespace fsg {
 namespace {
 
 constexpr int kT = 256;         // threads of the vector kernels and the level-0 tiles
-constexpr int kTileBig = 1024;  // threads of the tiles of the smaller levels
+// Threads per tile of the levels below 0 (few_tiles): a level of at most one tile
+// per CU leaves CUs idle and its time is one tile's chain of LDS phases, which 1024
+// threads shorten; with more tiles two workgroups of 512 share a CU and one's waits are
+// hidden by the other.  V-cycle per step, 512 against 1024 threads on every level: 513 x
+// 385 cells 584 / 558 us, 1024^2 810 / 783 us; one 2048^2 level-1 launch (1024 tiles)
+// down 12.9 / 16.6 us, up 10.5 / 11.7 us.
+constexpr int kTileFew = 1024, kTileMany = 512;
+inline bool few_tiles(int tiles) { return tiles <= 256; }  // 256 CUs
 constexpr uint8_t kAct = kMgUnknown;  // info bit: the cell is an unknown
 constexpr int kTileEmptyBit = (int)0x80000000u;  // k_mg_tile_map: the tile holds no unknown
 constexpr uint8_t kWall = 0x40;   // info bit: SOLID (also used for cells outside the grid)
@@ -882,6 +889,7 @@ struct MgXr {
   double* part_rr;  // out: one partial |r|^2 per block
 };
 
+template <int CT>
 __device__ __forceinline__ void coarse_stage(const MgCoarseArgs& a, double* part_rz,
                                              bool coherent);
 
@@ -908,9 +916,51 @@ struct BlockSpan {
   }
 };
 
-// S sweeps (2 on level 0, 2 .. kMgMaxSweeps on the levels below): the right-hand side
-// and info on [-(S + 1), 33 + S), sweep k on a ring one cell narrower than sweep k - 1,
-// the last on [-2, 34); the sweeps alternate between the x1 and x2 buffers.
+// A thread's cells in the tile kernels: a vertical strip of R cells (R even) of the
+// W x W window around the tile, W strips side by side, G of them on top of each other.
+// The strip's info, right-hand side and x stay in registers through the sweeps; LDS
+// holds x for the neighbours only (row pitch PW: one column of padding on either side,
+// one row above and below).  A tile kernel on few tiles is bound by the VALU issue of the
+// one CU that a tile runs on, so what counts is instructions per cell and sweep: a strip
+// of 4 reads 10 values for its 4 cells, all at fixed offsets from one address, where a
+// thread per cell read 7 for one and computed its indices anew in every sweep.
+// Per launch, a thread per cell before and strips now: 2048^2 level 0 down 52.2 -> 46 us,
+// up 29.7 -> 23.5, level 1 down 18.9 -> 12.9, up 14.5 -> 10.5; what is left there is memory
+// (down0 reads 33 and writes 16 bytes a cell) and one round trip at either end.
+// A sweep runs over the whole window.  The cells a sweep cannot know (their neighbours
+// lie outside the window) hold values of no meaning, one ring more with each sweep; the
+// window is wide enough that nothing that is stored depends on them.
+template <int W, int NT>
+struct Strip {
+  static constexpr int kMaxG = NT / W;
+  static constexpr int kR = (W + kMaxG - 1) / kMaxG;
+  static constexpr int R = kR + (kR & 1);
+  static constexpr int G = (W + R - 1) / R;
+  static constexpr int HP = G * R;  // rows, the last strips' unused ones included
+  static constexpr int PW = W + 2;
+  static constexpr int N = (HP + 2) * PW;
+};
+
+// K x's neighbour sums of a strip: the x of the cells left, right, below and above each,
+// added in this order.
+template <int R, int PW, typename T>
+__device__ __forceinline__ void strip_nbrs(const T* __restrict__ x, int base, const T (&own)[R],
+                                           T (&sum)[R]) {
+  T l[R], r[R];
+  const T dn = x[base - PW], up = x[base + R * PW];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    l[q] = x[base + q * PW - 1];
+    r[q] = x[base + q * PW + 1];
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    sum[q] = l[q] + r[q] + (q == 0 ? dn : own[q - 1]) + (q == R - 1 ? up : own[q + 1]);
+}
+
+// S sweeps (2 or 3 on level 0, 2 .. kMgMaxSweeps on the levels below): the right-hand
+// side and info on the window [-(S + 1), 33 + S) around the tile; after the S sweeps x is
+// known on [-2, 34), the residual on [-1, 33).
 template <bool L0, int NT, bool XR = false, bool TAIL = false, int S = 2>
 __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omega, float omega2,
                                                  int it,
@@ -926,10 +976,10 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   const BlockSpan clock(span);
   __shared__ double sm[NT / 64];
   __shared__ int s_last;
-  // TAIL (the last tile level, 1024 threads): the restriction is stored
-  // device-coherent and the last workgroup to finish runs the one-workgroup stage on
-  // it, in place of a k_mg_coarse launch.  The arrival count is ordered after every
-  // wave's stores, as in a grid barrier, but nobody waits.
+  // TAIL (the last tile level): the restriction is stored device-coherent and the last
+  // workgroup to finish runs the one-workgroup stage on it, in place of a k_mg_coarse
+  // launch.  The arrival count is ordered after every wave's stores, as in a grid
+  // barrier, but nobody waits.
   // inlined: as a call its LDS accesses would go through flat addresses
   auto run_tail = [&]() __attribute__((always_inline)) {
     if constexpr (TAIL) {
@@ -942,7 +992,7 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
       __syncthreads();
       if (s_last) {
         if (threadIdx.x == 0) st_dev(ticket, 0u);  // ready for the next launch
-        coarse_stage(ca, nullptr, true);
+        coarse_stage<NT>(ca, nullptr, true);
       }
     }
   };
@@ -956,40 +1006,53 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   const int tm = tmap ? tmap[blockIdx.x] : 0;
   const int tile = tmap ? tm & ~kTileEmptyBit : xcd_tile(blockIdx.x, gridDim.x);
   const bool empty = tmap ? tm < 0 : tflag && !tflag[tile];
-  constexpr int W3 = 34 + 2 * S, W2 = W3 - 2, W1 = 34;  // S = 2: 38, 36, 34
-  constexpr int W4 = W3 + 2;  // fused form: x_new on [-(S + 2), 34 + S)
+  constexpr int W = 34 + 2 * S, O = S + 1;  // the window and the tile's offset in it
+  using St = Strip<W, NT>;
+  constexpr int R = St::R, PW = St::PW;
   constexpr int WC = 18;  // coarse cells of the tile and their neighbours
   const int tiles_x = (c.nx + 15) >> 4;
   // each XCD takes one band of consecutive tiles, so halo rows are shared in its L2
   const int bx = tile % tiles_x, by = tile / tiles_x;
   const int fi0 = bx * 32, fj0 = by * 32;
   const bool do_xr = XR && it > 0;
+  // the strip: column wx, rows wy0 .. wy0 + R - 1 of the window
+  const int wx = threadIdx.x % W, g = threadIdx.x / W, wy0 = g * R;
+  const bool strip = g < St::G;
+  const int base = strip ? (wy0 + 1) * PW + wx + 1 : PW + 1;
+  const int gi = fi0 - O + wx, gj = fj0 - O + wy0;
+  int cell[R];
+  bool in[R], own[R];  // the cell lies in the grid; and in the tile
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    in[q] = strip && wy0 + q < W && gi >= 0 && gi < f.nx && gj + q >= 0 && gj + q < f.ny;
+    own[q] = in[q] && wx >= O && wx < O + 32 && wy0 + q >= O && wy0 + q < O + 32;
+    cell[q] = in[q] ? gi + (gj + q) * f.nx : 0;
+  }
   // Without the fused update, every load of a tile holding unknowns is issued before
   // the stop test's reads (their round trips overlap; a finished solve drops them) and
   // before the first LDS store (a load outside the grid reads cell 0 and is replaced
   // by the boundary value).
-  constexpr int NC = (WC * WC + NT - 1) / NT, NF = (W3 * W3 + NT - 1) / NT;
-  uint8_t cv[NC], fv[NF];
-  float rv[NF];
-  if (!empty && !do_xr) {
+  constexpr int NC = (WC * WC + NT - 1) / NT;
+  uint8_t cv[NC], fv[R];
+  float rv[R];
+  auto load_coarse = [&] {
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
       const int t = threadIdx.x + k * NT;
       const int I = bx * 16 + t % WC - 1, J = by * 16 + t / WC - 1;
-      const bool in = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
-      const uint8_t v = c.inf[in ? I + J * c.nx : 0];
-      cv[k] = in ? v : kWall;
+      const bool inc = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
+      const uint8_t v = c.inf[inc ? I + J * c.nx : 0];
+      cv[k] = inc ? v : kWall;
     }
+  };
+  if (!empty && !do_xr) {
+    load_coarse();
 #pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      const int i = fi0 + t % W3 - (S + 1), j = fj0 + t / W3 - (S + 1);
-      const bool in = t < W3 * W3 && i >= 0 && i < f.nx && j >= 0 && j < f.ny;
-      const int q = in ? i + j * f.nx : 0;
-      const uint8_t fq = f.inf[q];
-      const float rq = f.r[q];
-      fv[k] = in ? fq : 0;
-      rv[k] = in ? rq : 0.f;
+    for (int q = 0; q < R; ++q) {
+      const uint8_t fq = f.inf[cell[q]];
+      const float rq = f.r[cell[q]];
+      fv[q] = in[q] ? fq : 0;
+      rv[q] = in[q] ? rq : 0.f;
     }
   }
   if (check) {
@@ -1001,11 +1064,10 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     clock.end();
     return;
   }
-  __shared__ float s_r[W3 * W3], s_x1[W3 * W3], s_x2[W2 * W2];
-  // the last sweep lands in x2 (S even) or x1 (S odd); the residual reuses the other
-  // buffer, dead by then, so the smaller footprint lets more tiles share a CU
-  float* const s_res = (S & 1) ? s_x2 : s_x1;
-  const float* const s_xs = (S & 1) ? s_x1 : s_x2;
+  // sweeps alternate between the two buffers; the residual takes the one that is free
+  __shared__ float s_x[2][St::N];
+  __shared__ uint8_t s_cinf[WC * WC];
+  __shared__ double s_xn[XR ? St::N : 1];
   float wk[kMgMaxSweeps];
 #pragma unroll
   for (int k = 0; k < kMgMaxSweeps; ++k) wk[k] = sw.w[k];
@@ -1013,8 +1075,6 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     wk[0] = omega;
     wk[1] = omega2;
   }
-  __shared__ uint8_t s_inf[W3 * W3], s_cinf[WC * WC];
-  __shared__ double s_xn[XR ? W4 * W4 : 1];
   if (empty) {
     // no unknown in the tile on either level: its outputs are zero; written once per
     // solve (earlier solves may have left other values)
@@ -1047,40 +1107,37 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   }
   if (do_xr) {
     // every load of the tile first (a load outside the grid reads cell 0 and is
-    // replaced by the boundary value), then alpha, then the stores to LDS
-    constexpr int N4 = (W4 * W4 + NT - 1) / NT;
-    double bv[NF], xo[N4];
-    float pv[N4];
+    // replaced by the boundary value), then alpha, then the stores to LDS.  x_new is
+    // formed on the window and the ring around it, which other threads take: 4 (W + 1)
+    // cells, bottom and top row first
+    double bv[R], xo[R];
+    float pv[R];
+    load_coarse();
 #pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      const int t = threadIdx.x + k * NT;
-      const int I = bx * 16 + t % WC - 1, J = by * 16 + t / WC - 1;
-      const bool in = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
-      const uint8_t v = c.inf[in ? I + J * c.nx : 0];
-      cv[k] = in ? v : kWall;
+    for (int q = 0; q < R; ++q) {
+      // a strip past the window's rows holds the ring's first row too: the neighbour
+      // above the window's last one
+      const bool inx = in[q] || (strip && wy0 + q == W && gi >= 0 && gi < f.nx &&
+                                 gj + q >= 0 && gj + q < f.ny);
+      const int cx = inx ? gi + (gj + q) * f.nx : 0;
+      const uint8_t fq = f.inf[cell[q]];
+      const double bq = xr.b[cell[q]], xq = xr.x_old[cx];
+      const float pq = xr.p[cx];
+      fv[q] = in[q] ? fq : 0;
+      bv[q] = in[q] ? bq : 0.0;
+      xo[q] = inx ? xq : 0.0;
+      pv[q] = inx ? pq : 0.f;
     }
-#pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      const int i = fi0 + t % W3 - (S + 1), j = fj0 + t / W3 - (S + 1);
-      const bool in = t < W3 * W3 && i >= 0 && i < f.nx && j >= 0 && j < f.ny;
-      const int q = in ? i + j * f.nx : 0;
-      const uint8_t fq = f.inf[q];
-      const double bq = xr.b[q];
-      fv[k] = in ? fq : 0;
-      bv[k] = in ? bq : 0.0;
-    }
-#pragma unroll
-    for (int k = 0; k < N4; ++k) {
-      const int t = threadIdx.x + k * NT;
-      const int i = fi0 + t % W4 - (S + 2), j = fj0 + t / W4 - (S + 2);
-      const bool in = t < W4 * W4 && i >= 0 && i < f.nx && j >= 0 && j < f.ny;
-      const int q = in ? i + j * f.nx : 0;
-      const double xq = xr.x_old[q];
-      const float pq = xr.p[q];
-      xo[k] = in ? xq : 0.0;
-      pv[k] = in ? pq : 0.f;
-    }
+    const int rt = threadIdx.x;
+    const int rx = rt < 2 * PW ? (rt < PW ? rt : rt - PW) : (rt - 2 * PW < W ? 0 : PW - 1);
+    const int ry = rt < PW ? 0 : rt < 2 * PW ? W + 1 : 1 + (rt - 2 * PW) % W;
+    static_assert(NT >= 4 * (W + 1), "a thread per ring cell");
+    const bool ring = rt < 4 * (W + 1);
+    const int ri = fi0 - O - 1 + rx, rj = fj0 - O - 1 + ry;
+    const bool rin = ring && ri >= 0 && ri < f.nx && rj >= 0 && rj < f.ny;
+    const int rq = rin ? ri + rj * f.nx : 0;
+    const double rxo = xr.x_old[rq];
+    const float rp = xr.p[rq];
     const double pq = sum_part<NT>(xr.part_pq, xr.n_pq, sm);
     const double alpha = chk.sc->rho[(it - 1) & 1] / pq;
 #pragma unroll
@@ -1088,45 +1145,30 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
       const int t = threadIdx.x + k * NT;
       if (t < WC * WC) s_cinf[t] = cv[k];
     }
+    double xn[R];
 #pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      if (t < W3 * W3) s_inf[t] = fv[k];
-    }
+    for (int q = 0; q < R; ++q) xn[q] = xo[q] + alpha * (double)pv[q];
+    if (strip)
 #pragma unroll
-    for (int k = 0; k < N4; ++k) {
-      const int t = threadIdx.x + k * NT;
-      if (t < W4 * W4) s_xn[t] = xo[k] + alpha * (double)pv[k];
-    }
+      for (int q = 0; q < R; ++q)
+        if (wy0 + q < W) s_xn[base + q * PW] = xn[q];
+    if (ring) s_xn[rx + ry * PW] = rin ? rxo + alpha * (double)rp : 0.0;
     __syncthreads();
-    // r = b' - K x_new on [-(S + 1), 33 + S) (cells outside the grid hold x = 0 and
-    // add 0); the tile's own cells store x_new and r and add to |r|^2
-    double acc = 0.0;
+    // r = b' - K x_new on the window (cells outside the grid hold x = 0 and add 0); the
+    // tile's own cells store x_new and r and add to |r|^2
+    double sn[R], acc = 0.0;
+    strip_nbrs<R, PW>(s_xn, base, xn, sn);
 #pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      if (t >= W3 * W3) break;
-      const int li = t % W3, lj = t / W3;
-      const uint8_t fq = fv[k];
-      const int q4 = (li + 1) + (lj + 1) * W4;
-      const double xc = s_xn[q4];
+    for (int q = 0; q < R; ++q) {
       double r64 = 0.0;
-      if (is_act(fq)) {
-        double sn = 0.0;
-        sn += s_xn[q4 - 1];
-        sn += s_xn[q4 + 1];
-        sn += s_xn[q4 - W4];
-        sn += s_xn[q4 + W4];
-        r64 = bv[k] - ((double)(fq & 7) * xc - sn);
-        acc += (li > S && li < 33 + S && lj > S && lj < 33 + S) ? r64 * r64 : 0.0;
+      if (is_act(fv[q])) {
+        r64 = bv[q] - ((double)(fv[q] & 7) * xn[q] - sn[q]);
+        acc += own[q] ? r64 * r64 : 0.0;
       }
-      const float rv = (float)r64;
-      s_r[t] = rv;
-      s_x1[t] = is_act(fq) ? wk[0] * rv * inv_nns(fq) : 0.f;
-      const int i = fi0 + li - (S + 1), j = fj0 + lj - (S + 1);
-      if (li > S && li < 33 + S && lj > S && lj < 33 + S && i < f.nx && j < f.ny) {
-        xr.x_new[i + j * f.nx] = is_act(fq) ? xc : 0.0;
-        f.r[i + j * f.nx] = rv;
+      rv[q] = (float)r64;
+      if (own[q]) {
+        xr.x_new[cell[q]] = is_act(fv[q]) ? xn[q] : 0.0;
+        f.r[cell[q]] = rv[q];
       }
     }
     write_part<NT>(acc, xr.part_rr, sm);
@@ -1138,87 +1180,73 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
       const int t = threadIdx.x + k * NT;
       if (t < WC * WC) s_cinf[t] = cv[k];
     }
-#pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      if (t < W3 * W3) {
-        s_inf[t] = fv[k];
-        s_r[t] = rv[k];
-        s_x1[t] = is_act(fv[k]) ? wk[0] * rv[k] * inv_nns(fv[k]) : 0.f;
-      }
-    }
   }
+  // the first sweep from x = 0
+  float nn[R], inv[R], x[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    nn[q] = nns_of(fv[q]);
+    inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
+    x[q] = wk[0] * rv[q] * inv[q];
+  }
+  int cur = 0;
+  auto put = [&](float* dst, const float (&v)[R]) {
+    if (strip)
+#pragma unroll
+      for (int q = 0; q < R; ++q) dst[base + q * PW] = v[q];
+  };
+  put(s_x[cur], x);
   __syncthreads();
-  // sweeps 2 .. S: from the buffer of window win (offset d inside the right-hand
-  // side's window) to one of window win - 2; the last lands in s_xs ([-2, 34))
+  float sum[R];
 #pragma unroll
   for (int k = 2; k <= S; ++k) {
-    const int win = W3 - 2 * (k - 2), wout = win - 2, d = k - 2;
-    const float* xin = (k & 1) ? s_x2 : s_x1;
-    float* xout = (k & 1) ? s_x1 : s_x2;
+    strip_nbrs<R, PW>(s_x[cur], base, x, sum);
     const float wgt = wk[k - 1];
-    for (int t = threadIdx.x; t < wout * wout; t += NT) {
-      const int li = t % wout + 1, lj = t / wout + 1;
-      const int q = li + lj * win;
-      const int qr = (li + d) + (lj + d) * W3;
-      const uint8_t fv = s_inf[qr];
-      float v = 0.f;
-      if (is_act(fv)) {
-        const float n = nns_of(fv), x = xin[q];
-        const float kx = n * x - (xin[q - 1] + xin[q + 1] + xin[q - win] + xin[q + win]);
-        v = x + wgt * (s_r[qr] - kx) * inv_nns(fv);
-      }
-      xout[t] = v;
-    }
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
+    cur ^= 1;
+    put(s_x[cur], x);
     __syncthreads();
   }
-  for (int t = threadIdx.x; t < W1 * W1; t += NT) {
-    const int li = t % W1, lj = t / W1;  // fine offset li - 1, lj - 1
-    constexpr int WS = 36;               // the last sweep's window, [-2, 34)
-    const int q = (li + 1) + (lj + 1) * WS;
-    const int q3 = (li + S) + (lj + S) * W3;
-    const uint8_t fv = s_inf[q3];
-    const float x = s_xs[q];
-    float res = 0.f;
-    if (is_act(fv)) {
-      const float kx = nns_of(fv) * x - (s_xs[q - 1] + s_xs[q + 1] + s_xs[q - WS] + s_xs[q + WS]);
-      res = s_r[q3] - kx;
-    }
-    s_res[t] = res;
-    const int oi = li - 1, oj = lj - 1;
-    if (oi >= 0 && oi < 32 && oj >= 0 && oj < 32) {
-      const int i = fi0 + oi, j = fj0 + oj;
-      if (i < f.nx && j < f.ny) f.xs[i + j * f.nx] = x;
-    }
+  strip_nbrs<R, PW>(s_x[cur], base, x, sum);
+  cur ^= 1;
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const float res = is_act(fv[q]) ? rv[q] - (nn[q] * x[q] - sum[q]) : 0.f;
+    if (own[q]) f.xs[cell[q]] = x[q];
+    sum[q] = res;
   }
+  put(s_x[cur], sum);
   __syncthreads();
+  const float* const s_res = s_x[cur] + (O + 1) * PW + O + 1;  // the tile's first cell
   if (threadIdx.x < 256) {
     const int ci = threadIdx.x & 15, cj = threadIdx.x >> 4;
     const int I = bx * 16 + ci, J = by * 16 + cj;
     if (I < c.nx && J < c.ny) {
-      const int cc = I + J * c.nx;
       float v = 0.f;
       if (is_act(s_cinf[(ci + 1) + (cj + 1) * WC])) {
-        // fine offsets 2ci-1 .. 2ci+2 are s_res columns 2ci .. 2ci+3
+        // fine offsets 2ci-1 .. 2ci+2 and 2cj-1 .. 2cj+2
         const float w[4] = {0.25f, 0.75f, 0.75f, 0.25f};
+        float t[4][4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float* row = s_res + (2 * cj + b) * W1 + 2 * ci;
-          const float s = 0.25f * row[0] + 0.75f * row[1] + 0.75f * row[2] + 0.25f * row[3];
-          v += w[b] * s;
-        }
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) t[b][e] = s_res[(2 * cj - 1 + b) * PW + 2 * ci - 1 + e];
         // the four children moved the weight of their wall neighbours here
         auto ci_at = [&](int di, int dj) { return s_cinf[(ci + 1 + di) + (cj + 1 + dj) * WC]; };
 #pragma unroll
+        for (int b = 0; b < 4; ++b)
+          v += w[b] * (0.25f * t[b][0] + 0.75f * t[b][1] + 0.75f * t[b][2] + 0.25f * t[b][3]);
+#pragma unroll
         for (int b = 1; b <= 2; ++b)
 #pragma unroll
-          for (int a = 1; a <= 2; ++a) {
-            const int dx = a == 1 ? -1 : 1, dy = b == 1 ? -1 : 1;
-            const float m = moved_weight(ci_at(dx, 0), ci_at(0, dy), ci_at(dx, dy));
-            v += m * s_res[(2 * cj + b) * W1 + 2 * ci + a];
+          for (int e = 1; e <= 2; ++e) {
+            const int dx = e == 1 ? -1 : 1, dy = b == 1 ? -1 : 1;
+            v += moved_weight(ci_at(dx, 0), ci_at(0, dy), ci_at(dx, dy)) * t[b][e];
           }
       }
-      put_r(c.r + cc, v);
+      put_r(c.r + I + J * c.nx, v);
     }
   }
   run_tail();
@@ -1228,12 +1256,11 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   }
 }
 
-// Up: level l+1 -> level l.  A block owns 32 x 32 fine cells.  In LDS: the coarse
-// solution around the tile, r and info on [-S, 32 + S), the corrected x = xs + P e
-// there, then S post-sweeps, each on a ring one cell narrower than the one before (the
-// last on the tile, written to xo), alternating between the xc and y buffers.  S = 2
-// (level 0), or 2 .. kMgMaxSweeps on the levels below (sweep k uses w[k - 1]).
-// Level 0 also forms the partial of r.z (z = xo) for the next direction.
+// Up: level l+1 -> level l.  A block owns 32 x 32 fine cells, on the window [-S, 32 + S)
+// in strips as k_mg_down: the corrected x = xs + P e there, then S post-sweeps, the last
+// one's tile written to xo.  In LDS: the coarse solution and info around the tile, and x
+// in two buffers.  S = 2 or 3 on level 0, 2 .. kMgMaxSweeps on the levels below (sweep k
+// uses w[k - 1]).  Level 0 also forms the partial of r.z (z = xo) for the next direction.
 template <bool L0, int NT, int S = 2>
 __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega, float omega2,
                                                const CgScalars* sc, double* __restrict__ part_rz,
@@ -1241,12 +1268,14 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
                                                MgSweeps sw, const int* __restrict__ tmap) {
   static_assert(S >= 2 && S <= kMgMaxSweeps && (!L0 || S <= 3),
                 "level 0 takes two or three sweeps; smaller levels 2 .. kMgMaxSweeps");
-  constexpr int W2 = 32 + 2 * S, W1 = W2 - 2;  // S = 2: 36, 34
-  // coarse cells from fi0 / 2 - (S / 2 + 1): every coarse neighbour of the fine cells
-  // [-S, 32 + S)
+  constexpr int W = 32 + 2 * S;
+  using St = Strip<W, NT>;
+  constexpr int R = St::R, PW = St::PW;
+  // coarse cells from fi0 / 2 - (S / 2 + 1): every coarse neighbour of the window's cells
   constexpr int WC = 18 + S, CO = S / 2 + 1;
-  __shared__ float s_r[W2 * W2], s_xc[W2 * W2], s_y1[W1 * W1], s_e[WC * WC];
-  __shared__ uint8_t s_inf[W2 * W2], s_cinf[WC * WC];
+  static_assert(St::HP / 2 + (S & 1 ? 0 : 1) < WC, "the strips' coarse rows lie in the frame");
+  __shared__ float s_x[2][St::N], s_e[WC * WC];
+  __shared__ uint8_t s_cinf[WC * WC];
   __shared__ double sm[NT / 64];
   float wk[kMgMaxSweeps];
 #pragma unroll
@@ -1265,36 +1294,44 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
   const int bx = tile % tiles_x, by = tile / tiles_x;
   const int fi0 = bx * 32, fj0 = by * 32;
   const int ci0 = (fi0 >> 1) - CO, cj0 = (fj0 >> 1) - CO;  // coarse frame origin
+  const int wx = threadIdx.x % W, g = threadIdx.x / W, wy0 = g * R;
+  const bool strip = g < St::G;
+  const int base = strip ? (wy0 + 1) * PW + wx + 1 : PW + 1;
+  const int gi = fi0 - S + wx, gj = fj0 - S + wy0;
+  int cell[R];
+  bool in[R], own[R];  // the cell lies in the grid; and in the tile
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    in[q] = strip && wy0 + q < W && gi >= 0 && gi < f.nx && gj + q >= 0 && gj + q < f.ny;
+    own[q] = in[q] && wx >= S && wx < S + 32 && wy0 + q >= S && wy0 + q < S + 32;
+    cell[q] = in[q] ? gi + (gj + q) * f.nx : 0;
+  }
   // every load of a tile holding unknowns is issued before the stop flag's value is
   // known (one memory round trip for both; the loads of a finished solve are dropped)
   // and before the first LDS store (a load outside the grid reads cell 0 and is
   // replaced by the boundary value)
-  constexpr int NC = (WC * WC + NT - 1) / NT, NF = (W2 * W2 + NT - 1) / NT;
-  uint8_t cv[NC], fv[NF];
-  float ev[NC], rv[NF], xv[NF];
+  constexpr int NC = (WC * WC + NT - 1) / NT;
+  uint8_t cv[NC], fv[R];
+  float ev[NC], rv[R], x[R];
   if (!empty) {
 #pragma unroll
     for (int k = 0; k < NC; ++k) {
       const int t = threadIdx.x + k * NT;
       const int I = ci0 + t % WC, J = cj0 + t / WC;
-      const bool in = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
-      const int q = in ? I + J * c.nx : 0;
+      const bool inc = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
+      const int q = inc ? I + J * c.nx : 0;
       const float e = c.xo[q];
       const uint8_t ci = c.inf[q];
-      ev[k] = in ? e : 0.f;
-      cv[k] = in ? ci : kWall;
+      ev[k] = inc ? e : 0.f;
+      cv[k] = inc ? ci : kWall;
     }
 #pragma unroll
-    for (int k = 0; k < NF; ++k) {
-      const int t = threadIdx.x + k * NT;
-      const int i = fi0 + t % W2 - S, j = fj0 + t / W2 - S;
-      const bool in = t < W2 * W2 && i >= 0 && i < f.nx && j >= 0 && j < f.ny;
-      const int q = in ? i + j * f.nx : 0;
-      const uint8_t fq = f.inf[q];
-      const float rq = f.r[q], xq = f.xs[q];
-      fv[k] = in ? fq : 0;
-      rv[k] = in ? rq : 0.f;
-      xv[k] = in ? xq : 0.f;
+    for (int q = 0; q < R; ++q) {
+      const uint8_t fq = f.inf[cell[q]];
+      const float rq = f.r[cell[q]], xq = f.xs[cell[q]];
+      fv[q] = in[q] ? fq : 0;
+      rv[q] = in[q] ? rq : 0.f;
+      x[q] = in[q] ? xq : 0.f;
     }
   }
   if (sc->done) return;
@@ -1316,76 +1353,59 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
       s_cinf[t] = cv[k];
     }
   }
+  __syncthreads();
+  // the correction: two coarse columns (the cells' own and its x neighbour) times the
+  // strip's coarse rows, wy0 / 2 + (S even) and on; window rows of even number lie in odd
+  // fine rows where S is odd
+  float nn[R], inv[R];
+  {
+    constexpr bool kOdd = (S & 1) != 0;
+    constexpr int NR = R / 2 + (kOdd ? 1 : 2);
+    const int il = ((wx - S) >> 1) + CO, inl = il + (((wx - S) & 1) ? 1 : -1);
+    const int q0 = strip ? (wy0 / 2) * WC + il : WC, q1 = strip ? (wy0 / 2) * WC + inl : WC;
+    float e0[NR], e1[NR];
+    uint8_t f0[NR], f1[NR];
 #pragma unroll
-  for (int k = 0; k < NF; ++k) {
-    const int t = threadIdx.x + k * NT;
-    if (t < W2 * W2) {
-      s_inf[t] = fv[k];
-      s_r[t] = rv[k];
-      s_xc[t] = xv[k];
+    for (int k = 0; k < NR; ++k) {
+      e0[k] = s_e[q0 + k * WC];
+      e1[k] = s_e[q1 + k * WC];
+      f0[k] = s_cinf[q0 + k * WC];
+      f1[k] = s_cinf[q1 + k * WC];
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const bool odd = ((q & 1) != 0) != kOdd;  // the fine row is odd
+      const int J = kOdd ? (q + 1) / 2 : 1 + q / 2, Jn = odd ? J + 1 : J - 1;
+      const float pe = prolong_value(e0[J], e1[J], f1[J], e0[Jn], f0[Jn], e1[Jn], f1[Jn]);
+      x[q] = is_act(fv[q]) ? x[q] + pe : 0.f;
+      nn[q] = nns_of(fv[q]);
+      inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
     }
   }
-  __syncthreads();
-  for (int t = threadIdx.x; t < W2 * W2; t += NT) {
-    if (!is_act(s_inf[t])) {
-      s_xc[t] = 0.f;
-      continue;
-    }
-    const int i = fi0 + t % W2 - S, j = fj0 + t / W2 - S;
-    const int I = i >> 1, J = j >> 1;  // floor for the halo left of / below 0 too
-    const int In = (i & 1) ? I + 1 : I - 1;
-    const int Jn = (j & 1) ? J + 1 : J - 1;
-    const int q00 = (I - ci0) + (J - cj0) * WC, q10 = (In - ci0) + (J - cj0) * WC;
-    const int q01 = (I - ci0) + (Jn - cj0) * WC, q11 = (In - ci0) + (Jn - cj0) * WC;
-    s_xc[t] += prolong_value(s_e[q00], s_e[q10], s_cinf[q10], s_e[q01], s_cinf[q01], s_e[q11],
-                             s_cinf[q11]);
-  }
-  __syncthreads();
-  // post-sweeps 1 .. S-1: from the buffer of window win (offset d inside the
-  // right-hand side's window) to one of window win - 2
+  // post-sweeps 1 .. S-1 through LDS, the last straight to the outputs
+  float sum[R];
+  int cur = 0;
 #pragma unroll
-  for (int k = 1; k < S; ++k) {
-    const int win = W2 - 2 * (k - 1), wout = win - 2, d = k - 1;
-    const float* xin = (k & 1) ? s_xc : s_y1;
-    float* xout = (k & 1) ? s_y1 : s_xc;
-    const float wgt = wk[k - 1];
-    for (int t = threadIdx.x; t < wout * wout; t += NT) {
-      const int li = t % wout + 1, lj = t / wout + 1;
-      const int q = li + lj * win;
-      const int qr = (li + d) + (lj + d) * W2;
-      const uint8_t fv = s_inf[qr];
-      float v = 0.f;
-      if (is_act(fv)) {
-        const float n = nns_of(fv), x = xin[q];
-        const float kx = n * x - (xin[q - 1] + xin[q + 1] + xin[q - win] + xin[q + win]);
-        v = x + wgt * (s_r[qr] - kx) * inv_nns(fv);
-      }
-      xout[t] = v;
-    }
+  for (int k = 1; k <= S; ++k) {
+    if (strip)
+#pragma unroll
+      for (int q = 0; q < R; ++q) s_x[cur][base + q * PW] = x[q];
     __syncthreads();
+    strip_nbrs<R, PW>(s_x[cur], base, x, sum);
+    const float wgt = wk[k - 1];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
+    cur ^= 1;
   }
-  // the last post-sweep, on the tile, from the window [-1, 33) (in y1 for S even,
-  // in xc for S odd)
-  constexpr int WL = 34;
-  const float* const s_yl = (S & 1) ? s_xc : s_y1;
   double rz = 0.0;
-  const float wl = wk[S - 1];
-  for (int t = threadIdx.x; t < 32 * 32; t += NT) {
-    const int oi = t & 31, oj = t >> 5;
-    const int i = fi0 + oi, j = fj0 + oj;
-    if (i >= f.nx || j >= f.ny) continue;
-    const int q = (oi + 1) + (oj + 1) * WL;
-    const int q2 = (oi + S) + (oj + S) * W2;
-    const uint8_t fv = s_inf[q2];
-    float v = 0.f;
-    if (is_act(fv)) {
-      const float n = nns_of(fv), x = s_yl[q];
-      const float kx = n * x - (s_yl[q - 1] + s_yl[q + 1] + s_yl[q - WL] + s_yl[q + WL]);
-      v = x + wl * (s_r[q2] - kx) * inv_nns(fv);
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    if (own[q]) {
+      const float v = is_act(fv[q]) ? x[q] : 0.f;
+      f.xo[cell[q]] = v;
+      if (L0) rz += (double)rv[q] * (double)v;
     }
-    f.xo[i + j * f.nx] = v;
-    if (L0) rz += (double)s_r[q2] * (double)v;
-  }
   if (L0) write_part<NT>(rz, part_rz, sm);
 }
 
@@ -1417,6 +1437,7 @@ constexpr float kCoarsestOmega = 0.8f;  // damped Jacobi on the coarsest level (
 // result is left in X when nl == 1, else in T.
 // Inlined into its kernels so that R, X, T and INF are addressed as LDS (a called
 // function sees generic pointers and goes through the slower flat path).
+template <int CT>
 __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx,
                                              const int* __restrict__ lny,
                                              const int* __restrict__ loff, float w, float w2,
@@ -1431,7 +1452,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
     for (int sw = 0; sw < trunc; ++sw) {
       const float* src = ((trunc - sw) & 1) ? X : T;
       float* dst = ((trunc - sw) & 1) ? T : X;
-      for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+      for (int q = threadIdx.x; q < n; q += CT) {
         float v = 0.f;
         if (is_act(INF[q])) {
           const float rn = inv_nns(INF[q]);
@@ -1456,7 +1477,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
     const uint8_t* inf = INF + o;
     const float inv_nx = 1.0f / (float)nx;
     // two sweeps from zero; the first sweep's neighbour values w r / n formed on the fly
-    for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < n; q += CT) {
       float v = 0.f;
       if (is_act(inf[q])) {
         int i, j;
@@ -1481,7 +1502,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
       x[q] = v;
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < n; q += CT) {
       float v = 0.f;
       if (is_act(inf[q])) {
         int i, j;
@@ -1493,7 +1514,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
     __syncthreads();
     const int cnx = lnx[l + 1], cny = lny[l + 1], co = loff[l + 1];
     const float inv_cnx = 1.0f / (float)cnx;
-    for (int q = threadIdx.x; q < cnx * cny; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < cnx * cny; q += CT) {
       int I, J;
       small_divmod(q, cnx, inv_cnx, I, J);
       float v = 0.f;
@@ -1586,7 +1607,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
     const float* e = (l + 1 == nl - 1 ? X : T) + co;
     const uint8_t* cinf = INF + co;
     const float inv_nx = 1.0f / (float)nx;
-    for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < n; q += CT) {
       float v = 0.f;
       if (is_act(inf[q])) {
         int i, j;
@@ -1610,7 +1631,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
       t[q] = v;
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < n; q += CT) {
       float v = 0.f;
       if (is_act(inf[q])) {
         const float nn = nns_of(inf[q]);
@@ -1621,7 +1642,7 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
       x[q] = v;
     }
     __syncthreads();
-    for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+    for (int q = threadIdx.x; q < n; q += CT) {
       float v = 0.f;
       if (is_act(inf[q])) {
         const float nn = nns_of(inf[q]);
@@ -1650,6 +1671,7 @@ __device__ __forceinline__ void kclock_end(unsigned long long* clk, unsigned lon
 // LDS, cycle, store level lc's result (and, when the hierarchy starts here, the r.z
 // partial).  `coherent`: the right-hand side was written by other workgroups of the
 // same launch with device-coherent stores, so it is read the same way.
+template <int CT>
 __device__ __forceinline__ void coarse_stage(const MgCoarseArgs& a, double* part_rz,
                                              bool coherent) {
   __shared__ double sm[2 * 16];
@@ -1670,24 +1692,24 @@ __device__ __forceinline__ void coarse_stage(const MgCoarseArgs& a, double* part
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(a.inf_all);
     uint32_t* dst = reinterpret_cast<uint32_t*>(INF);
-    for (int q = threadIdx.x; q < tot / 4; q += kCoarseThreads) dst[q] = src[q];
+    for (int q = threadIdx.x; q < tot / 4; q += CT) dst[q] = src[q];
     const int n0 = a.nx[a.lc] * a.ny[a.lc];
-    for (int q = threadIdx.x; q < n0; q += kCoarseThreads)
+    for (int q = threadIdx.x; q < n0; q += CT)
       R[q] = coherent ? ld_dev(a.r_in + q) : a.r_in[q];
   }
   __syncthreads();
-  coarse_cycle(nl, s_lv, s_lv + kMgMaxLevels, s_lv + 2 * kMgMaxLevels, a.omega, a.omega2,
+  coarse_cycle<CT>(nl, s_lv, s_lv + kMgMaxLevels, s_lv + 2 * kMgMaxLevels, a.omega, a.omega2,
                a.sweeps, R, X, T, INF, a.trunc);
   const int n = a.nx[a.lc] * a.ny[a.lc];
   const float* res = nl == 1 && a.trunc == 0 ? X : T;
   double rz = 0.0;
-  for (int q = threadIdx.x; q < n; q += kCoarseThreads) {
+  for (int q = threadIdx.x; q < n; q += CT) {
     a.x_out[q] = res[q];
     rz += (double)R[q] * (double)res[q];
   }
   if (part_rz) {
     double v[1] = {rz};
-    block_sum<1, kCoarseThreads>(v, sm);
+    block_sum<1, CT>(v, sm);
     if (threadIdx.x == 0) part_rz[0] = v[0];
   }
 }
@@ -1707,7 +1729,7 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse(MgCoarseArgs a, Mg
     kclock_end(clk, t0);
     return;
   }
-  coarse_stage(a, part_rz, false);
+  coarse_stage<kCoarseThreads>(a, part_rz, false);
   if (clk) {
     __syncthreads();
     kclock_end(clk, t0);
@@ -1789,7 +1811,7 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_scene_coarse(SceneCoarseA
   __syncthreads();
   const int cl = t.nl - 1;
   const int sweeps = 2 * (t.nx[cl] > t.ny[cl] ? t.nx[cl] : t.ny[cl]) + 8;
-  coarse_cycle(t.nl, t.nx, t.ny, t.off, a.omega, a.omega2, sweeps, R, X, T, INF, a.trunc);
+  coarse_cycle<kCoarseThreads>(t.nl, t.nx, t.ny, t.off, a.omega, a.omega2, sweeps, R, X, T, INF, a.trunc);
   const float* res = t.nl == 1 && a.trunc == 0 ? X : T;
   for (int q = threadIdx.x; q < n0; q += kCoarseThreads)
     a.x_out[(size_t)(t.cx + q % nx) + (size_t)(t.cy + q / nx) * a.pitch] = res[q];
@@ -2464,13 +2486,13 @@ hipError_t mg_set_lds_limit(size_t bytes) {
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (e != hipSuccess) return e;
   // the last tile level's down kernel hosts the same stage (its own static LDS aside)
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_down<false, kTileBig, false, true>),
+  e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (e != hipSuccess) return e;
-  for (const void* f : {reinterpret_cast<const void*>(&k_mg_down<false, kTileBig, false, true, 3>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileBig, false, true, 4>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileBig, false, true, 5>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileBig, false, true, 6>)}) {
+  for (const void* f : {reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 3>),
+                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 4>),
+                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 5>),
+                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 6>)}) {
     e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
   }
@@ -2683,8 +2705,7 @@ void launch_mg_down(hipStream_t s, MgHost& m, int l, int it, int max_iter, doubl
   // the stop test: level 0's kernel, or level 1's in the fused form (level 0 forms
   // the residual it tests)
   const int check = l == (m.fused ? 1 : 0) ? 1 : 0;
-  // level 0: m.l0_threads per tile (256 by default: many tiles); smaller levels: 1024
-  // threads, so that each LDS phase of the few tiles takes one or two passes
+  // level 0: m.l0_threads per tile (256 by default: many tiles); the others: few_tiles
   if (l == 0) {
     // fused form: iteration it - 1's update, the buffers k_mg_xr would use then
     const MgXr xr = m.fused ? MgXr{m.x[(it + 1) & 1], m.x[it & 1], m.p[it & 1], m.b, m.part_pq,
@@ -2717,17 +2738,22 @@ void launch_mg_down(hipStream_t s, MgHost& m, int l, int it, int max_iter, doubl
       go_s(std::integral_constant<int, kT>{});
   } else {
     // the last tile level also runs the one-workgroup stage (mg_tail_coarse): its own
-    // instance, so that the other levels (and every level of a batch) carry none of it;
-    // m.level_sweeps (2 or 4) sweeps before the coarse correction
+    // instance, so that the other levels (and every level of a batch) carry none of it
+    // (its coarse level holds at most kMgCoarseCells cells, so it has at most 64 tiles);
+    // m.level_sweeps sweeps before the coarse correction
     const MgSweeps sw = mg_sweeps(m);
     auto go = [&](auto ns) {
       constexpr int S = decltype(ns)::value;
       if (l == m.lc - 1 && mg_tail_coarse(m))
-        k_mg_down<false, kTileBig, false, true, S><<<blocks, kTileBig, m.coarse_lds, s>>>(
+        k_mg_down<false, kTileFew, false, true, S><<<blocks, kTileFew, m.coarse_lds, s>>>(
             mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
             m.tflag_l[l], MgXr{}, nullptr, m.coarse, m.ticket, sw, nullptr);
+      else if (few_tiles(mg_up_blocks(m.nx[l], m.ny[l])))
+        k_mg_down<false, kTileFew, false, false, S><<<blocks, kTileFew, 0, s>>>(
+            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
+            m.tflag_l[l], MgXr{}, nullptr, MgCoarseArgs{}, nullptr, sw, nullptr);
       else
-        k_mg_down<false, kTileBig, false, false, S><<<blocks, kTileBig, 0, s>>>(
+        k_mg_down<false, kTileMany, false, false, S><<<blocks, kTileMany, 0, s>>>(
             mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
             m.tflag_l[l], MgXr{}, nullptr, MgCoarseArgs{}, nullptr, sw, nullptr);
     };
@@ -2775,10 +2801,14 @@ void launch_mg_up(hipStream_t s, const MgHost& m, int l, int it, CgScalars* sc) 
   else {
     auto go = [&](auto ns) {
       constexpr int S = decltype(ns)::value;
-      k_mg_up<false, kTileBig, S><<<blocks, kTileBig, 0, s>>>(mg_level(m, l), mg_level(m, l + 1),
-                                                              m.coarse.omega, m.coarse.omega2, sc,
-                                                              nullptr, it, m.tflag_l[l],
-                                                              mg_sweeps(m), nullptr);
+      if (few_tiles(blocks))
+        k_mg_up<false, kTileFew, S><<<blocks, kTileFew, 0, s>>>(
+            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
+            m.tflag_l[l], mg_sweeps(m), nullptr);
+      else
+        k_mg_up<false, kTileMany, S><<<blocks, kTileMany, 0, s>>>(
+            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
+            m.tflag_l[l], mg_sweeps(m), nullptr);
     };
     switch (m.level_sweeps) {
       case 3: go(std::integral_constant<int, 3>{}); break;
