@@ -76,15 +76,23 @@ def kernel_bytes(name, nx, ny, P, levels=None):
     }
     if name in table:
         return table[name]
+    if name == "cg_mg_cycle":
+        if levels is not None:
+            return None
+        # the levels from the first of at most 64 tiles of 32 x 32 on: right-hand side and
+        # info read, the pre-smoothed values written and read, the result written (26 B,
+        # values between levels are 8 bytes), a level's coarse level read and written
+        n = [(nx, ny)]
+        while len(n) < len(cells):
+            n.append(((n[-1][0] + 1) // 2, (n[-1][1] + 1) // 2))
+        l1 = next(l for l in range(1, lc + 1) if -(-n[l][0] // 32) * -(-n[l][1] // 32) <= 64)
+        return (sum(26.0 * cells[l] + 18.0 * cells[l + 1] for l in range(l1, lc)) +
+                16.0 * cells[lc] + float(sum(cells[lc:])))
     for pre, fine_b, coarse_b in (("cg_mg_down", 9.0, 5.0), ("cg_mg_up", 13.0, 5.0)):
         if name.startswith(pre):
             tail = name[len(pre):].rstrip("+")
             l = int(tail)
-            b = fine_b * cells[l] + coarse_b * cells[l + 1]
-            if pre == "cg_mg_down" and levels is None and l == lc - 1 and lc >= 2:
-                # the last tile level's down kernel also runs the one-workgroup stage
-                b += table["cg_mg_coarse"]
-            return b
+            return fine_b * cells[l] + coarse_b * cells[l + 1]
     return None
 
 
@@ -144,7 +152,6 @@ MEASURED_TRAFFIC_1024 = {
     "cg_mg_down0": (2.0 * 3201.4 + 6303.8) * 1024,
     "cg_mg_up0": (2.0 * 1828.3 + 1309.8) * 1024,
     "cg_mg_dir": (2.0 * 1229.6 + 1637.5) * 1024,
-    "cg_mg_down4": (2.0 * 66.2 + 20.8) * 1024,
     "particle_scatter": (2.0 * 8065.4 + 18469.3) * 1024,
     "particle_gather": (2.0 * 10294.5 + 16676.3) * 1024,
     "face_update": (2.0 * 12821.0 + 28672.2) * 1024,
@@ -156,6 +163,10 @@ TUNE_STEPS = 8
 
 # a kernel moving less than this per launch is bound by launch and barrier latency
 ROOFLINE_MIN_BYTES = 1e6
+
+# the multigrid levels of few tiles and the one-workgroup stage, in one launch: a chain of
+# waits between its workgroups
+LATENCY_KERNELS = {"cg_mg_cycle"}
 
 # timers that wrap more than one kernel (or one kernel at several levels)
 MULTI_KERNEL_TIMERS = {"cg_mg_setup", "cg_mg_finish", "cg_mg_down7+", "cg_mg_up7+", "bucket_order"}
@@ -830,7 +841,8 @@ def main():
             return b / n if b is not None and n else None
         return kernel_bytes(k, args.n, args.n, P)
 
-    hbm = {k: v for k, v in single.items() if (launch_bytes(k) or 0.0) >= ROOFLINE_MIN_BYTES}
+    hbm = {k: v for k, v in single.items()
+           if k not in LATENCY_KERNELS and (launch_bytes(k) or 0.0) >= ROOFLINE_MIN_BYTES}
     latency = sorted(((k, v) for k, v in single.items() if k not in hbm), key=lambda kv: -kv[1])
     pool = hbm or single
     dominant = args.roofline_kernel or (max(pool, key=pool.get) if pool else None)

@@ -417,6 +417,9 @@ void extend_sweeps(fsg_domain* h, bool record_info) {
   swap_vel(h);
 }
 
+// LDS of the one-workgroup stage, at most
+constexpr size_t kCoarseLdsLimit = 128 * 1024;
+
 // Multigrid hierarchy: halve (rounding up) until both sides are <= 4 cells; the
 // levels from the first one of <= kMgCoarseCells cells run in one workgroup.
 int mg_prepare(fsg_domain* h) {
@@ -448,6 +451,7 @@ int mg_prepare(fsg_domain* h) {
       return fail(h, FSG_E_INVALID, "multigrid solver: grid too elongated for the hierarchy");
     m.fused = m.lc >= 2;
   }
+  m.l1 = mg_cycle_level(m);
   // cell offsets of the one-workgroup levels (its LDS layout and its info array)
   MgCoarseArgs& a = m.coarse;
   int off = 0;
@@ -466,9 +470,13 @@ int mg_prepare(fsg_domain* h) {
       ok &= dalloc(h, &m.inf[l], n) == hipSuccess;
     else if (coarse_inf)
       m.inf[l] = coarse_inf + a.off[l];
-    ok &= dalloc(h, &m.rl[l], n) == hipSuccess;
-    ok &= dalloc(h, &m.xs[l], n) == hipSuccess;
-    ok &= dalloc(h, &m.xo[l], n) == hipSuccess;
+    // the levels of the shared launch exchange their values in its own words
+    const bool shared = m.l1 < m.lc && l >= m.l1;
+    if (!shared || l == m.l1) {
+      ok &= dalloc(h, &m.rl[l], n) == hipSuccess;
+      ok &= dalloc(h, &m.xo[l], n) == hipSuccess;
+    }
+    if (!shared) ok &= dalloc(h, &m.xs[l], n) == hipSuccess;
   }
   const size_t C = ncell(h);
   ok &= dalloc(h, &m.b, C) == hipSuccess;
@@ -494,10 +502,10 @@ int mg_prepare(fsg_domain* h) {
   if (m.per_scene)
     for (int l = 1; l < m.lc; ++l)
       ok &= dalloc(h, &m.tflag_l[l], (size_t)mg_up_blocks(m.nx[l], m.ny[l])) == hipSuccess;
-  if (!m.per_scene && m.lc >= 2) {
-    ok &= dalloc(h, &m.ticket, 1) == hipSuccess;
-    if (ok) ok &= hipMemsetAsync(m.ticket, 0, sizeof(unsigned), h->stream) == hipSuccess;
-  }
+  ok &= mg_cycle_prepare(m, h->batch ? h->batch->S : 1, [&](size_t bytes) -> void* {
+    uint8_t* p = nullptr;
+    return dalloc(h, &p, bytes) == hipSuccess ? p : nullptr;
+  });
   if (!ok) return fail(h, FSG_E_NOMEM, "multigrid solver: device allocation failed");
   m.lab[0] = h->label;
   a.lc = m.lc;
@@ -513,9 +521,16 @@ int mg_prepare(fsg_domain* h) {
   a.x_out = m.xo[m.lc];
   // The one-workgroup levels hold at most ~2 x kMgCoarseCells cells (13 bytes each);
   // the kernel's LDS limit is raised once, process-wide, to a fixed 128 KiB.
-  constexpr size_t kCoarseLdsLimit = 128 * 1024;
   m.coarse_lds = (size_t)a.total * (3 * sizeof(float) + 1);
   if (h->batch) m.coarse_lds = (size_t)h->batch->stride * (3 * sizeof(float) + 1);
+  a.words = 0;
+  if (h->batch)
+    for (const fsg::SceneCoarse& c : h->batch->coarse)
+      m.coarse_lds = std::max(m.coarse_lds, 2 * (size_t)c.words * sizeof(float));
+  else {
+    m.stage_words = mg_stage_words(m.nlev - m.lc, m.nx + m.lc, m.ny + m.lc, kCoarseLdsLimit, false);
+    m.coarse_lds = std::max(m.coarse_lds, 2 * (size_t)m.stage_words * sizeof(float));
+  }
   if (m.coarse_lds > kCoarseLdsLimit)
     return fail(h, FSG_E_INVALID, "multigrid solver: coarse levels exceed the LDS budget");
   if (mg_set_lds_limit(kCoarseLdsLimit) != hipSuccess)
@@ -539,6 +554,7 @@ fsg::SceneCoarseArgs scene_coarse_args(const fsg_domain* h) {
   a.omega = m.coarse.omega;
   a.omega2 = m.coarse.omega2;
   a.trunc = m.coarse.trunc;
+  a.lds = m.coarse_lds;
   return a;
 }
 
@@ -573,6 +589,7 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
     m.coarse.omega = m.coarse.omega2 = 0.8f;
   }
   m.coarse.trunc = h->prm.mg_coarse_sweeps;
+  m.coarse.words = m.coarse.trunc == 0 ? m.stage_words : 0;
   m.fused = !h->batch && m.lc >= 2 && h->prm.mg_fuse_update != 0;
   m.l0_threads = h->prm.mg_tile_threads;
   m.level_sweeps = h->prm.mg_level_sweeps;
@@ -602,8 +619,7 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   int& prev_iters = adj_rhs ? h->mg_prev_iters_adj : h->mg_prev_iters;
   int it = 0, batch = std::max(last_iters + 1, 4), more = 2;
   CgScalars hs{};
-  // one timer name per level (the last tile level's down kernel also runs the
-  // one-workgroup stage)
+  // one timer name per level with launches of its own
   static const char* const kDownNames[8] = {"cg_mg_down0", "cg_mg_down1", "cg_mg_down2",
                                             "cg_mg_down3", "cg_mg_down4", "cg_mg_down5",
                                             "cg_mg_down6", "cg_mg_down7+"};
@@ -617,26 +633,37 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   // iteration q's head, the kernels after it return at once.
   const int head_levels = h->batch ? 0 : m.fused ? 2 : 1;
   const bool whole_head = !h->batch && m.lc < head_levels;
+  // the levels with launches of their own; the others (cycle) share one, which in the
+  // fused form runs the stop test if it begins with level 1
+  const bool cycle = mg_has_cycle(m);
+  const int own_levels = cycle ? m.l1 : m.lc;
+  const bool cycle_head = m.fused && m.l1 == 1;
   auto enqueue_part = [&](int it, bool head) {
     if (h->batch && head)
       timed(h, "cg_mg_check", [&] {
         launch_mgb_check(h->stream, h->batch->cg_args(h->g.nx, h->g.ny), it, max_iter, tol, h->sc);
       });
     if (!whole_head)
-      for (int l = 0; l < m.lc; ++l)
+      for (int l = 0; l < own_levels; ++l)
         if ((l < head_levels) == head)
           timed(h, kDownNames[std::min(l, 7)],
                 [&] { launch_mg_down(h->stream, m, l, it, max_iter, tol, h->sc); });
+    if (cycle && cycle_head == head)
+      timed(h, "cg_mg_cycle", [&] {
+        fsg::SceneCoarseArgs sa;
+        if (h->batch) sa = scene_coarse_args(h);
+        launch_mg_cycle(h->stream, m, it, max_iter, tol, h->sc, h->batch ? &sa : nullptr);
+      });
     if (head != whole_head) return;
     if (whole_head)
-      for (int l = 0; l < m.lc; ++l)
+      for (int l = 0; l < own_levels; ++l)
         timed(h, kDownNames[std::min(l, 7)],
               [&] { launch_mg_down(h->stream, m, l, it, max_iter, tol, h->sc); });
-    if (h->batch)
+    if (h->batch && !cycle)
       timed(h, "cg_mg_coarse", [&] { launch_mg_scene_coarse(h->stream, scene_coarse_args(h), h->sc); });
-    else if (!mg_tail_coarse(m))
+    else if (!cycle)
       timed(h, "cg_mg_coarse", [&] { launch_mg_coarse(h->stream, m, it, max_iter, tol, h->sc); });
-    for (int l = m.lc - 1; l >= 0; --l)
+    for (int l = own_levels - 1; l >= 0; --l)
       timed(h, kUpNames[std::min(l, 7)], [&] { launch_mg_up(h->stream, m, l, it, h->sc); });
     if (h->batch) {
       const fsg::MgbArgs ba = h->batch->cg_args(h->g.nx, h->g.ny);
@@ -693,6 +720,7 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
     HIPCHK(h, hipStreamSynchronize(h->stream));
     memcpy(&hs, &h->hsc->sc, sizeof(hs));
     if (F < 0) F = h->hsc->n_fluid;
+    if (hs.stuck) return fail(h, FSG_E_HIP, "multigrid solver: a wait on the device ran out");
     return FSG_OK;
   };
   if (use_graph && h->mg_graphs.iters == 0) {
@@ -1854,6 +1882,7 @@ int fsg_batch_create(fsg_domain** out, int32_t n_scenes, const int32_t* nx, cons
     }
     if (c.nx[c.nl - 1] * c.ny[c.nl - 1] > 64) return bail(FSG_E_INVALID, "scene hierarchy");
     c.total = (off + 3) & ~3;
+    c.words = mg_stage_words(c.nl, c.nx, c.ny, kCoarseLdsLimit, true);
     b->stride = std::max(b->stride, c.total);
     b->coarse.push_back(c);
   }

@@ -5,20 +5,44 @@
 
 namespace fsg {
 
+// DPP move of a double; lanes without a source take 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+// Sums over the wave, in lane 63, the values' steps interleaved (register moves only: a
+// shuffle tree of doubles costs 12 LDS-latency exchanges).
+template <int CTRL, int ROWS, int NV>
+__device__ __forceinline__ void dpp_step(double (&v)[NV]) {
+  double t[NV];
+#pragma unroll
+  for (int q = 0; q < NV; ++q) t[q] = dpp_f64<CTRL, ROWS>(v[q]);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) v[q] += t[q];
+}
+template <int NV>
+__device__ __forceinline__ void wave_sums(double (&v)[NV]) {
+  dpp_step<0x111, 0xF>(v);
+  dpp_step<0x112, 0xF>(v);
+  dpp_step<0x114, 0xF>(v);
+  dpp_step<0x118, 0xF>(v);
+  dpp_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
+  dpp_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
+}
 // Sum NV doubles over a block of NT threads; the result is returned in every
-// thread.  The order is fixed (wave shuffle tree, then waves in order), so equal
-// inputs give bit-identical sums in every block and every launch.
+// thread.  The order is fixed (the lanes' register moves, then waves in order), so equal
+// inputs give bit-identical sums in every block and every launch.  A tree of shuffles in
+// place of the moves keeps the LDS pipe of a CU with 32 waves busy for 1.3 us.
 // sm: NV * (NT / 64) doubles of LDS.
 template <int NV, int NT>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* sm) {
   constexpr int NW = NT / 64;
-#pragma unroll
-  for (int q = 0; q < NV; ++q)
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_down(v[q], off, 64);
+  wave_sums(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   __syncthreads();
-  if (lane == 0)
+  if (lane == 63)
 #pragma unroll
     for (int q = 0; q < NV; ++q) sm[q * NW + wave] = v[q];
   __syncthreads();

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include <math.h>
+#include <functional>
 
 #include "fsg_device.h"
 
@@ -163,6 +164,8 @@ struct CgScalars {
   unsigned long long total_unknown_iters;
   long long total_solves;
   double rho[2];         // multigrid form: r.z of the current / previous direction
+  int stuck;             // multigrid form: 1 if a wait between tasks ran out (k_mg_cycle)
+  int pad_;
 };
 
 // The scalars a solve's host loop reads back after each batch of iterations, written by
@@ -253,10 +256,34 @@ struct MgCoarseArgs {
   int lc, nlev, total, sweeps;
   float omega, omega2;
   int trunc;  // 0: V-cycle over levels lc .. nlev-1; k > 0: k Jacobi sweeps on level lc only
+  int words;  // > 0: the cells are kept in registers, this many words of LDS per buffer
   int nx[kMgMaxLevels], ny[kMgMaxLevels], off[kMgMaxLevels];
   const uint8_t* inf_all;  // info of levels lc .. nlev-1, contiguous (offsets off[l] - off[lc])
   const float* r_in;  // right-hand side of level lc
   float* x_out;       // cycle result of level lc
+};
+
+// The V-cycle's smaller tile levels and the one-workgroup stage in one launch: its levels
+// (lv[nl] is the one-workgroup level), the tasks' order and the words that carry values
+// between them (a float and the launch's number).
+struct MgCycleLevel {
+  int nx = 0, ny = 0, tiles_x = 0;
+  unsigned down0 = 0, up0 = 0;       // first task of the level's tiles going down / up
+  const uint8_t* inf = nullptr;
+  const uint8_t* tflag = nullptr;    // a batch: the tiles that hold an unknown
+  const float* r = nullptr;          // the first level's right-hand side
+  float* xo = nullptr;               // the first level's result
+  unsigned long long* tr = nullptr;  // right-hand side (below the first level)
+  unsigned long long* ts = nullptr;  // after pre-smoothing (tile levels)
+  unsigned long long* te = nullptr;  // result (below the first level)
+};
+struct MgCycleArgs {
+  int nl = 0;                            // tile levels, 0: none
+  unsigned coarse0 = 0, up0 = 0, n_tasks = 0;
+  unsigned long long* ticket = nullptr;  // the launch's number (high half), the next task
+  unsigned* flag = nullptr;              // the stop test's result (twice the launch + 0 or 1)
+  unsigned* hint = nullptr;              // per task: the launch in which it last finished
+  MgCycleLevel lv[kMgMaxLevels];
 };
 
 // Packed batch of scenes: scene s's own hierarchy below level `la` of the packed one.
@@ -266,6 +293,7 @@ struct SceneCoarse {
   int cx, cy;     // first cell of the scene's rectangle in the packed grid of level la
   int nl, total;  // its levels (the first is the rectangle); cells over all, a multiple of 4
   int nx[kSceneMaxLevels], ny[kSceneMaxLevels], off[kSceneMaxLevels];
+  int words;  // as MgCoarseArgs::words
 };
 struct SceneCoarseArgs {
   const SceneCoarse* tab = nullptr;
@@ -278,6 +306,7 @@ struct SceneCoarseArgs {
   float* x_out = nullptr;        // packed cycle result of level la
   float omega = 0.8f, omega2 = 0.8f;
   int trunc = 0;  // as MgCoarseArgs::trunc, on each scene's first level
+  size_t lds = 0; // bytes of LDS per scene's stage
 };
 
 // Packed batch: per-scene CG scalars (one CG per scene in lock step).
@@ -319,10 +348,9 @@ struct MgHost {
   // (the level's omega, omega2) or 3 .. kMgMaxSweeps (degree-S Chebyshev weights)
   int level_sweeps = 2;
   int level0_sweeps = 2;  // the same on level 0: 2 (omega, omega2) or 3 (degree-3 Chebyshev)
-  // the last tile level's down kernel also runs the one-workgroup stage (its last
-  // workgroup to finish), so no k_mg_coarse launch; ticket: its arrival counter
-  bool coarse_tail = true;
-  unsigned* ticket = nullptr;
+  // tile levels l1 .. lc-1 and the one-workgroup stage run in one launch (cyc)
+  int l1 = 0;
+  MgCycleArgs cyc;
   int nlev = 0, lc = 0;
   int nx[kMgMaxLevels] = {}, ny[kMgMaxLevels] = {};
   uint8_t* lab[kMgMaxLevels] = {};  // [0]: the domain's labels
@@ -338,6 +366,7 @@ struct MgHost {
   double* part_liq = nullptr;  // LIQUID cells per setup block (the solve without compaction)
   MgCoarseArgs coarse{};
   size_t coarse_lds = 0;
+  int stage_words = 0;  // MgCoarseArgs::words where the stage is not truncated
 };
 
 // Packed batch of scenes: each scene's right-hand side is scaled to unit norm before
@@ -352,7 +381,15 @@ struct MgBatchScale {
 };
 
 int mg_vec_blocks(int C);
-bool mg_tail_coarse(const MgHost& m);  // the one-workgroup stage runs in the down kernel
+// LDS words per buffer of the stage with its cells in registers; 0: the levels below the
+// first are too many cells for it, or the buffers too large
+int mg_stage_words(int nl, const int* nx, const int* ny, size_t lds_limit, bool scene);
+bool mg_has_cycle(const MgHost& m);  // tile levels l1 .. lc-1 and the stage: launch_mg_cycle
+int mg_cycle_level(const MgHost& m);  // l1 (lc or more: no tile level shares a launch)
+bool mg_cycle_prepare(MgHost& m, int n_stages, const std::function<void*(size_t)>& alloc);
+// scenes: a batch's (its own stage per scene), else null
+void launch_mg_cycle(hipStream_t s, const MgHost& m, int it, int max_iter, double tol,
+                     CgScalars* sc, const SceneCoarseArgs* scenes);
 int mg_part_rr_size(const MgHost& m);  // entries of MgHost::part_rr
 int mg_up_blocks(int nx, int ny);
 int mg_dir_blocks(const MgHost& m);  // blocks of k_mg_dir (partials of p.Kp)

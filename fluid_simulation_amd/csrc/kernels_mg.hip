@@ -32,10 +32,10 @@
 // level-(l+1) right-hand side is P^T of the level-l residual (the 4^-l scale of the
 // rediscretised operators cancels), so every level uses the unit stencil.
 //
-// Kernels per CG iteration: mg_down (one per fine level: 2 pre-smoothing sweeps,
-// residual and restriction fused in one LDS tile), mg_coarse (one workgroup: the
-// V-cycle of the levels of <= 1024 cells in LDS), mg_up (one per fine level:
-// prolongation, correction and 2 post-smoothing sweeps fused), mg_dir (p = z +
+// Kernels per CG iteration: mg_down (one per large tile level: the pre-smoothing sweeps,
+// residual and restriction fused in one tile), mg_cycle (the smaller tile levels both ways
+// and, in one workgroup, the V-cycle of the levels of <= 1024 cells), mg_up (one per large
+// tile level: prolongation, correction and post-smoothing sweeps fused), mg_dir (p = z +
 // beta p, K p and p.Kp), mg_xr (x += alpha p in FP64 and r = b' - K x).  Every
 // kernel returns at once when the solve is done, and each sums the block partials
 // of the previous kernel itself in a fixed order, so the scalars are identical in
@@ -44,6 +44,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
 
 #include <type_traits>
 
@@ -56,14 +57,12 @@ namespace fsg {
 namespace {
 
 constexpr int kT = 256;         // threads of the vector kernels and the level-0 tiles
-// Threads per tile of the levels below 0 (few_tiles): a level of at most one tile
-// per CU leaves CUs idle and its time is one tile's chain of LDS phases, which 1024
-// threads shorten; with more tiles two workgroups of 512 share a CU and one's waits are
-// hidden by the other.  V-cycle per step, 512 against 1024 threads on every level: 513 x
-// 385 cells 584 / 558 us, 1024^2 810 / 783 us; one 2048^2 level-1 launch (1024 tiles)
-// down 12.9 / 16.6 us, up 10.5 / 11.7 us.
-constexpr int kTileFew = 1024, kTileMany = 512;
-inline bool few_tiles(int tiles) { return tiles <= 256; }  // 256 CUs
+// The tile levels below 0 of more tiles than this have a launch each (in either direction),
+// the others share k_mg_cycle: a task costs a draw of 12 ns from one counter and its polls,
+// so a level of 256 tiles is as fast by itself (1024^2: 661 us per step with the line at 64
+// tiles, 672 at 256; 2048^2: 1013, 1027 and, at 1024, 1108 us).
+constexpr int kCycleTiles = 64;
+constexpr int kTileMany = 512;  // threads per tile of the former
 constexpr uint8_t kAct = kMgUnknown;  // info bit: the cell is an unknown
 constexpr int kTileEmptyBit = (int)0x80000000u;  // k_mg_tile_map: the tile holds no unknown
 constexpr uint8_t kWall = 0x40;   // info bit: SOLID (also used for cells outside the grid)
@@ -144,21 +143,28 @@ __device__ __forceinline__ void small_divmod(int q, int nx, float inv_nx, int& i
   i = q - j * nx;
 }
 
+// One thread's part of the sum of n block partials: b, b + NT, ...
+template <int NT>
+__device__ __forceinline__ double thread_part(const double* __restrict__ part, int n) {
+  double v = 0.0;
+  int b = threadIdx.x;
+  // four loads in flight per thread
+  for (; b + 3 * NT < n; b += 4 * NT) {
+    const double a0 = part[b], a1 = part[b + NT], a2 = part[b + 2 * NT], a3 = part[b + 3 * NT];
+    v += a0;
+    v += a1;
+    v += a2;
+    v += a3;
+  }
+  for (; b < n; b += NT) v += part[b];
+  return v;
+}
+
 // Sum of n block partials, the same fixed order in every block (NT threads;
 // sm: NT / 64 doubles).
 template <int NT = kT>
 __device__ __forceinline__ double sum_part(const double* __restrict__ part, int n, double* sm) {
-  double v[1] = {0.0};
-  int b = threadIdx.x;
-  // four loads in flight per thread; the additions keep the order b, b + NT, ...
-  for (; b + 3 * NT < n; b += 4 * NT) {
-    const double a0 = part[b], a1 = part[b + NT], a2 = part[b + 2 * NT], a3 = part[b + 3 * NT];
-    v[0] += a0;
-    v[0] += a1;
-    v[0] += a2;
-    v[0] += a3;
-  }
-  for (; b < n; b += NT) v[0] += part[b];
+  double v[1] = {thread_part<NT>(part, n)};
   block_sum<1, NT>(v, sm);
   return v[0];
 }
@@ -427,6 +433,7 @@ __global__ void __launch_bounds__(kT) k_mg_setup1(int nx, int ny, int project_me
   write_part<kT>(acc_r, part_rr, sm);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->done = 0;
+    sc->stuck = 0;
     sc->iter = 0;
     sc->spmv = 0;
     sc->err = 0.0;
@@ -657,6 +664,7 @@ __global__ void __launch_bounds__(kT) k_mg_setup0t(Geom g, const uint8_t* __rest
     if (threadIdx.x == 0) {
       CgScalars* sc = fold.sc;
       sc->done = 0;
+      sc->stuck = 0;
       sc->iter = 0;
       sc->spmv = 0;
       sc->err = 0.0;
@@ -834,26 +842,39 @@ struct MgCheck {
   int external;  // 1: the stop test ran in its own kernel (per-scene CG); read `done` only
 };
 
-// Every block takes the same decision from the same partials.  `done` is read by
-// one thread and broadcast, since block 0 may set it while other blocks start.
+// Every block takes the same decision from the same partials.  `done` is read by one thread
+// and broadcast, since the writer may set it while other blocks start; either value of it
+// leads to that decision, so it need not be read device-coherent.
 template <int NT>
-__device__ __forceinline__ bool mg_check(const MgCheck& k, int it, double* sm) {
+__device__ __forceinline__ bool mg_check(const MgCheck& k, int it, bool writer, double* sm) {
   __shared__ int s_done;
-  if (threadIdx.x == 0) s_done = ld_dev(&k.sc->done);
-  __syncthreads();
-  if (s_done || k.external) return s_done != 0;
-  const double rr = sum_part<NT>(k.part_rr, k.n_rr, sm);
-  double bb, thr;
+  // every load is issued before the first is needed (one memory round trip)
+  int done = 0;
+  if (threadIdx.x == 0)
+    done = __hip_atomic_load(&k.sc->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  double part[1] = {0.0}, bb = 0.0, thr = 0.0;
+  if (!k.external) {
+    bb = it == 0 ? thread_part<NT>(k.part_bb, k.n_bb) : k.sc->rhs_norm2;
+    thr = k.sc->threshold;
+    part[0] = thread_part<NT>(k.part_rr, k.n_rr);
+  }
+  if (threadIdx.x == 0) s_done = done;
+  if (k.external) {
+    __syncthreads();
+    return s_done != 0;
+  }
+  block_sum<1, NT>(part, sm);  // its barriers are behind s_done too
+  if (s_done) return true;
+  const double rr = part[0];
   if (it == 0) {
-    bb = sum_part<NT>(k.part_bb, k.n_bb, sm);
+    double w[1] = {bb};
+    block_sum<1, NT>(w, sm);
+    bb = w[0];
     thr = k.tol2 * bb;
     if (thr < DBL_MIN) thr = DBL_MIN;
-  } else {
-    bb = k.sc->rhs_norm2;
-    thr = k.sc->threshold;
   }
   const bool stop = bb == 0.0 || rr < thr || it >= k.max_iter;
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (writer && threadIdx.x == 0) {
     if (it == 0) {
       k.sc->rhs_norm2 = bb;
       k.sc->threshold = thr;
@@ -888,10 +909,6 @@ struct MgXr {
   int n_pq;
   double* part_rr;  // out: one partial |r|^2 per block
 };
-
-template <int CT>
-__device__ __forceinline__ void coarse_stage(const MgCoarseArgs& a, double* part_rz,
-                                             bool coherent);
 
 // Smoothing weights of the tile levels below level 0 when they take S > 2 sweeps
 // before and after the coarse correction (sweep k uses w[k - 1]); with S = 2 every
@@ -958,50 +975,223 @@ __device__ __forceinline__ void strip_nbrs(const T* __restrict__ x, int base, co
     sum[q] = l[q] + r[q] + (q == 0 ? dn : own[q - 1]) + (q == R - 1 ? up : own[q + 1]);
 }
 
+// A thread's strip of the tile at fine cell (fi0, fj0), whose first cell is cell (O, O) of
+// the W x W window.
+template <int NT, int W, int O>
+struct TileStrip : Strip<W, NT> {
+  using St = Strip<W, NT>;
+  using St::R;
+  int wx, wy0, base, gi, gj;
+  bool strip;
+  int cell[R];         // grid index, 0 outside the grid
+  bool in[R], own[R];  // the cell lies in the grid; and in the tile
+  __device__ __forceinline__ TileStrip(int fi0, int fj0, int nx, int ny) {
+    // the strip: column wx, rows wy0 .. wy0 + R - 1 of the window
+    const int g = threadIdx.x / W;
+    wx = threadIdx.x % W;
+    wy0 = g * R;
+    strip = g < St::G;
+    base = strip ? (wy0 + 1) * St::PW + wx + 1 : St::PW + 1;
+    gi = fi0 - O + wx;
+    gj = fj0 - O + wy0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      in[q] = strip && wy0 + q < W && gi >= 0 && gi < nx && gj + q >= 0 && gj + q < ny;
+      own[q] = in[q] && wx >= O && wx < O + 32 && wy0 + q >= O && wy0 + q < O + 32;
+      cell[q] = in[q] ? gi + (gj + q) * nx : 0;
+    }
+  }
+};
+
+// The tile kernels' sweep weights: sw's for S > 2 sweeps, else the level's omega, omega2.
+template <int S>
+__device__ __forceinline__ void sweep_weights(const MgSweeps& sw, float omega, float omega2,
+                                              float (&wk)[kMgMaxSweeps]) {
+#pragma unroll
+  for (int k = 0; k < kMgMaxSweeps; ++k) wk[k] = sw.w[k];
+  if (S == 2) {
+    wk[0] = omega;
+    wk[1] = omega2;
+  }
+}
+
+// Down on one tile, from the strips' info fv and right-hand side rv and the coarse info
+// around the tile in s_cinf (18 x 18): S sweeps from zero, the residual, its restriction.
+// put_xs(q, x): the smoothed x of strip cell q (a cell of the tile); put_r(index, v): a
+// coarse right-hand side.  stopped() is asked (by all threads) before the first of them: if
+// true, nothing is put.
+// The last barrier before the restriction is in here; one is needed before the LDS
+// buffers s_x0, s_x1 (Strip::N floats each) are written again.
+constexpr int kDownWC = 18;  // coarse cells of a tile and their neighbours
+template <int NT, int S, class PutXs, class PutR, class Stopped>
+__device__ __forceinline__ void down_core(const TileStrip<NT, 34 + 2 * S, S + 1>& ts,
+                                          const uint8_t (&fv)[Strip<34 + 2 * S, NT>::R],
+                                          const float (&rv)[Strip<34 + 2 * S, NT>::R],
+                                          const float (&wk)[kMgMaxSweeps], float* s_x0,
+                                          float* s_x1, const uint8_t* s_cinf, int bx, int by,
+                                          int cnx, int cny, PutXs&& put_xs, PutR&& put_r,
+                                          Stopped&& stopped) {
+  constexpr int W = 34 + 2 * S, O = S + 1, WC = kDownWC;
+  using St = Strip<W, NT>;
+  constexpr int R = St::R, PW = St::PW;
+  const int base = ts.base;
+  // the first sweep from x = 0
+  float nn[R], inv[R], x[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    nn[q] = nns_of(fv[q]);
+    inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
+    x[q] = wk[0] * rv[q] * inv[q];
+  }
+  // sweeps alternate between the two buffers; the residual takes the one that is free
+  float *cur = s_x0, *other = s_x1;
+  auto put = [&](float* dst, const float (&v)[R]) {
+    if (ts.strip)
+#pragma unroll
+      for (int q = 0; q < R; ++q) dst[base + q * PW] = v[q];
+  };
+  put(cur, x);
+  __syncthreads();
+  float sum[R];
+#pragma unroll
+  for (int k = 2; k <= S; ++k) {
+    strip_nbrs<R, PW>(cur, base, x, sum);
+    const float wgt = wk[k - 1];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
+    float* const t = cur;
+    cur = other;
+    other = t;
+    put(cur, x);
+    __syncthreads();
+  }
+  if (stopped()) return;
+  strip_nbrs<R, PW>(cur, base, x, sum);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const float res = is_act(fv[q]) ? rv[q] - (nn[q] * x[q] - sum[q]) : 0.f;
+    if (ts.own[q]) put_xs(q, x[q]);
+    sum[q] = res;
+  }
+  put(other, sum);
+  __syncthreads();
+  const float* const s_res = other + (O + 1) * PW + O + 1;  // the tile's first cell
+  if (threadIdx.x < 256) {
+    const int ci = threadIdx.x & 15, cj = threadIdx.x >> 4;
+    const int I = bx * 16 + ci, J = by * 16 + cj;
+    if (I < cnx && J < cny) {
+      float v = 0.f;
+      if (is_act(s_cinf[(ci + 1) + (cj + 1) * WC])) {
+        // fine offsets 2ci-1 .. 2ci+2 and 2cj-1 .. 2cj+2
+        const float w[4] = {0.25f, 0.75f, 0.75f, 0.25f};
+        float t[4][4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) t[b][e] = s_res[(2 * cj - 1 + b) * PW + 2 * ci - 1 + e];
+        // the four children moved the weight of their wall neighbours here
+        auto ci_at = [&](int di, int dj) { return s_cinf[(ci + 1 + di) + (cj + 1 + dj) * WC]; };
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          v += w[b] * (0.25f * t[b][0] + 0.75f * t[b][1] + 0.75f * t[b][2] + 0.25f * t[b][3]);
+#pragma unroll
+        for (int b = 1; b <= 2; ++b)
+#pragma unroll
+          for (int e = 1; e <= 2; ++e) {
+            const int dx = e == 1 ? -1 : 1, dy = b == 1 ? -1 : 1;
+            v += moved_weight(ci_at(dx, 0), ci_at(0, dy), ci_at(dx, dy)) * t[b][e];
+          }
+      }
+      put_r(I + J * cnx, v);
+    }
+  }
+}
+
+// Up on one tile: x (on entry after the pre-sweeps) += P e from the coarse solution and
+// info around the tile in s_e, s_cinf (WC x WC from CO cells before the tile's first
+// coarse cell), then S post-sweeps; x is the level's result on the tile's cells.  The
+// coarse frame is in LDS, a barrier after its stores behind it.
+template <int S>
+struct UpFrame {
+  // coarse cells from fi0 / 2 - (S / 2 + 1): every coarse neighbour of the window's cells
+  static constexpr int WC = 18 + S, CO = S / 2 + 1;
+};
+template <int NT, int S>
+__device__ __forceinline__ void up_core(const TileStrip<NT, 32 + 2 * S, S>& ts,
+                                        const uint8_t (&fv)[Strip<32 + 2 * S, NT>::R],
+                                        const float (&rv)[Strip<32 + 2 * S, NT>::R],
+                                        float (&x)[Strip<32 + 2 * S, NT>::R],
+                                        const float (&wk)[kMgMaxSweeps], float* s_x0, float* s_x1,
+                                        const float* s_e, const uint8_t* s_cinf) {
+  constexpr int W = 32 + 2 * S, WC = UpFrame<S>::WC, CO = UpFrame<S>::CO;
+  using St = Strip<W, NT>;
+  constexpr int R = St::R, PW = St::PW;
+  static_assert(St::HP / 2 + (S & 1 ? 0 : 1) < WC, "the strips' coarse rows lie in the frame");
+  const int base = ts.base;
+  // the correction: two coarse columns (the cells' own and its x neighbour) times the
+  // strip's coarse rows, wy0 / 2 + (S even) and on; window rows of even number lie in odd
+  // fine rows where S is odd
+  float nn[R], inv[R];
+  {
+    constexpr bool kOdd = (S & 1) != 0;
+    constexpr int NR = R / 2 + (kOdd ? 1 : 2);
+    const int il = ((ts.wx - S) >> 1) + CO, inl = il + (((ts.wx - S) & 1) ? 1 : -1);
+    const int q0 = ts.strip ? (ts.wy0 / 2) * WC + il : WC;
+    const int q1 = ts.strip ? (ts.wy0 / 2) * WC + inl : WC;
+    float e0[NR], e1[NR];
+    uint8_t f0[NR], f1[NR];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      e0[k] = s_e[q0 + k * WC];
+      e1[k] = s_e[q1 + k * WC];
+      f0[k] = s_cinf[q0 + k * WC];
+      f1[k] = s_cinf[q1 + k * WC];
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const bool odd = ((q & 1) != 0) != kOdd;  // the fine row is odd
+      const int J = kOdd ? (q + 1) / 2 : 1 + q / 2, Jn = odd ? J + 1 : J - 1;
+      const float pe = prolong_value(e0[J], e1[J], f1[J], e0[Jn], f0[Jn], e1[Jn], f1[Jn]);
+      x[q] = is_act(fv[q]) ? x[q] + pe : 0.f;
+      nn[q] = nns_of(fv[q]);
+      inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
+    }
+  }
+  // every sweep reads its neighbours from LDS
+  float sum[R];
+  float *cur = s_x0, *other = s_x1;
+#pragma unroll
+  for (int k = 1; k <= S; ++k) {
+    if (ts.strip)
+#pragma unroll
+      for (int q = 0; q < R; ++q) cur[base + q * PW] = x[q];
+    __syncthreads();
+    strip_nbrs<R, PW>(cur, base, x, sum);
+    const float wgt = wk[k - 1];
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
+    float* const t = cur;
+    cur = other;
+    other = t;
+  }
+}
+
 // S sweeps (2 or 3 on level 0, 2 .. kMgMaxSweeps on the levels below): the right-hand
 // side and info on the window [-(S + 1), 33 + S) around the tile; after the S sweeps x is
 // known on [-2, 34), the residual on [-1, 33).
-template <bool L0, int NT, bool XR = false, bool TAIL = false, int S = 2>
+template <bool L0, int NT, bool XR = false, int S = 2>
 __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omega, float omega2,
-                                                 int it,
-                                                 MgCheck chk, int check,
+                                                 int it, MgCheck chk, int check,
                                                  const uint8_t* __restrict__ tflag, MgXr xr,
-                                                 unsigned long long* span,
-                                                 MgCoarseArgs ca, unsigned* __restrict__ ticket,
-                                                 MgSweeps sw, const int* __restrict__ tmap) {
+                                                 unsigned long long* span, MgSweeps sw,
+                                                 const int* __restrict__ tmap) {
   static_assert(!XR || L0, "the fused update belongs to level 0");
-  static_assert(!TAIL || !L0, "the one-workgroup stage follows the last tile level");
   static_assert(S >= 2 && S <= kMgMaxSweeps && (!L0 || S <= 3),
                 "level 0 takes two or three sweeps; smaller levels 2 .. kMgMaxSweeps");
   const BlockSpan clock(span);
   __shared__ double sm[NT / 64];
-  __shared__ int s_last;
-  // TAIL (the last tile level): the restriction is stored device-coherent and the last
-  // workgroup to finish runs the one-workgroup stage on it, in place of a k_mg_coarse
-  // launch.  The arrival count is ordered after every wave's stores, as in a grid
-  // barrier, but nobody waits.
-  // inlined: as a call its LDS accesses would go through flat addresses
-  auto run_tail = [&]() __attribute__((always_inline)) {
-    if constexpr (TAIL) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-      __builtin_amdgcn_s_waitcnt(0);
-      __syncthreads();
-      if (threadIdx.x == 0)
-        s_last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
-      __syncthreads();
-      if (s_last) {
-        if (threadIdx.x == 0) st_dev(ticket, 0u);  // ready for the next launch
-        coarse_stage<NT>(ca, nullptr, true);
-      }
-    }
-  };
-  auto put_r = [&](float* dst, float v) {
-    if constexpr (TAIL)
-      st_dev(dst, v);
-    else
-      *dst = v;
-  };
   // the tile (and its flag) are read with the stop flag (one memory round trip)
   const int tm = tmap ? tmap[blockIdx.x] : 0;
   const int tile = tmap ? tm & ~kTileEmptyBit : xcd_tile(blockIdx.x, gridDim.x);
@@ -1009,25 +1199,13 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   constexpr int W = 34 + 2 * S, O = S + 1;  // the window and the tile's offset in it
   using St = Strip<W, NT>;
   constexpr int R = St::R, PW = St::PW;
-  constexpr int WC = 18;  // coarse cells of the tile and their neighbours
+  constexpr int WC = kDownWC;
   const int tiles_x = (c.nx + 15) >> 4;
   // each XCD takes one band of consecutive tiles, so halo rows are shared in its L2
   const int bx = tile % tiles_x, by = tile / tiles_x;
   const int fi0 = bx * 32, fj0 = by * 32;
   const bool do_xr = XR && it > 0;
-  // the strip: column wx, rows wy0 .. wy0 + R - 1 of the window
-  const int wx = threadIdx.x % W, g = threadIdx.x / W, wy0 = g * R;
-  const bool strip = g < St::G;
-  const int base = strip ? (wy0 + 1) * PW + wx + 1 : PW + 1;
-  const int gi = fi0 - O + wx, gj = fj0 - O + wy0;
-  int cell[R];
-  bool in[R], own[R];  // the cell lies in the grid; and in the tile
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-    in[q] = strip && wy0 + q < W && gi >= 0 && gi < f.nx && gj + q >= 0 && gj + q < f.ny;
-    own[q] = in[q] && wx >= O && wx < O + 32 && wy0 + q >= O && wy0 + q < O + 32;
-    cell[q] = in[q] ? gi + (gj + q) * f.nx : 0;
-  }
+  const TileStrip<NT, W, O> ts(fi0, fj0, f.nx, f.ny);
   // Without the fused update, every load of a tile holding unknowns is issued before
   // the stop test's reads (their round trips overlap; a finished solve drops them) and
   // before the first LDS store (a load outside the grid reads cell 0 and is replaced
@@ -1049,14 +1227,14 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     load_coarse();
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const uint8_t fq = f.inf[cell[q]];
-      const float rq = f.r[cell[q]];
-      fv[q] = in[q] ? fq : 0;
-      rv[q] = in[q] ? rq : 0.f;
+      const uint8_t fq = f.inf[ts.cell[q]];
+      const float rq = f.r[ts.cell[q]];
+      fv[q] = ts.in[q] ? fq : 0;
+      rv[q] = ts.in[q] ? rq : 0.f;
     }
   }
   if (check) {
-    if (mg_check<NT>(chk, it, sm)) {
+    if (mg_check<NT>(chk, it, blockIdx.x == 0, sm)) {
       clock.end();
       return;
     }
@@ -1064,17 +1242,11 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     clock.end();
     return;
   }
-  // sweeps alternate between the two buffers; the residual takes the one that is free
   __shared__ float s_x[2][St::N];
   __shared__ uint8_t s_cinf[WC * WC];
   __shared__ double s_xn[XR ? St::N : 1];
   float wk[kMgMaxSweeps];
-#pragma unroll
-  for (int k = 0; k < kMgMaxSweeps; ++k) wk[k] = sw.w[k];
-  if (S == 2) {
-    wk[0] = omega;
-    wk[1] = omega2;
-  }
+  sweep_weights<S>(sw, omega, omega2, wk);
   if (empty) {
     // no unknown in the tile on either level: its outputs are zero; written once per
     // solve (earlier solves may have left other values)
@@ -1085,7 +1257,7 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
       }
       for (int t = threadIdx.x; t < 16 * 16; t += NT) {
         const int I = bx * 16 + (t & 15), J = by * 16 + (t >> 4);
-        if (I < c.nx && J < c.ny) put_r(c.r + I + J * c.nx, 0.f);
+        if (I < c.nx && J < c.ny) c.r[I + J * c.nx] = 0.f;
       }
     }
     if (do_xr) {
@@ -1101,7 +1273,6 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
         }
       if (threadIdx.x == 0) xr.part_rr[blockIdx.x] = 0.0;
     }
-    run_tail();
     clock.end();
     return;
   }
@@ -1117,14 +1288,14 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     for (int q = 0; q < R; ++q) {
       // a strip past the window's rows holds the ring's first row too: the neighbour
       // above the window's last one
-      const bool inx = in[q] || (strip && wy0 + q == W && gi >= 0 && gi < f.nx &&
-                                 gj + q >= 0 && gj + q < f.ny);
-      const int cx = inx ? gi + (gj + q) * f.nx : 0;
-      const uint8_t fq = f.inf[cell[q]];
-      const double bq = xr.b[cell[q]], xq = xr.x_old[cx];
+      const bool inx = ts.in[q] || (ts.strip && ts.wy0 + q == W && ts.gi >= 0 && ts.gi < f.nx &&
+                                 ts.gj + q >= 0 && ts.gj + q < f.ny);
+      const int cx = inx ? ts.gi + (ts.gj + q) * f.nx : 0;
+      const uint8_t fq = f.inf[ts.cell[q]];
+      const double bq = xr.b[ts.cell[q]], xq = xr.x_old[cx];
       const float pq = xr.p[cx];
-      fv[q] = in[q] ? fq : 0;
-      bv[q] = in[q] ? bq : 0.0;
+      fv[q] = ts.in[q] ? fq : 0;
+      bv[q] = ts.in[q] ? bq : 0.0;
       xo[q] = inx ? xq : 0.0;
       pv[q] = inx ? pq : 0.f;
     }
@@ -1148,27 +1319,27 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     double xn[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) xn[q] = xo[q] + alpha * (double)pv[q];
-    if (strip)
+    if (ts.strip)
 #pragma unroll
       for (int q = 0; q < R; ++q)
-        if (wy0 + q < W) s_xn[base + q * PW] = xn[q];
+        if (ts.wy0 + q < W) s_xn[ts.base + q * PW] = xn[q];
     if (ring) s_xn[rx + ry * PW] = rin ? rxo + alpha * (double)rp : 0.0;
     __syncthreads();
     // r = b' - K x_new on the window (cells outside the grid hold x = 0 and add 0); the
     // tile's own cells store x_new and r and add to |r|^2
     double sn[R], acc = 0.0;
-    strip_nbrs<R, PW>(s_xn, base, xn, sn);
+    strip_nbrs<R, PW>(s_xn, ts.base, xn, sn);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       double r64 = 0.0;
       if (is_act(fv[q])) {
         r64 = bv[q] - ((double)(fv[q] & 7) * xn[q] - sn[q]);
-        acc += own[q] ? r64 * r64 : 0.0;
+        acc += ts.own[q] ? r64 * r64 : 0.0;
       }
       rv[q] = (float)r64;
-      if (own[q]) {
-        xr.x_new[cell[q]] = is_act(fv[q]) ? xn[q] : 0.0;
-        f.r[cell[q]] = rv[q];
+      if (ts.own[q]) {
+        xr.x_new[ts.cell[q]] = is_act(fv[q]) ? xn[q] : 0.0;
+        f.r[ts.cell[q]] = rv[q];
       }
     }
     write_part<NT>(acc, xr.part_rr, sm);
@@ -1181,75 +1352,9 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
       if (t < WC * WC) s_cinf[t] = cv[k];
     }
   }
-  // the first sweep from x = 0
-  float nn[R], inv[R], x[R];
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-    nn[q] = nns_of(fv[q]);
-    inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
-    x[q] = wk[0] * rv[q] * inv[q];
-  }
-  int cur = 0;
-  auto put = [&](float* dst, const float (&v)[R]) {
-    if (strip)
-#pragma unroll
-      for (int q = 0; q < R; ++q) dst[base + q * PW] = v[q];
-  };
-  put(s_x[cur], x);
-  __syncthreads();
-  float sum[R];
-#pragma unroll
-  for (int k = 2; k <= S; ++k) {
-    strip_nbrs<R, PW>(s_x[cur], base, x, sum);
-    const float wgt = wk[k - 1];
-#pragma unroll
-    for (int q = 0; q < R; ++q)
-      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
-    cur ^= 1;
-    put(s_x[cur], x);
-    __syncthreads();
-  }
-  strip_nbrs<R, PW>(s_x[cur], base, x, sum);
-  cur ^= 1;
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-    const float res = is_act(fv[q]) ? rv[q] - (nn[q] * x[q] - sum[q]) : 0.f;
-    if (own[q]) f.xs[cell[q]] = x[q];
-    sum[q] = res;
-  }
-  put(s_x[cur], sum);
-  __syncthreads();
-  const float* const s_res = s_x[cur] + (O + 1) * PW + O + 1;  // the tile's first cell
-  if (threadIdx.x < 256) {
-    const int ci = threadIdx.x & 15, cj = threadIdx.x >> 4;
-    const int I = bx * 16 + ci, J = by * 16 + cj;
-    if (I < c.nx && J < c.ny) {
-      float v = 0.f;
-      if (is_act(s_cinf[(ci + 1) + (cj + 1) * WC])) {
-        // fine offsets 2ci-1 .. 2ci+2 and 2cj-1 .. 2cj+2
-        const float w[4] = {0.25f, 0.75f, 0.75f, 0.25f};
-        float t[4][4];
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) t[b][e] = s_res[(2 * cj - 1 + b) * PW + 2 * ci - 1 + e];
-        // the four children moved the weight of their wall neighbours here
-        auto ci_at = [&](int di, int dj) { return s_cinf[(ci + 1 + di) + (cj + 1 + dj) * WC]; };
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-          v += w[b] * (0.25f * t[b][0] + 0.75f * t[b][1] + 0.75f * t[b][2] + 0.25f * t[b][3]);
-#pragma unroll
-        for (int b = 1; b <= 2; ++b)
-#pragma unroll
-          for (int e = 1; e <= 2; ++e) {
-            const int dx = e == 1 ? -1 : 1, dy = b == 1 ? -1 : 1;
-            v += moved_weight(ci_at(dx, 0), ci_at(0, dy), ci_at(dx, dy)) * t[b][e];
-          }
-      }
-      put_r(c.r + I + J * c.nx, v);
-    }
-  }
-  run_tail();
+  down_core<NT, S>(ts, fv, rv, wk, s_x[0], s_x[1], s_cinf, bx, by, c.nx, c.ny,
+                   [&](int q, float x) { f.xs[ts.cell[q]] = x; },
+                   [&](int q, float v) { c.r[q] = v; }, [] { return false; });
   if (span) {
     __syncthreads();
     clock.end();
@@ -1270,20 +1375,13 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
                 "level 0 takes two or three sweeps; smaller levels 2 .. kMgMaxSweeps");
   constexpr int W = 32 + 2 * S;
   using St = Strip<W, NT>;
-  constexpr int R = St::R, PW = St::PW;
-  // coarse cells from fi0 / 2 - (S / 2 + 1): every coarse neighbour of the window's cells
-  constexpr int WC = 18 + S, CO = S / 2 + 1;
-  static_assert(St::HP / 2 + (S & 1 ? 0 : 1) < WC, "the strips' coarse rows lie in the frame");
+  constexpr int R = St::R;
+  constexpr int WC = UpFrame<S>::WC, CO = UpFrame<S>::CO;
   __shared__ float s_x[2][St::N], s_e[WC * WC];
   __shared__ uint8_t s_cinf[WC * WC];
   __shared__ double sm[NT / 64];
   float wk[kMgMaxSweeps];
-#pragma unroll
-  for (int k = 0; k < kMgMaxSweeps; ++k) wk[k] = sw.w[k];
-  if (S == 2) {
-    wk[0] = omega;
-    wk[1] = omega2;
-  }
+  sweep_weights<S>(sw, omega, omega2, wk);
   const int tiles_x = (f.nx + 31) >> 5;
   // each XCD takes one band of consecutive tiles, so halo rows are shared in its L2
   // (or the live tiles' share of them, tmap); the tile, its flag and the stop flag are
@@ -1294,18 +1392,7 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
   const int bx = tile % tiles_x, by = tile / tiles_x;
   const int fi0 = bx * 32, fj0 = by * 32;
   const int ci0 = (fi0 >> 1) - CO, cj0 = (fj0 >> 1) - CO;  // coarse frame origin
-  const int wx = threadIdx.x % W, g = threadIdx.x / W, wy0 = g * R;
-  const bool strip = g < St::G;
-  const int base = strip ? (wy0 + 1) * PW + wx + 1 : PW + 1;
-  const int gi = fi0 - S + wx, gj = fj0 - S + wy0;
-  int cell[R];
-  bool in[R], own[R];  // the cell lies in the grid; and in the tile
-#pragma unroll
-  for (int q = 0; q < R; ++q) {
-    in[q] = strip && wy0 + q < W && gi >= 0 && gi < f.nx && gj + q >= 0 && gj + q < f.ny;
-    own[q] = in[q] && wx >= S && wx < S + 32 && wy0 + q >= S && wy0 + q < S + 32;
-    cell[q] = in[q] ? gi + (gj + q) * f.nx : 0;
-  }
+  const TileStrip<NT, W, S> ts(fi0, fj0, f.nx, f.ny);
   // every load of a tile holding unknowns is issued before the stop flag's value is
   // known (one memory round trip for both; the loads of a finished solve are dropped)
   // and before the first LDS store (a load outside the grid reads cell 0 and is
@@ -1327,11 +1414,11 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
     }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const uint8_t fq = f.inf[cell[q]];
-      const float rq = f.r[cell[q]], xq = f.xs[cell[q]];
-      fv[q] = in[q] ? fq : 0;
-      rv[q] = in[q] ? rq : 0.f;
-      x[q] = in[q] ? xq : 0.f;
+      const uint8_t fq = f.inf[ts.cell[q]];
+      const float rq = f.r[ts.cell[q]], xq = f.xs[ts.cell[q]];
+      fv[q] = ts.in[q] ? fq : 0;
+      rv[q] = ts.in[q] ? rq : 0.f;
+      x[q] = ts.in[q] ? xq : 0.f;
     }
   }
   if (sc->done) return;
@@ -1354,56 +1441,13 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
     }
   }
   __syncthreads();
-  // the correction: two coarse columns (the cells' own and its x neighbour) times the
-  // strip's coarse rows, wy0 / 2 + (S even) and on; window rows of even number lie in odd
-  // fine rows where S is odd
-  float nn[R], inv[R];
-  {
-    constexpr bool kOdd = (S & 1) != 0;
-    constexpr int NR = R / 2 + (kOdd ? 1 : 2);
-    const int il = ((wx - S) >> 1) + CO, inl = il + (((wx - S) & 1) ? 1 : -1);
-    const int q0 = strip ? (wy0 / 2) * WC + il : WC, q1 = strip ? (wy0 / 2) * WC + inl : WC;
-    float e0[NR], e1[NR];
-    uint8_t f0[NR], f1[NR];
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      e0[k] = s_e[q0 + k * WC];
-      e1[k] = s_e[q1 + k * WC];
-      f0[k] = s_cinf[q0 + k * WC];
-      f1[k] = s_cinf[q1 + k * WC];
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const bool odd = ((q & 1) != 0) != kOdd;  // the fine row is odd
-      const int J = kOdd ? (q + 1) / 2 : 1 + q / 2, Jn = odd ? J + 1 : J - 1;
-      const float pe = prolong_value(e0[J], e1[J], f1[J], e0[Jn], f0[Jn], e1[Jn], f1[Jn]);
-      x[q] = is_act(fv[q]) ? x[q] + pe : 0.f;
-      nn[q] = nns_of(fv[q]);
-      inv[q] = is_act(fv[q]) ? inv_nns(fv[q]) : 0.f;
-    }
-  }
-  // post-sweeps 1 .. S-1 through LDS, the last straight to the outputs
-  float sum[R];
-  int cur = 0;
-#pragma unroll
-  for (int k = 1; k <= S; ++k) {
-    if (strip)
-#pragma unroll
-      for (int q = 0; q < R; ++q) s_x[cur][base + q * PW] = x[q];
-    __syncthreads();
-    strip_nbrs<R, PW>(s_x[cur], base, x, sum);
-    const float wgt = wk[k - 1];
-#pragma unroll
-    for (int q = 0; q < R; ++q)
-      x[q] = is_act(fv[q]) ? x[q] + wgt * (rv[q] - (nn[q] * x[q] - sum[q])) * inv[q] : 0.f;
-    cur ^= 1;
-  }
+  up_core<NT, S>(ts, fv, rv, x, wk, s_x[0], s_x[1], s_e, s_cinf);
   double rz = 0.0;
 #pragma unroll
   for (int q = 0; q < R; ++q)
-    if (own[q]) {
+    if (ts.own[q]) {
       const float v = is_act(fv[q]) ? x[q] : 0.f;
-      f.xo[cell[q]] = v;
+      f.xo[ts.cell[q]] = v;
       if (L0) rz += (double)rv[q] * (double)v;
     }
   if (L0) write_part<NT>(rz, part_rz, sm);
@@ -1429,6 +1473,8 @@ __device__ __forceinline__ float nbr_sum(const float* a, int c, int i, int j, in
 }
 
 constexpr int kCoarseThreads = 1024;
+// stage_cycle's cells per thread below the first level: one domain's stage, a scene's
+constexpr int kStageKB = 1, kSceneKB = 2;
 constexpr float kCoarsestOmega = 0.8f;  // damped Jacobi on the coarsest level (<= 64 cells)
 
 // The one-workgroup V-cycle over the levels 0 .. nl-1 of a small hierarchy held in
@@ -1656,6 +1702,254 @@ __device__ __forceinline__ void coarse_cycle(int nl, const int* __restrict__ lnx
   }
 }
 
+// The one-workgroup V-cycle with its cells in registers: a thread keeps its cells' right-hand
+// side, solution and stencil, weights of the corrections and LDS positions included, for
+// K cells of the first level and KB of the levels below it, whose cells lie one level after
+// another over the workgroup's wavefronts (a level begins at a wavefront).  All of that is
+// formed before the right-hand side is asked for.  LDS holds two buffers of x with a border
+// of zeros around every level (pitch nx + 2, ny + 3 rows: the restriction of an odd level
+// reads two past its end), so no read needs a bounds check; a phase is four to sixteen LDS
+// reads, the arithmetic and a barrier, six phases per level.  In LDS alone, indices and
+// neighbour tests formed anew in every phase, 32 x 32 cells took 8.8 us, this form 5.2 us:
+// what is left is the chain of LDS round trips and barriers (19 of them).
+//
+// lx(l), ly(l), lo(l): a level's size and its offset in inf.  rhs(r): the first level's
+// right-hand side of the cells threadIdx.x + k NT (act[k]: an unknown).  out(k, x): the
+// result there.  lds: 2 * words floats.
+struct StageCell {
+  int pos = 0;                 // in LDS
+  bool in = false, act = false;
+  float nn = 0.f, inv = 0.f, r = 0.f, x = 0.f;
+  // the correction: the coarse cell in LDS; bits 0, 1: the neighbours are those at + x, + y;
+  // 2, 3, 4: the x, y, diagonal neighbour is a wall
+  int epos = 0, ebits = 0;
+};
+
+// 2 max(nx, ny) + 8 damped-Jacobi sweeps from zero on the coarsest level, a cell per lane
+// (lane = i + j nx).
+template <int NX>
+__device__ __forceinline__ float coarsest_dpp(float r, float nn, float rn, bool act, int ny,
+                                              int sweeps) {
+  // at most 16 cells: one row of 16 lanes, neighbours by lane shifts within it
+  const int lane = threadIdx.x & 63, i = lane % NX, j = lane / NX;
+  const bool ml = i > 0, mr = i < NX - 1, md = j > 0, mu = j < ny - 1;
+  auto shift = [](float v, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v),
+                                                      decltype(ctrl)::value, 0xF, 0xF, true));
+  };
+  float x = 0.f;
+  for (int sw = 0; sw < sweeps; ++sw) {
+    const float xl = shift(x, std::integral_constant<int, 0x111>{});       // row_shr:1
+    const float xr = shift(x, std::integral_constant<int, 0x101>{});       // row_shl:1
+    const float xd = shift(x, std::integral_constant<int, 0x110 + NX>{});  // row_shr:NX
+    const float xu = shift(x, std::integral_constant<int, 0x100 + NX>{});  // row_shl:NX
+    float s = ml ? xl : 0.f;
+    s += mr ? xr : 0.f;
+    s += md ? xd : 0.f;
+    s += mu ? xu : 0.f;
+    x = act ? x + kCoarsestOmega * (r - (nn * x - s)) * rn : 0.f;
+  }
+  return x;
+}
+__device__ __forceinline__ float coarsest_sweeps(float r, float nn, float rn, bool act, int nx,
+                                                 int ny, int sweeps) {
+  if (nx <= 4 && ny <= 4) {
+    switch (nx) {
+      case 1: return coarsest_dpp<1>(r, nn, rn, act, ny, sweeps);
+      case 2: return coarsest_dpp<2>(r, nn, rn, act, ny, sweeps);
+      case 3: return coarsest_dpp<3>(r, nn, rn, act, ny, sweeps);
+      default: return coarsest_dpp<4>(r, nn, rn, act, ny, sweeps);
+    }
+  }
+  const int q = threadIdx.x & 63, i = q % nx, j = q / nx;
+  float x = 0.f;
+  for (int sw = 0; sw < sweeps; ++sw) {
+    const float xl = __shfl(x, q - 1 < 0 ? 0 : q - 1, 64);
+    const float xr = __shfl(x, q + 1 > 63 ? 63 : q + 1, 64);
+    const float xd = __shfl(x, q - nx < 0 ? 0 : q - nx, 64);
+    const float xu = __shfl(x, q + nx > 63 ? 63 : q + nx, 64);
+    float s = i > 0 ? xl : 0.f;
+    s += i < nx - 1 ? xr : 0.f;
+    s += j > 0 ? xd : 0.f;
+    s += j < ny - 1 ? xu : 0.f;
+    x = act ? x + kCoarsestOmega * (r - (nn * x - s)) * rn : 0.f;
+  }
+  return x;
+}
+
+template <int NT, int K, int KB, class Lx, class Ly, class Lo, class Rhs, class Out>
+__device__ __forceinline__ void stage_cycle(int nl, Lx&& lx, Ly&& ly, Lo&& lo,
+                                            const uint8_t* inf, float w, float w2, int sweeps,
+                                            float* lds, int words, Rhs&& rhs, Out&& out) {
+  float *P0 = lds, *P1 = lds + words;
+  for (int q = threadIdx.x; q < 2 * words; q += NT) lds[q] = 0.f;
+  StageCell A[K], B[KB];
+  float bm[KB][4];  // extra weights of the four children in the restriction
+  int rpos[KB], bl[KB];
+  auto set = [&](StageCell& c, int l, int q, int po, int& i, int& j) {
+    const int nx = lx(l), ny = ly(l);
+    c.in = q < nx * ny;
+    small_divmod(c.in ? q : 0, nx, 1.0f / (float)nx, i, j);
+    const uint8_t f = inf[lo(l) + (c.in ? q : 0)];
+    c.act = c.in && is_act(f);
+    c.nn = nns_of(f);
+    c.inv = c.act ? inv_nns(f) : 0.f;
+    c.pos = po + (j + 1) * (nx + 2) + i + 1;
+    if (l + 1 < nl) {
+      const int cnx = lx(l + 1), cny = ly(l + 1), co = lo(l + 1);
+      const int I = i >> 1, J = j >> 1;
+      const int In = (i & 1) ? I + 1 : I - 1, Jn = (j & 1) ? J + 1 : J - 1;
+      const bool iok = In >= 0 && In < cnx, jok = Jn >= 0 && Jn < cny;
+      const int Ic = iok ? In : I, Jc = jok ? Jn : J;
+      const uint8_t fx = inf[co + Ic + J * cnx], fy = inf[co + I + Jc * cnx];
+      const uint8_t fxy = inf[co + Ic + Jc * cnx];
+      const bool bx = !iok || is_wall(fx), by = !jok || is_wall(fy);
+      const bool bxy = !(iok && jok) || is_wall(fxy);
+      c.epos = po + (nx + 2) * (ny + 3) + (J + 1) * (cnx + 2) + I + 1;
+      c.ebits = (i & 1) | ((j & 1) << 1) | (bx << 2) | (by << 3) | (bxy << 4);
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    int i, j;
+    set(A[k], 0, threadIdx.x + k * NT, 0, i, j);
+  }
+#pragma unroll
+  for (int b = 0; b < KB; ++b) {
+    // the level of this wavefront's cells
+    const int slot = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u) + b * NT);
+    int l = 1, s0 = 0, po = nl > 0 ? (lx(0) + 2) * (ly(0) + 3) : 0, fpo = 0;
+    for (; l < nl; ++l) {
+      const int n64 = (lx(l) * ly(l) + 63) & ~63;
+      if (slot < s0 + n64) break;
+      s0 += n64;
+      fpo = po;
+      po += (lx(l) + 2) * (ly(l) + 3);
+    }
+    bl[b] = l < nl ? l : -1;
+    rpos[b] = 0;
+    if (l < nl) {
+      int i, j;
+      set(B[b], l, slot - s0 + (threadIdx.x & 63), po, i, j);
+      const int nx = lx(l), ny = ly(l), o = lo(l);
+      rpos[b] = fpo + 2 * j * (lx(l - 1) + 2) + 2 * i;
+      uint8_t g[3][3];
+#pragma unroll
+      for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          const int ii = i + dx - 1, jj = j + dy - 1;
+          const bool in = ii >= 0 && ii < nx && jj >= 0 && jj < ny;
+          const uint8_t fv = inf[o + (in ? ii + jj * nx : 0)];
+          g[dy][dx] = in ? fv : kWall;
+        }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int dx = (c & 1) ? 2 : 0, dy = (c >> 1) ? 2 : 0;
+        bm[b][c] = moved_weight(g[1][dx], g[dy][1], g[dy][dx]);
+      }
+    }
+  }
+  auto get_rhs = [&] {
+    bool act[K];
+    float r[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) act[k] = A[k].act;
+    rhs(act, r);
+#pragma unroll
+    for (int k = 0; k < K; ++k) A[k].r = r[k];
+  };
+  __syncthreads();  // the zeros are there
+  if (nl == 1) {
+    get_rhs();
+    if (threadIdx.x < 64)
+      A[0].x = coarsest_sweeps(A[0].r, A[0].nn, A[0].inv, A[0].act, lx(0), ly(0), sweeps);
+    out(0, A[0].x);
+    return;
+  }
+  // f on every cell of level l that this thread holds
+  auto each = [&](int l, auto&& f) {
+    if (l == 0) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) f(A[k], k);
+    } else {
+#pragma unroll
+      for (int b = 0; b < KB; ++b)
+        if (bl[b] == l) f(B[b], b);
+    }
+  };
+  auto nbrs = [&](const float* P, int pos, int pitch) {
+    return P[pos - 1] + P[pos + 1] + P[pos - pitch] + P[pos + pitch];
+  };
+  auto sweep = [&](int l, const float* src, float wgt, float* dst) {
+    const int pitch = lx(l) + 2;
+    each(l, [&](StageCell& c, int) {
+      const float s = nbrs(src, c.pos, pitch);
+      c.x = c.act ? c.x + wgt * (c.r - (c.nn * c.x - s)) * c.inv : 0.f;
+      if (dst && c.in) dst[c.pos] = c.x;
+    });
+  };
+  get_rhs();
+  each(0, [&](StageCell& c, int) {
+    c.x = w * c.r * c.inv;
+    if (c.in) P0[c.pos] = c.x;
+  });
+  __syncthreads();
+  for (int l = 0; l < nl - 1; ++l) {
+    const int pitch = lx(l) + 2;
+    sweep(l, P0, w2, P1);
+    __syncthreads();
+    each(l, [&](StageCell& c, int) {
+      const float s = nbrs(P1, c.pos, pitch);
+      const float res = c.act ? c.r - (c.nn * c.x - s) : 0.f;
+      if (c.in) P0[c.pos] = res;
+    });
+    __syncthreads();
+    each(l + 1, [&](StageCell& c, int b) {
+      // fine rows / columns 2J-1 .. 2J+2 and 2I-1 .. 2I+2
+      const float wt[4] = {0.25f, 0.75f, 0.75f, 0.25f};
+      float t[4][4], v = 0.f;
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) t[y][x] = P0[rpos[b] + y * pitch + x];
+#pragma unroll
+      for (int y = 0; y < 4; ++y)
+        v += wt[y] * (wt[0] * t[y][0] + wt[1] * t[y][1] + wt[2] * t[y][2] + wt[3] * t[y][3]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v += bm[b][q] * t[1 + (q >> 1)][1 + (q & 1)];
+      c.r = c.act ? v : 0.f;
+      if (l + 1 < nl - 1) {
+        c.x = w * c.r * c.inv;
+        if (c.in) P0[c.pos] = c.x;
+      } else {
+        c.x = coarsest_sweeps(c.r, c.nn, c.inv, c.act, lx(l + 1), ly(l + 1), sweeps);
+        if (c.in) P1[c.pos] = c.x;
+      }
+    });
+    __syncthreads();
+  }
+  for (int l = nl - 2; l >= 0; --l) {
+    const int epitch = lx(l + 1) + 2;
+    each(l, [&](StageCell& c, int) {
+      const int edx = (c.ebits & 1) ? 1 : -1, edy = (c.ebits & 2) ? epitch : -epitch;
+      const float e0 = P1[c.epos], ex = P1[c.epos + edx], ey = P1[c.epos + edy];
+      const float exy = P1[c.epos + edx + edy];
+      const uint8_t fx = (c.ebits & 4) ? kWall : 0, fy = (c.ebits & 8) ? kWall : 0;
+      const float pe = prolong_value(e0, ex, fx, ey, fy, exy, (c.ebits & 16) ? kWall : 0);
+      c.x = c.act ? c.x + pe : 0.f;
+      if (c.in) P1[c.pos] = c.x;
+    });
+    __syncthreads();
+    sweep(l, P1, w, P0);
+    __syncthreads();
+    sweep(l, P0, w2, l > 0 ? P1 : nullptr);
+    if (l > 0) __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) out(k, A[k].x);
+}
+
 // The kernel's own duration from the device wall clock (clk != null): clk[0] += end -
 // start (ticks), clk[1] += 1, by thread 0 after the workgroup's last barrier.
 __device__ __forceinline__ void kclock_end(unsigned long long* clk, unsigned long long t0) {
@@ -1665,55 +1959,61 @@ __device__ __forceinline__ void kclock_end(unsigned long long* clk, unsigned lon
   }
 }
 
-// With check != 0 (the hierarchy starts in this kernel) it runs level 0's
-// convergence test first and forms the r.z partial at the end.
-// The one-workgroup stage: load its levels' info and level lc's right-hand side into
-// LDS, cycle, store level lc's result (and, when the hierarchy starts here, the r.z
-// partial).  `coherent`: the right-hand side was written by other workgroups of the
-// same launch with device-coherent stores, so it is read the same way.
-template <int CT>
-__device__ __forceinline__ void coarse_stage(const MgCoarseArgs& a, double* part_rz,
-                                             bool coherent) {
-  __shared__ double sm[2 * 16];
-  __shared__ int s_lv[3 * kMgMaxLevels];
-  extern __shared__ float lds[];
-  const int tot = a.total;  // a multiple of 4
-  float* R = lds;
-  float* X = R + tot;
-  float* T = X + tot;
-  uint8_t* INF = reinterpret_cast<uint8_t*>(T + tot);
-  const int nl = a.nlev - a.lc;
-  if (threadIdx.x < nl) {
+// The one-workgroup levels' sizes and LDS offsets (a.off[l] - a.off[a.lc]) in s_lv.
+__device__ __forceinline__ void coarse_sizes(const MgCoarseArgs& a, int* s_lv) {
+  if (threadIdx.x < a.nlev - a.lc) {
     const int l = a.lc + threadIdx.x;
     s_lv[threadIdx.x] = a.nx[l];
     s_lv[kMgMaxLevels + threadIdx.x] = a.ny[l];
     s_lv[2 * kMgMaxLevels + threadIdx.x] = a.off[l] - a.off[a.lc];
   }
-  {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(a.inf_all);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(INF);
-    for (int q = threadIdx.x; q < tot / 4; q += CT) dst[q] = src[q];
-    const int n0 = a.nx[a.lc] * a.ny[a.lc];
-    for (int q = threadIdx.x; q < n0; q += CT)
-      R[q] = coherent ? ld_dev(a.r_in + q) : a.r_in[q];
-  }
-  __syncthreads();
-  coarse_cycle<CT>(nl, s_lv, s_lv + kMgMaxLevels, s_lv + 2 * kMgMaxLevels, a.omega, a.omega2,
-               a.sweeps, R, X, T, INF, a.trunc);
-  const int n = a.nx[a.lc] * a.ny[a.lc];
-  const float* res = nl == 1 && a.trunc == 0 ? X : T;
-  double rz = 0.0;
-  for (int q = threadIdx.x; q < n; q += CT) {
-    a.x_out[q] = res[q];
-    rz += (double)R[q] * (double)res[q];
-  }
-  if (part_rz) {
-    double v[1] = {rz};
-    block_sum<1, CT>(v, sm);
-    if (threadIdx.x == 0) part_rz[0] = v[0];
-  }
 }
 
+// The one-workgroup stage of one domain: rhs as for stage_cycle with K = 1; out(r, x) for a
+// thread that holds a cell of the first level.
+template <int NT, class Rhs, class Out>
+__device__ __forceinline__ void coarse_run(const MgCoarseArgs& a, float* lds, int* s_lv,
+                                           Rhs&& rhs, Out&& out) {
+  static_assert(kMgCoarseCells <= NT, "a thread per cell of the first level");
+  const int nl = a.nlev - a.lc, n = a.nx[a.lc] * a.ny[a.lc];
+  if (a.words > 0) {
+    float r0 = 0.f;
+    stage_cycle<NT, 1, kStageKB>(
+        nl, [&](int l) { return a.nx[a.lc + l]; }, [&](int l) { return a.ny[a.lc + l]; },
+        [&](int l) { return a.off[a.lc + l] - a.off[a.lc]; }, a.inf_all, a.omega, a.omega2,
+        a.sweeps, lds, a.words,
+        [&](const bool (&act)[1], float (&r)[1]) {
+          rhs(act, r);
+          r0 = r[0];
+        },
+        [&](int, float x) {
+          if (threadIdx.x < n) out(r0, x);
+        });
+    return;
+  }
+  // truncated to the first level, or too elongated for the registers
+  const int tot = a.total;  // a multiple of 4
+  float *R = lds, *X = R + tot, *T = X + tot;
+  uint8_t* INF = reinterpret_cast<uint8_t*>(T + tot);
+  coarse_sizes(a, s_lv);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(a.inf_all);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(INF);
+  for (int q = threadIdx.x; q < tot / 4; q += NT) dst[q] = src[q];
+  const bool act[1] = {threadIdx.x < n && is_act(a.inf_all[threadIdx.x < n ? threadIdx.x : 0])};
+  float r[1];
+  rhs(act, r);
+  if (threadIdx.x < n) R[threadIdx.x] = r[0];
+  __syncthreads();
+  coarse_cycle<NT>(nl, s_lv, s_lv + kMgMaxLevels, s_lv + 2 * kMgMaxLevels, a.omega, a.omega2,
+                   a.sweeps, R, X, T, INF, a.trunc);
+  const float* res = nl == 1 && a.trunc == 0 ? X : T;
+  if (threadIdx.x < n) out(r[0], res[threadIdx.x]);
+}
+
+// The one-workgroup stage as a launch of its own (hierarchies with at most one tile
+// level): load its levels' info and level lc's right-hand side into LDS, cycle, store level
+// lc's result.  With check != 0 (the hierarchy starts in this kernel) it runs level 0's
+// convergence test first and forms the r.z partial at the end.
 __global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse(MgCoarseArgs a, MgCheck chk, int it,
                                                              int check,
                                                              double* __restrict__ part_rz,
@@ -1721,7 +2021,7 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse(MgCoarseArgs a, Mg
   const unsigned long long t0 = clk ? wall_clock64() : 0ull;
   __shared__ double sm[2 * 16];
   if (check) {
-    if (mg_check<kCoarseThreads>(chk, it, sm)) {
+    if (mg_check<kCoarseThreads>(chk, it, true, sm)) {
       kclock_end(clk, t0);
       return;
     }
@@ -1729,7 +2029,23 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_coarse(MgCoarseArgs a, Mg
     kclock_end(clk, t0);
     return;
   }
-  coarse_stage<kCoarseThreads>(a, part_rz, false);
+  __shared__ int s_lv[3 * kMgMaxLevels];
+  extern __shared__ float lds[];
+  double rz = 0.0;
+  coarse_run<kCoarseThreads>(
+      a, lds, s_lv,
+      [&](const bool (&)[1], float (&r)[1]) {
+        r[0] = threadIdx.x < a.nx[a.lc] * a.ny[a.lc] ? a.r_in[threadIdx.x] : 0.f;
+      },
+      [&](float r, float x) {
+        a.x_out[threadIdx.x] = x;
+        rz = (double)r * (double)x;
+      });
+  if (part_rz) {
+    double v[1] = {rz};
+    block_sum<1, kCoarseThreads>(v, sm);
+    if (threadIdx.x == 0) part_rz[0] = v[0];
+  }
   if (clk) {
     __syncthreads();
     kclock_end(clk, t0);
@@ -1785,36 +2101,415 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_scene_setup(SceneCoarseAr
   }
 }
 
+// One V-cycle of scene `scene`'s own levels.  rhs(act, cell, r):
+// the right-hand side at the packed cells cell[k]; out(cell, x): the result there.
+constexpr int kSceneK = kSceneCoarseCells / kCoarseThreads;
+template <class Rhs, class Out>
+__device__ __forceinline__ void scene_run(const SceneCoarseArgs& a, int scene, float* lds,
+                                          Rhs&& rhs, Out&& out) {
+  constexpr int NT = kCoarseThreads, K = kSceneK;
+  // the table entry through scalar loads (it is not written while a kernel runs)
+  const auto& t = *(const __attribute__((address_space(4))) SceneCoarse*)(a.tab + scene);
+  const int nx = t.nx[0], n = nx * t.ny[0], cl = t.nl - 1;
+  const int sweeps = 2 * (t.nx[cl] > t.ny[cl] ? t.nx[cl] : t.ny[cl]) + 8;
+  const uint8_t* inf = a.inf_all + (size_t)scene * a.stride;
+  const float inv_nx = 1.0f / (float)nx;
+  int cell[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int q = threadIdx.x + k * NT;
+    int i, j;
+    small_divmod(q < n ? q : 0, nx, inv_nx, i, j);
+    cell[k] = t.cx + i + (t.cy + j) * a.pitch;
+  }
+  if (t.words > 0 && a.trunc == 0) {
+    stage_cycle<NT, K, kSceneKB>(
+        t.nl, [&](int l) { return t.nx[l]; },
+        [&](int l) { return t.ny[l]; }, [&](int l) { return t.off[l]; }, inf, a.omega, a.omega2, sweeps, lds, t.words,
+        [&](const bool (&act)[K], float (&r)[K]) { rhs(act, cell, r); },
+        [&](int k, float x) {
+          if (threadIdx.x + k * NT < n) out(cell[k], x);
+        });
+    return;
+  }
+  const int tot = a.stride;  // a multiple of 4, >= t.total
+  float *R = lds, *X = R + tot, *T = X + tot;
+  uint8_t* INF = reinterpret_cast<uint8_t*>(T + tot);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(inf);
+  uint32_t* dst = reinterpret_cast<uint32_t*>(INF);
+  for (int q = threadIdx.x; q < t.total / 4; q += NT) dst[q] = src[q];
+  bool act[K];
+  float r[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int q = threadIdx.x + k * NT;
+    act[k] = q < n && is_act(inf[q < n ? q : 0]);
+  }
+  rhs(act, cell, r);
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (threadIdx.x + k * NT < n) R[threadIdx.x + k * NT] = r[k];
+  __shared__ int s_lv[3 * kSceneMaxLevels];
+  if (threadIdx.x < t.nl) {
+    s_lv[threadIdx.x] = a.tab[scene].nx[threadIdx.x];
+    s_lv[kSceneMaxLevels + threadIdx.x] = a.tab[scene].ny[threadIdx.x];
+    s_lv[2 * kSceneMaxLevels + threadIdx.x] = a.tab[scene].off[threadIdx.x];
+  }
+  __syncthreads();
+  coarse_cycle<NT>(t.nl, s_lv, s_lv + kSceneMaxLevels, s_lv + 2 * kSceneMaxLevels, a.omega, a.omega2, sweeps, R, X, T, INF, a.trunc);
+  const float* res = t.nl == 1 && a.trunc == 0 ? X : T;
+#pragma unroll
+  for (int k = 0; k < K; ++k)
+    if (threadIdx.x + k * NT < n) out(cell[k], res[threadIdx.x + k * NT]);
+}
+
 // One V-cycle of every scene's own levels: right-hand side from the packed level la,
 // result back into it (cells outside every rectangle keep their zero).
 __global__ void __launch_bounds__(kCoarseThreads) k_mg_scene_coarse(SceneCoarseArgs a,
                                                                    const CgScalars* sc) {
-  __shared__ SceneCoarse t;
   if (sc->done) return;
-  if (threadIdx.x == 0) t = a.tab[blockIdx.x];
-  __syncthreads();
   extern __shared__ float lds[];
-  const int tot = a.stride;  // a multiple of 4, >= t.total
-  float* R = lds;
-  float* X = R + tot;
-  float* T = X + tot;
-  uint8_t* INF = reinterpret_cast<uint8_t*>(T + tot);
-  const int nx = t.nx[0], n0 = nx * t.ny[0];
+  scene_run(
+      a, blockIdx.x, lds,
+      [&](const bool (&act)[kSceneK], const int (&cell)[kSceneK], float (&r)[kSceneK]) {
+#pragma unroll
+        for (int k = 0; k < kSceneK; ++k) {
+          const float v = a.r_in[cell[k]];
+          r[k] = act[k] ? v : 0.f;
+        }
+      },
+      [&](int cell, float x) { a.x_out[cell] = x; });
+}
+
+// ---------------------------------------------------------------- the smaller levels
+// The V-cycle's tile levels from the first of at most kCycleTiles tiles on, and the
+// one-workgroup stage (a batch: every scene's), in one launch.  On their own each of these
+// kernels takes 4.5-8 us of which the arithmetic is about 1.5: the rest is the boundary
+// between two launches and the first loads after it.  Here the grid is all tasks of the
+// launch -- a task is one tile going down, one one-workgroup stage or one tile going up --
+// and a task starts as soon as the values that it reads are there, 0.5 us after they were
+// stored.  Three levels (256^2 .. 64^2) and the stage: 26 us, in seven launches 50 us.  Per
+// step: 130 x 96 cells 362 -> 304 us, 513 x 385 558 -> 434, 1024^2 783 -> 661, 2048^2
+// 1120 -> 1013.
+//
+// Tasks are taken from a counter in the order of the cycle (down level by level, the
+// stage, up level by level), and a task waits only for tasks before it: those are finished
+// or held by workgroups that are running, so every wait ends however few workgroups the
+// device holds at a time.
+//
+// A value that crosses tasks is one 64-bit word, the float and the launch's number, stored
+// and loaded device-coherent: a reader that finds the number has the value, so nothing
+// is fenced, counted or cleared.  Only unknowns are waited for; elsewhere every level's
+// values are zero.  A task that would wait long first watches one word (hint) of a task
+// two steps ahead of it in the chain with one thread, so that the idle tasks' polls do not
+// crowd out the others' loads.
+//
+// Waits are bounded all the same (kSpinMax polls of about a microsecond): one that runs out
+// marks the solve as failed instead of keeping the device busy for good.
+constexpr int kCycNT = 1024;
+constexpr int kSpinMax = 1 << 20;
+
+__device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
+  return ((unsigned long long)tag << 32) | __float_as_uint(v);
+}
+__device__ __forceinline__ float untag(unsigned long long w) {
+  return __uint_as_float((unsigned)w);
+}
+
+// v[k] = the value of word p[k] once it carries the tag, for the k with need[k]; 0 else.
+// (Without need p[k] is still read: it points to any word.)
+template <int N>
+__device__ __forceinline__ void wait_tagged(const unsigned long long* const (&p)[N],
+                                            const bool (&need)[N], unsigned tag, int* stuck,
+                                            float (&v)[N]) {
+  unsigned long long w[N];
+  for (int n = 0;; ++n) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) w[k] = ld_dev(p[k]);
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < N; ++k) ok &= !need[k] || (unsigned)(w[k] >> 32) == tag;
+    if (ok) break;
+    if (n == kSpinMax) {
+      st_dev(stuck, 1);
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = need[k] ? untag(w[k]) : 0.f;
+}
+
+// Until the task's hint carries the tag (thread 0 watches; a barrier).
+// Hints lie kHintPitch words apart: polls of one line follow each other at 10 ns or so, so
+// neither other pollers nor the store should share it.
+constexpr int kHintPitch = 32;
+constexpr int kFlags = 32;  // copies of the stop test's result, a line each
+__device__ __forceinline__ void wait_hint(const unsigned* hint, int task, unsigned tag,
+                                          int* stuck) {
+  if (threadIdx.x == 0)
+    for (int n = 0; ld_dev(hint + task * kHintPitch) != tag; ++n) {
+      if (n == kSpinMax) {
+        st_dev(stuck, 1);
+        break;
+      }
+      __builtin_amdgcn_s_sleep(4);
+    }
+  __syncthreads();
+}
+
+template <int S, class Stopped>
+__device__ __forceinline__ void cycle_down(const MgCycleArgs& a, int k, int tile, unsigned tag,
+                                           const float (&wk)[kMgMaxSweeps], int* stuck,
+                                           float* lds, Stopped&& stopped) {
+  constexpr int NT = kCycNT, W = 34 + 2 * S, WC = kDownWC;
+  using St = Strip<W, NT>;
+  constexpr int R = St::R;
+  static_assert(WC * WC <= NT, "a thread per cell of the coarse frame");
+  const MgCycleLevel f = a.lv[k], c = a.lv[k + 1];
+  const bool empty = f.tflag && !f.tflag[tile];  // no unknown on either level
+  float *s_x0 = lds, *s_x1 = lds + St::N;
+  uint8_t* s_cinf = reinterpret_cast<uint8_t*>(lds + 2 * St::N);
+  const int bx = tile % f.tiles_x, by = tile / f.tiles_x;
+  const TileStrip<NT, W, S + 1> ts(bx * 32, by * 32, f.nx, f.ny);
+  uint8_t fv[R];
+  float rv[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const uint8_t fq = f.inf[ts.cell[q]];
+    fv[q] = ts.in[q] ? fq : 0;
+  }
+  uint8_t cv;
   {
-    const uint32_t* src =
-        reinterpret_cast<const uint32_t*>(a.inf_all + (size_t)blockIdx.x * a.stride);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(INF);
-    for (int q = threadIdx.x; q < t.total / 4; q += kCoarseThreads) dst[q] = src[q];
-    for (int q = threadIdx.x; q < n0; q += kCoarseThreads)
-      R[q] = a.r_in[(size_t)(t.cx + q % nx) + (size_t)(t.cy + q / nx) * a.pitch];
+    const int t = threadIdx.x;
+    const int I = bx * 16 + t % WC - 1, J = by * 16 + t / WC - 1;
+    const bool inc = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
+    const uint8_t v = c.inf[inc ? I + J * c.nx : 0];
+    cv = inc ? v : kWall;
+  }
+  if (k == 0) {  // written by the kernel before this one
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const float rq = f.r[ts.cell[q]];
+      rv[q] = ts.in[q] ? rq : 0.f;
+    }
+  }
+  // a task of the first level asks for the stop test's result when it has its own
+  if (empty || (k > 0 && stopped())) return;
+  if (k > 0) {
+    if (k >= 2) {
+      const MgCycleLevel g = a.lv[k - 2];
+      wait_hint(a.hint, g.down0 + 4 * bx + 4 * by * g.tiles_x, tag, stuck);
+    }
+    const unsigned long long* p[R];
+    bool need[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      p[q] = f.tr + ts.cell[q];
+      need[q] = is_act(fv[q]);
+    }
+    wait_tagged<R>(p, need, tag, stuck, rv);
+  }
+  if (threadIdx.x < WC * WC) s_cinf[threadIdx.x] = cv;
+  down_core<NT, S>(ts, fv, rv, wk, s_x0, s_x1, s_cinf, bx, by, c.nx, c.ny,
+                   [&](int q, float x) { st_dev(f.ts + ts.cell[q], tagged(x, tag)); },
+                   [&](int q, float v) { st_dev(c.tr + q, tagged(v, tag)); },
+                   [&] { return k == 0 && stopped(); });
+}
+
+template <int S, class Stopped>
+__device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, unsigned tag,
+                                         int it, const float (&wk)[kMgMaxSweeps], int* stuck,
+                                         float* lds, Stopped&& stopped) {
+  constexpr int NT = kCycNT, W = 32 + 2 * S, WC = UpFrame<S>::WC, CO = UpFrame<S>::CO;
+  using St = Strip<W, NT>;
+  constexpr int R = St::R;
+  static_assert(WC * WC <= NT, "a thread per cell of the coarse frame");
+  const MgCycleLevel f = a.lv[k], c = a.lv[k + 1];
+  const int bx = tile % f.tiles_x, by = tile / f.tiles_x;
+  const int fi0 = bx * 32, fj0 = by * 32;
+  const bool empty = f.tflag && !f.tflag[tile];
+  float *s_x0 = lds, *s_x1 = lds + St::N, *s_e = lds + 2 * St::N;
+  uint8_t* s_cinf = reinterpret_cast<uint8_t*>(s_e + WC * WC);
+  const TileStrip<NT, W, S> ts(fi0, fj0, f.nx, f.ny);
+  uint8_t fv[R], cv;
+  float rv[R], x[R], r0[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const uint8_t fq = f.inf[ts.cell[q]];
+    const float rq = k == 0 ? f.r[ts.cell[q]] : 0.f;
+    fv[q] = ts.in[q] ? fq : 0;
+    r0[q] = ts.in[q] ? rq : 0.f;
+  }
+  int ce;
+  {
+    const int t = threadIdx.x;
+    const int I = (fi0 >> 1) - CO + t % WC, J = (fj0 >> 1) - CO + t / WC;
+    const bool inc = t < WC * WC && I >= 0 && I < c.nx && J >= 0 && J < c.ny;
+    ce = inc ? I + J * c.nx : 0;
+    const uint8_t v = c.inf[ce];
+    cv = inc ? v : kWall;
+  }
+  if (stopped()) return;
+  if (empty) {
+    // no unknown on either level: zero (written once per solve)
+    const int i = fi0 + (threadIdx.x & 31), j = fj0 + (threadIdx.x >> 5);
+    if (k == 0 && it == 0 && i < f.nx && j < f.ny) f.xo[i + j * f.nx] = 0.f;
+    return;
+  }
+  // the level's own values on the way down once the tile's task is done (its neighbours'
+  // follow soon), then the coarse result
+  wait_hint(a.hint, f.down0 + tile, tag, stuck);
+  {
+    const unsigned long long* p[2 * R];
+    bool need[2 * R];
+    float v[2 * R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      p[q] = f.ts + ts.cell[q];
+      need[q] = is_act(fv[q]);
+      p[R + q] = k == 0 ? p[q] : f.tr + ts.cell[q];
+      need[R + q] = need[q];
+    }
+    wait_tagged<2 * R>(p, need, tag, stuck, v);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      x[q] = v[q];
+      rv[q] = k == 0 ? r0[q] : v[R + q];
+    }
+  }
+  if (k + 2 < a.nl) {
+    const MgCycleLevel g = a.lv[k + 2];
+    wait_hint(a.hint, g.up0 + (bx >> 2) + (by >> 2) * g.tiles_x, tag, stuck);
+  } else {
+    const int sh = a.nl - 1 - k;
+    const MgCycleLevel g = a.lv[a.nl - 1];
+    wait_hint(a.hint, g.down0 + (bx >> sh) + (by >> sh) * g.tiles_x, tag, stuck);
+  }
+  const unsigned long long* const pe[1] = {c.te + ce};
+  const bool ne[1] = {is_act(cv)};
+  float ev[1];
+  wait_tagged<1>(pe, ne, tag, stuck, ev);
+  if (threadIdx.x < WC * WC) {
+    s_e[threadIdx.x] = ev[0];
+    s_cinf[threadIdx.x] = cv;
   }
   __syncthreads();
-  const int cl = t.nl - 1;
-  const int sweeps = 2 * (t.nx[cl] > t.ny[cl] ? t.nx[cl] : t.ny[cl]) + 8;
-  coarse_cycle<kCoarseThreads>(t.nl, t.nx, t.ny, t.off, a.omega, a.omega2, sweeps, R, X, T, INF, a.trunc);
-  const float* res = t.nl == 1 && a.trunc == 0 ? X : T;
-  for (int q = threadIdx.x; q < n0; q += kCoarseThreads)
-    a.x_out[(size_t)(t.cx + q % nx) + (size_t)(t.cy + q / nx) * a.pitch] = res[q];
+  up_core<NT, S>(ts, fv, rv, x, wk, s_x0, s_x1, s_e, s_cinf);
+#pragma unroll
+  for (int q = 0; q < R; ++q)
+    if (ts.own[q]) {
+      const float xo = is_act(fv[q]) ? x[q] : 0.f;
+      if (k == 0)
+        f.xo[ts.cell[q]] = xo;
+      else
+        st_dev(f.te + ts.cell[q], tagged(xo, tag));
+    }
+}
+
+// The one-workgroup stage of one domain, and of scene `s` of a batch (the cells of its
+// rectangle of the packed level, cells outside every rectangle hold no unknown).
+__device__ __forceinline__ void cycle_coarse(const MgCoarseArgs& a, const MgCycleLevel& f,
+                                             unsigned tag, int* stuck, float* lds) {
+  __shared__ int s_lv[3 * kMgMaxLevels];
+  const int n = f.nx * f.ny;
+  coarse_run<kCycNT>(
+      a, lds, s_lv,
+      [&](const bool (&act)[1], float (&r)[1]) {
+        const unsigned long long* const p[1] = {f.tr + (threadIdx.x < n ? threadIdx.x : 0)};
+        wait_tagged<1>(p, act, tag, stuck, r);
+      },
+      [&](float, float x) { st_dev(f.te + threadIdx.x, tagged(x, tag)); });
+}
+
+__device__ __forceinline__ void cycle_scene(const SceneCoarseArgs& a, const MgCycleLevel& f,
+                                            int scene, unsigned tag, int* stuck, float* lds) {
+  static_assert(kCycNT == kCoarseThreads, "the stage's workgroup");
+  scene_run(
+      a, scene, lds,
+      [&](const bool (&act)[kSceneK], const int (&cell)[kSceneK], float (&r)[kSceneK]) {
+        const unsigned long long* p[kSceneK];
+#pragma unroll
+        for (int k = 0; k < kSceneK; ++k) p[k] = f.tr + cell[k];
+        wait_tagged<kSceneK>(p, act, tag, stuck, r);
+      },
+      [&](int cell, float x) { st_dev(f.te + cell, tagged(x, tag)); });
+}
+
+// S sweeps per tile level; BATCH: the scenes' stages in place of one.  check != 0: the stop
+// test runs here, as the first task, and the others wait for its result before they wait
+// for anything else (in every workgroup, at 512 of them, it took 3.5 us more).
+template <int S, bool BATCH>
+__global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk, int it, int check,
+                                                     MgSweeps sw, MgCoarseArgs ca,
+                                                     SceneCoarseArgs sa) {
+  extern __shared__ float lds[];
+  __shared__ double sm[kCycNT / 64];
+  __shared__ unsigned long long s_ticket;
+  __shared__ int s_stop;
+  // the counter: the launch's number and the next task.  Every workgroup draws one; the one
+  // with the last task sets the counter for the next launch.
+  unsigned long long ticket = 0;
+  if (threadIdx.x == 0)
+    ticket = __hip_atomic_fetch_add(a.ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  int done = 0;
+  if (threadIdx.x == 0)
+    done = __hip_atomic_load(&chk.sc->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (threadIdx.x == 0) {
+    s_ticket = ticket;
+    s_stop = done;
+  }
+  __syncthreads();
+  const unsigned task = __builtin_amdgcn_readfirstlane((unsigned)s_ticket);
+  const unsigned launch = __builtin_amdgcn_readfirstlane((unsigned)(s_ticket >> 32));
+  if (task == a.n_tasks - 1 && threadIdx.x == 0)
+    st_dev(a.ticket, (unsigned long long)(launch + 1) << 32);
+  if (s_stop) return;
+  const unsigned tag = launch + 1;  // the words start out as zero
+  if (task == 0) {  // the stop test, for all
+    if (check) {
+      const bool stop = mg_check<kCycNT>(chk, it, true, sm);
+      if (threadIdx.x < kFlags) st_dev(a.flag + threadIdx.x * kHintPitch, 2 * tag + (stop ? 1 : 0));
+    }
+    return;
+  }
+  int* const stuck = &chk.sc->stuck;
+  // (a task calls it when its first loads are under way, all threads alike)
+  auto stopped = [&]() __attribute__((always_inline)) {
+    if (!check) return false;
+    if (threadIdx.x == 0) {
+      const unsigned* const flag = a.flag + (task % kFlags) * kHintPitch;
+      unsigned w = ld_dev(flag);
+      for (int n = 0; (w >> 1) != (tag & 0x7fffffffu); w = ld_dev(flag)) {
+        if (++n == kSpinMax) {
+          st_dev(stuck, 1);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      s_stop = (int)(w & 1);
+    }
+    __syncthreads();
+    return s_stop != 0;
+  };
+  float wk[kMgMaxSweeps];
+  sweep_weights<S>(sw, ca.omega, ca.omega2, wk);
+  if (task < a.coarse0) {
+    int k = 0;
+    while (k + 1 < a.nl && task >= a.lv[k + 1].down0) ++k;
+    cycle_down<S>(a, k, (int)(task - a.lv[k].down0), tag, wk, stuck, lds, stopped);
+  } else if (task < a.up0) {
+    if (stopped()) return;
+    if constexpr (BATCH)
+      cycle_scene(sa, a.lv[a.nl], (int)(task - a.coarse0), tag, stuck, lds);
+    else
+      cycle_coarse(ca, a.lv[a.nl], tag, stuck, lds);
+  } else {
+    int k = a.nl - 1;
+    while (k > 0 && task >= a.lv[k - 1].up0) --k;
+    cycle_up<S>(a, k, (int)(task - a.lv[k].up0), tag, it, wk, stuck, lds, stopped);
+  }
+  if (threadIdx.x == 0) st_dev(a.hint + task * kHintPitch, tag);
 }
 
 // ---------------------------------------------------------------- CG vectors
@@ -2485,17 +3180,22 @@ hipError_t mg_set_lds_limit(size_t bytes) {
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_coarse),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
   if (e != hipSuccess) return e;
-  // the last tile level's down kernel hosts the same stage (its own static LDS aside)
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  // as does the smaller levels' kernel
+  auto cyc = [&](auto ns) {
+    constexpr int S = decltype(ns)::value;
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_cycle<S, false>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_cycle<S, true>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  };
+  cyc(std::integral_constant<int, 2>{});
+  cyc(std::integral_constant<int, 3>{});
+  cyc(std::integral_constant<int, 4>{});
+  cyc(std::integral_constant<int, 5>{});
+  cyc(std::integral_constant<int, 6>{});
   if (e != hipSuccess) return e;
-  for (const void* f : {reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 3>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 4>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 5>),
-                        reinterpret_cast<const void*>(&k_mg_down<false, kTileFew, false, true, 6>)}) {
-    e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    if (e != hipSuccess) return e;
-  }
   return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_mg_scene_coarse),
                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
@@ -2505,8 +3205,7 @@ void launch_mg_scene_setup(hipStream_t s, const SceneCoarseArgs& a) {
 }
 
 void launch_mg_scene_coarse(hipStream_t s, const SceneCoarseArgs& a, CgScalars* sc) {
-  k_mg_scene_coarse<<<a.n_scenes, kCoarseThreads, (size_t)a.stride * (3 * sizeof(float) + 1), s>>>(
-      a, sc);
+  k_mg_scene_coarse<<<a.n_scenes, kCoarseThreads, a.lds, s>>>(a, sc);
 }
 
 void launch_mg_setup(hipStream_t s, const Geom& g, const MgHost& m, const uint8_t* label,
@@ -2689,6 +3388,18 @@ static MgSweeps mg_sweeps(const MgHost& m) { return cheb_sweeps(m.level_sweeps);
 // level 0: three sweeps take the degree-3 weights on [0.2, 2]
 static MgSweeps mg_sweeps0(const MgHost& m) { return cheb_sweeps(m.level0_sweeps); }
 
+// f(S) with S = the sweeps of the tile levels below level 0 as a constant
+template <class F>
+static void with_sweeps(const MgHost& m, F&& f) {
+  switch (m.level_sweeps) {
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    default: f(std::integral_constant<int, 2>{}); break;
+  }
+}
+
 // One CG iteration = V-cycle (z = B r) + direction + update.  Level 0's down kernel
 // (or the one-workgroup kernel when the hierarchy starts there) runs the stop test
 // of this iteration first.
@@ -2716,13 +3427,13 @@ void launch_mg_down(hipStream_t s, MgHost& m, int l, int it, int max_iter, doubl
     auto go = [&](auto nt, auto ns) {
       constexpr int NT = decltype(nt)::value, S = decltype(ns)::value;
       if (m.fused)
-        k_mg_down<true, NT, true, false, S><<<blocks, NT, 0, s>>>(
+        k_mg_down<true, NT, true, S><<<blocks, NT, 0, s>>>(
             mg_level(m, 0), mg_level(m, 1), m.coarse.omega, m.coarse.omega2, it, chk, ck, m.tflag,
-            xr, span, MgCoarseArgs{}, nullptr, sw0, m.tmap);
+            xr, span, sw0, m.tmap);
       else
-        k_mg_down<true, NT, false, false, S><<<blocks, NT, 0, s>>>(
+        k_mg_down<true, NT, false, S><<<blocks, NT, 0, s>>>(
             mg_level(m, 0), mg_level(m, 1), m.coarse.omega, m.coarse.omega2, it, chk, ck, m.tflag,
-            xr, span, MgCoarseArgs{}, nullptr, sw0, m.tmap);
+            xr, span, sw0, m.tmap);
     };
     auto go_s = [&](auto nt) {
       if (m.level0_sweeps == 3)
@@ -2737,38 +3448,100 @@ void launch_mg_down(hipStream_t s, MgHost& m, int l, int it, int max_iter, doubl
     else
       go_s(std::integral_constant<int, kT>{});
   } else {
-    // the last tile level also runs the one-workgroup stage (mg_tail_coarse): its own
-    // instance, so that the other levels (and every level of a batch) carry none of it
-    // (its coarse level holds at most kMgCoarseCells cells, so it has at most 64 tiles);
-    // m.level_sweeps sweeps before the coarse correction
+    // the tile levels of more than kCycleTiles tiles (launch_mg_cycle runs the others)
     const MgSweeps sw = mg_sweeps(m);
-    auto go = [&](auto ns) {
+    with_sweeps(m, [&](auto ns) {
       constexpr int S = decltype(ns)::value;
-      if (l == m.lc - 1 && mg_tail_coarse(m))
-        k_mg_down<false, kTileFew, false, true, S><<<blocks, kTileFew, m.coarse_lds, s>>>(
-            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
-            m.tflag_l[l], MgXr{}, nullptr, m.coarse, m.ticket, sw, nullptr);
-      else if (few_tiles(mg_up_blocks(m.nx[l], m.ny[l])))
-        k_mg_down<false, kTileFew, false, false, S><<<blocks, kTileFew, 0, s>>>(
-            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
-            m.tflag_l[l], MgXr{}, nullptr, MgCoarseArgs{}, nullptr, sw, nullptr);
-      else
-        k_mg_down<false, kTileMany, false, false, S><<<blocks, kTileMany, 0, s>>>(
-            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
-            m.tflag_l[l], MgXr{}, nullptr, MgCoarseArgs{}, nullptr, sw, nullptr);
-    };
-    switch (m.level_sweeps) {
-      case 3: go(std::integral_constant<int, 3>{}); break;
-      case 4: go(std::integral_constant<int, 4>{}); break;
-      case 5: go(std::integral_constant<int, 5>{}); break;
-      case 6: go(std::integral_constant<int, 6>{}); break;
-      default: go(std::integral_constant<int, 2>{}); break;
-    }
+      k_mg_down<false, kTileMany, false, S><<<blocks, kTileMany, 0, s>>>(
+          mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, it, chk, check,
+          m.tflag_l[l], MgXr{}, nullptr, sw, nullptr);
+    });
   }
 }
 
-bool mg_tail_coarse(const MgHost& m) {
-  return !m.per_scene && m.lc >= 2 && m.ticket != nullptr && m.coarse_tail;
+int mg_stage_words(int nl, const int* nx, const int* ny, size_t lds_limit, bool scene) {
+  int words = 0, slots = 0;
+  for (int l = 0; l < nl; ++l) {
+    words += (nx[l] + 2) * (ny[l] + 3);
+    if (l > 0) slots += (nx[l] * ny[l] + 63) & ~63;
+  }
+  if (slots > (scene ? kSceneKB : kStageKB) * kCoarseThreads ||
+      2 * (size_t)words * sizeof(float) > lds_limit) return 0;
+  return words;
+}
+
+bool mg_has_cycle(const MgHost& m) { return m.cyc.nl > 0; }
+
+int mg_cycle_level(const MgHost& m) {
+  int l = 1;
+  while (l < m.lc && mg_up_blocks(m.nx[l], m.ny[l]) > kCycleTiles) ++l;
+  return l;
+}
+
+// The cycle's levels, task order and words (the word arrays are allocated here through
+// alloc(bytes), which returns zeroed device memory or null).
+bool mg_cycle_prepare(MgHost& m, int n_stages, const std::function<void*(size_t)>& alloc) {
+  MgCycleArgs& a = m.cyc;
+  a.nl = std::max(0, m.lc - m.l1);
+  if (a.nl == 0) return true;
+  unsigned task = 1;  // 0: the stop test
+  auto words = [&](int l) {
+    return (unsigned long long*)alloc((size_t)m.nx[l] * m.ny[l] * sizeof(unsigned long long));
+  };
+  bool ok = true;
+  for (int k = 0; k <= a.nl; ++k) {
+    const int l = m.l1 + k;
+    MgCycleLevel& v = a.lv[k];
+    v.nx = m.nx[l];
+    v.ny = m.ny[l];
+    v.tiles_x = (v.nx + 31) / 32;
+    v.inf = m.inf[l];
+    v.tflag = m.tflag_l[l];
+    v.r = m.rl[l];
+    v.xo = m.xo[l];
+    if (k > 0) {
+      ok &= (v.tr = words(l)) != nullptr;
+      ok &= (v.te = words(l)) != nullptr;
+    }
+    if (k < a.nl) {
+      ok &= (v.ts = words(l)) != nullptr;
+      v.down0 = task;
+      task += (unsigned)mg_up_blocks(v.nx, v.ny);
+    }
+  }
+  a.coarse0 = task;
+  a.up0 = task += (unsigned)n_stages;
+  for (int k = a.nl - 1; k >= 0; --k) {
+    a.lv[k].up0 = task;
+    task += (unsigned)mg_up_blocks(a.lv[k].nx, a.lv[k].ny);
+  }
+  a.n_tasks = task;
+  ok &= (a.ticket = (unsigned long long*)alloc(sizeof(unsigned long long))) != nullptr;
+  ok &= (a.flag = (unsigned*)alloc(kFlags * kHintPitch * sizeof(unsigned))) != nullptr;
+  ok &= (a.hint = (unsigned*)alloc((size_t)task * kHintPitch * sizeof(unsigned))) != nullptr;
+  return ok;
+}
+
+void launch_mg_cycle(hipStream_t s, const MgHost& m, int it, int max_iter, double tol,
+                     CgScalars* sc, const SceneCoarseArgs* scenes) {
+  const MgCheck chk = mg_check_args(m, it, max_iter, tol, sc);
+  const int check = m.fused && m.l1 == 1 ? 1 : 0;
+  const MgSweeps sw = mg_sweeps(m);
+  with_sweeps(m, [&](auto ns) {
+    constexpr int S = decltype(ns)::value;
+    using Dn = Strip<34 + 2 * S, kCycNT>;
+    using Up = Strip<32 + 2 * S, kCycNT>;
+    constexpr int WU = UpFrame<S>::WC;
+    constexpr size_t dn = 2 * Dn::N * sizeof(float) + kDownWC * kDownWC;
+    constexpr size_t up = (2 * Up::N + WU * WU) * sizeof(float) + WU * WU;
+    const size_t lds = std::max(std::max(dn, up), m.coarse_lds);
+    if (scenes)
+      k_mg_cycle<S, true><<<m.cyc.n_tasks, kCycNT, lds, s>>>(m.cyc, chk, it, check, sw, m.coarse,
+                                                             *scenes);
+    else
+      k_mg_cycle<S, false><<<m.cyc.n_tasks, kCycNT, lds, s>>>(m.cyc, chk, it, check, sw, m.coarse,
+                                                              SceneCoarseArgs{});
+  });
 }
 
 void launch_mg_coarse(hipStream_t s, const MgHost& m, int it, int max_iter, double tol,
@@ -2799,24 +3572,12 @@ void launch_mg_up(hipStream_t s, const MgHost& m, int l, int it, CgScalars* sc) 
   else if (l == 0)
     go0(std::integral_constant<int, kT>{});
   else {
-    auto go = [&](auto ns) {
+    with_sweeps(m, [&](auto ns) {
       constexpr int S = decltype(ns)::value;
-      if (few_tiles(blocks))
-        k_mg_up<false, kTileFew, S><<<blocks, kTileFew, 0, s>>>(
-            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
-            m.tflag_l[l], mg_sweeps(m), nullptr);
-      else
-        k_mg_up<false, kTileMany, S><<<blocks, kTileMany, 0, s>>>(
-            mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
-            m.tflag_l[l], mg_sweeps(m), nullptr);
-    };
-    switch (m.level_sweeps) {
-      case 3: go(std::integral_constant<int, 3>{}); break;
-      case 4: go(std::integral_constant<int, 4>{}); break;
-      case 5: go(std::integral_constant<int, 5>{}); break;
-      case 6: go(std::integral_constant<int, 6>{}); break;
-      default: go(std::integral_constant<int, 2>{}); break;
-    }
+      k_mg_up<false, kTileMany, S><<<blocks, kTileMany, 0, s>>>(
+          mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
+          m.tflag_l[l], mg_sweeps(m), nullptr);
+    });
   }
 }
 

@@ -60,38 +60,12 @@ constexpr int kPcgThreads = 512;
 constexpr unsigned kSpinLimit = 1u << 22;  // seconds of waiting: treated as a fault
 constexpr int kSlotWords = 4;              // 64-bit words per block and sum: 2 doubles
 
-// DPP move of a double; lanes without a source take 0.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_f64(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
 // Sum over the first 8 lanes of each 16-lane row, in lane 7 of the row.
 __device__ __forceinline__ double row_sum8(double v) {
   v += dpp_f64<0x111, 0xF>(v);  // row_shr:1, 2, 4
   v += dpp_f64<0x112, 0xF>(v);
   v += dpp_f64<0x114, 0xF>(v);
   return v;
-}
-// Sums over the wave, in lane 63, the values' steps interleaved (register moves only: a
-// shuffle tree of doubles costs 12 LDS-latency exchanges).
-template <int CTRL, int ROWS, int NV>
-__device__ __forceinline__ void dpp_step(double (&v)[NV]) {
-  double t[NV];
-#pragma unroll
-  for (int q = 0; q < NV; ++q) t[q] = dpp_f64<CTRL, ROWS>(v[q]);
-#pragma unroll
-  for (int q = 0; q < NV; ++q) v[q] += t[q];
-}
-template <int NV>
-__device__ __forceinline__ void wave_sums(double (&v)[NV]) {
-  dpp_step<0x111, 0xF>(v);
-  dpp_step<0x112, 0xF>(v);
-  dpp_step<0x114, 0xF>(v);
-  dpp_step<0x118, 0xF>(v);
-  dpp_step<0x142, 0xA>(v);  // row_bcast:15 into rows 1 and 3
-  dpp_step<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
 }
 // Lane `from`'s value, in every lane.
 __device__ __forceinline__ double lane_value(double v, int from) {

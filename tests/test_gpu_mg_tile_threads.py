@@ -1,6 +1,5 @@
-"""The multigrid tile levels below level 0 on either side of the line at which a level's
-tile count changes the threads per tile (256 tiles: 1024 threads; 257: 512), and where
-level 1 is larger than 256 tiles in both directions, against the FP64 oracle."""
+"""Multigrid hierarchies whose level 1 has 256, 257 and more tiles: levels with launches of
+their own above those that share one, against the FP64 oracle."""
 from __future__ import annotations
 
 import pytest
