@@ -294,7 +294,7 @@ class Domain:
 
     def particles(self) -> np.ndarray:
         n = self.num_particles()
-        out = np.zeros((n, 4), dtype=np.float32)
+        out = np.empty((n, 4), dtype=np.float32)
         self._chk(self._L.fsg_get_particles(self._h, out.ctypes.data, n), "fsg_get_particles")
         return out
 
@@ -308,8 +308,8 @@ class Domain:
                   "fsg_set_velocity")
 
     def velocity(self, which=VEL_FRONT):
-        u = np.zeros((self.ny, self.nx), np.float32)
-        v = np.zeros((self.ny, self.nx), np.float32)
+        u = np.empty((self.ny, self.nx), np.float32)
+        v = np.empty((self.ny, self.nx), np.float32)
         self._chk(self._L.fsg_get_velocity(self._h, which, u.ctypes.data, v.ctypes.data),
                   "fsg_get_velocity")
         return u, v
@@ -322,7 +322,7 @@ class Domain:
         self._chk(self._L.fsg_set_labels(self._h, a.ctypes.data), "fsg_set_labels")
 
     def labels(self) -> np.ndarray:
-        a = np.zeros((self.ny, self.nx), np.uint8)
+        a = np.empty((self.ny, self.nx), np.uint8)
         self._chk(self._L.fsg_get_labels(self._h, a.ctypes.data), "fsg_get_labels")
         return a
 
@@ -353,7 +353,7 @@ class Domain:
 
     # -- inspection -----------------------------------------------------------
     def _grid(self, fn, dtype):
-        a = np.zeros((self.ny, self.nx), dtype)
+        a = np.empty((self.ny, self.nx), dtype)
         self._chk(getattr(self._L, fn)(self._h, a.ctypes.data), fn)
         return a
 
@@ -367,22 +367,22 @@ class Domain:
         return self._grid("fsg_get_fluid_indices", np.int32)
 
     def valid_masks(self):
-        mu = np.zeros((self.ny, self.nx), np.uint8)
-        mv = np.zeros((self.ny, self.nx), np.uint8)
+        mu = np.empty((self.ny, self.nx), np.uint8)
+        mv = np.empty((self.ny, self.nx), np.uint8)
         self._chk(self._L.fsg_get_valid_masks(self._h, mu.ctypes.data, mv.ctypes.data),
                   "fsg_get_valid_masks")
         return mu, mv
 
     def ext_info(self):
-        iu = np.zeros((self.ny, self.nx), np.uint8)
-        iv = np.zeros((self.ny, self.nx), np.uint8)
+        iu = np.empty((self.ny, self.nx), np.uint8)
+        iv = np.empty((self.ny, self.nx), np.uint8)
         self._chk(self._L.fsg_get_ext_info(self._h, iu.ctypes.data, iv.ctypes.data),
                   "fsg_get_ext_info")
         return iu, iv
 
     def reject_flags(self):
         n = self.num_particles()
-        a = np.zeros(n, np.uint8)
+        a = np.empty(n, np.uint8)
         self._chk(self._L.fsg_get_reject_flags(self._h, a.ctypes.data), "fsg_get_reject_flags")
         return a
 
@@ -519,9 +519,9 @@ class Domain:
 
     def adjoint_get(self):
         n = self.num_particles()
-        pbar = np.zeros((n, 4), np.float32)
-        bu = np.zeros((self.ny, self.nx), np.float32)
-        bv = np.zeros((self.ny, self.nx), np.float32)
+        pbar = np.empty((n, 4), np.float32)
+        bu = np.empty((self.ny, self.nx), np.float32)
+        bv = np.empty((self.ny, self.nx), np.float32)
         self._chk(self._L.fsg_adjoint_get(self._h, pbar.ctypes.data if n else None,
                                           bu.ctypes.data, bv.ctypes.data), "fsg_adjoint_get")
         return pbar, bu, bv
@@ -536,8 +536,8 @@ class Domain:
             "fsg_adjoint_set_front")
 
     def adjoint_get_front(self):
-        fu = np.zeros((self.ny, self.nx), np.float32)
-        fv = np.zeros((self.ny, self.nx), np.float32)
+        fu = np.empty((self.ny, self.nx), np.float32)
+        fv = np.empty((self.ny, self.nx), np.float32)
         self._chk(self._L.fsg_adjoint_get_front(self._h, fu.ctypes.data, fv.ctypes.data),
                   "fsg_adjoint_get_front")
         return fu, fv
@@ -552,7 +552,7 @@ class Domain:
         return it.value
 
     def density(self) -> np.ndarray:
-        rho = np.zeros((self.ny, self.nx), np.float32)
+        rho = np.empty((self.ny, self.nx), np.float32)
         self._chk(self._L.fsg_particle_density(self._h, rho.ctypes.data), "fsg_particle_density")
         return rho
 
@@ -624,7 +624,7 @@ class Batch(Domain):
     def scene_particles(self, s):
         n = C.c_int64()
         self._chk(self._L.fsg_batch_num_particles(self._h, s, C.byref(n)), "num_particles")
-        out = np.zeros((n.value, 4), np.float32)
+        out = np.empty((n.value, 4), np.float32)
         if n.value:
             self._chk(self._L.fsg_batch_get_particles(self._h, s, out.ctypes.data, n.value),
                       "fsg_batch_get_particles")
@@ -632,15 +632,15 @@ class Batch(Domain):
 
     def scene_velocity(self, s, which=VEL_FRONT):
         nx, ny = self.sizes[s]
-        u = np.zeros((ny, nx), np.float32)
-        v = np.zeros((ny, nx), np.float32)
+        u = np.empty((ny, nx), np.float32)
+        v = np.empty((ny, nx), np.float32)
         self._chk(self._L.fsg_batch_get_velocity(self._h, s, which, u.ctypes.data, v.ctypes.data),
                   "fsg_batch_get_velocity")
         return u, v
 
     def scene_labels(self, s):
         nx, ny = self.sizes[s]
-        lab = np.zeros((ny, nx), np.uint8)
+        lab = np.empty((ny, nx), np.uint8)
         self._chk(self._L.fsg_batch_get_labels(self._h, s, lab.ctypes.data),
                   "fsg_batch_get_labels")
         return lab
