@@ -35,6 +35,19 @@ __device__ __forceinline__ float div_y(float a, const Geom& g) {
   return g.pow2_y ? a * g.inv_dy : a / g.dy;
 }
 
+// (row[i], row[min(i + 1, nx - 1)]) for 0 <= i < nx, nx >= 2, in one 8-byte load (of 4-byte
+// alignment): a wave whose particles lie far apart spends a cycle per lane and load
+// instruction on addresses, which is what bounds the particle kernels' samples.
+struct FloatPair {
+  float x, y;
+};
+__device__ __forceinline__ FloatPair load_pair(const float* __restrict__ row, int i, int nx) {
+  const int a = i < nx - 1 ? i : nx - 2;
+  FloatPair p = *reinterpret_cast<const FloatPair*>(row + a);
+  if (i != a) p.x = p.y;
+  return p;
+}
+
 // Grid<T>::valueInterpolated (include/Grid.h:117-144) on a row-major grid:
 // truncating casts, fraction before clamping, i+1 clamped after i, x then y lerp.
 // xs, ys are the coordinates already divided by the spacing; nx, ny bound the
@@ -48,14 +61,11 @@ __device__ __forceinline__ float interp_pitched(const float* __restrict__ g, int
   const float fj = ys - (float)j;
   i = clampi(i, 0, nx - 1);
   j = clampi(j, 0, ny - 1);
-  const int i1 = clampi(i + 1, 0, nx - 1);
   const int j1 = clampi(j + 1, 0, ny - 1);
-  const float v00 = g[i + j * pitch];
-  const float v10 = g[i1 + j * pitch];
-  const float v01 = g[i + j1 * pitch];
-  const float v11 = g[i1 + j1 * pitch];
-  const float v0 = (1.0f - fi) * v00 + fi * v10;
-  const float v1 = (1.0f - fi) * v01 + fi * v11;
+  const FloatPair r0 = load_pair(g + j * pitch, i, nx);
+  const FloatPair r1 = load_pair(g + j1 * pitch, i, nx);
+  const float v0 = (1.0f - fi) * r0.x + fi * r0.y;
+  const float v1 = (1.0f - fi) * r1.x + fi * r1.y;
   return (1.0f - fj) * v0 + fj * v1;
 }
 

@@ -27,13 +27,13 @@ __device__ __forceinline__ int64_t gtid() {
   return (int64_t)blockIdx.x * kAT + threadIdx.x;
 }
 
-// d/dfi and d/dfj of Grid::valueInterpolated's bilinear form at corners s
+// d/dfi and d/dfj of Grid::valueInterpolated's bilinear form at corners s (of
+// interp_corners: i1 is i + 1 within the grid)
 __device__ __forceinline__ void interp_grad(const float* __restrict__ g, int nx,
                                             const SplatCorners& s, float& dfi, float& dfj) {
-  const float v00 = g[s.i + s.j * nx], v10 = g[s.i1 + s.j * nx];
-  const float v01 = g[s.i + s.j1 * nx], v11 = g[s.i1 + s.j1 * nx];
-  dfi = (1.0f - s.fj) * (v10 - v00) + s.fj * (v11 - v01);
-  dfj = ((1.0f - s.fi) * v01 + s.fi * v11) - ((1.0f - s.fi) * v00 + s.fi * v10);
+  const FloatPair r0 = load_pair(g + s.j * nx, s.i, nx), r1 = load_pair(g + s.j1 * nx, s.i, nx);
+  dfi = (1.0f - s.fj) * (r0.y - r0.x) + s.fj * (r1.y - r1.x);
+  dfj = ((1.0f - s.fi) * r1.x + s.fi * r1.y) - ((1.0f - s.fi) * r0.x + s.fi * r0.y);
 }
 
 // transpose of the bilinear sample: value * weights added to the 4 corners

