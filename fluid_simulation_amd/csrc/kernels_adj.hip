@@ -59,6 +59,39 @@ __device__ __forceinline__ float inv_or_div(float a, float d, int pow2, float in
   return pow2 ? a * inv : a / d;
 }
 
+// The smallest rectangle of cells around the live lanes' (i, j) .. (i1, j1), in every thread
+// of the block (i1 < i0: no lane is live).
+struct Box {
+  int i0, j0, i1, j1;
+};
+__device__ __forceinline__ Box block_box(bool live, int i, int j, int i1, int j1) {
+  Box b{live ? i : INT_MAX, live ? j : INT_MAX, live ? i1 : INT_MIN, live ? j1 : INT_MIN};
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    b.i0 = min(b.i0, __shfl_xor(b.i0, off, 64));
+    b.j0 = min(b.j0, __shfl_xor(b.j0, off, 64));
+    b.i1 = max(b.i1, __shfl_xor(b.i1, off, 64));
+    b.j1 = max(b.j1, __shfl_xor(b.j1, off, 64));
+  }
+  __shared__ int s_box[4][kAT / 64];
+  const int wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    s_box[0][wave] = b.i0;
+    s_box[1][wave] = b.j0;
+    s_box[2][wave] = b.i1;
+    s_box[3][wave] = b.j1;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kAT / 64; ++w) {
+    b.i0 = min(b.i0, s_box[0][w]);
+    b.j0 = min(b.j0, s_box[1][w]);
+    b.i1 = max(b.i1, s_box[2][w]);
+    b.j1 = max(b.j1, s_box[3][w]);
+  }
+  return b;
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------- G2P + advect
@@ -96,32 +129,10 @@ __global__ void __launch_bounds__(kAT) k_adj_g2p(Geom g, const float4* __restric
   // the splat of vbx into su and vby into sv: summed in an LDS copy of the block's
   // footprint when it fits (neighbouring particles share cells), then one atomic per
   // touched value; otherwise straight to the grids
-  int i0 = live ? min(cu.i, cv.i) : INT_MAX, j0 = live ? min(cu.j, cv.j) : INT_MAX;
-  int i1 = live ? max(cu.i1, cv.i1) : INT_MIN, j1 = live ? max(cu.j1, cv.j1) : INT_MIN;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    i0 = min(i0, __shfl_xor(i0, off, 64));
-    j0 = min(j0, __shfl_xor(j0, off, 64));
-    i1 = max(i1, __shfl_xor(i1, off, 64));
-    j1 = max(j1, __shfl_xor(j1, off, 64));
-  }
-  __shared__ int s_box[4][kAT / 64];
   __shared__ float2 s_tile[kAdjSplatTile];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) {
-    s_box[0][wave] = i0;
-    s_box[1][wave] = j0;
-    s_box[2][wave] = i1;
-    s_box[3][wave] = j1;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int w = 0; w < kAT / 64; ++w) {
-    i0 = min(i0, s_box[0][w]);
-    j0 = min(j0, s_box[1][w]);
-    i1 = max(i1, s_box[2][w]);
-    j1 = max(j1, s_box[3][w]);
-  }
+  const Box box = block_box(live, min(cu.i, cv.i), min(cu.j, cv.j), max(cu.i1, cv.i1),
+                            max(cu.j1, cv.j1));
+  const int i0 = box.i0, j0 = box.j0, i1 = box.i1, j1 = box.j1;
   const int bw = i1 - i0 + 1, bh = j1 - j0 + 1;
   const bool tiled = bw > 0 && bh > 0 && (int64_t)bw * bh <= kAdjSplatTile;
   if (!tiled) {
@@ -435,25 +446,54 @@ __global__ void __launch_bounds__(kAT) k_adj_p2g(Geom g, const float4* __restric
 // y / dy) with Grid::addToValueInterpolated's weights.
 // FX: the terms are added as 64-bit fixed-point integers (fx_term) into rho_fx, so
 // the density does not depend on the order of the atomics (fsg_params.deterministic).
+// The terms go to an LDS copy of the block's footprint where that fits (as the splat's; four
+// terms in [0, 1] per particle, so 256 particles' sums are far from the fixed point's range),
+// then one atomic per touched cell: 1,040,000 particles near their storage order on 512^2
+// cells 177 -> 18.6 us, fixed-point sums.
+constexpr int kDensityTile = 2048;
 template <bool FX>
 __global__ void __launch_bounds__(kAT) k_density(Geom g, const float4* __restrict__ pt,
                                                  int64_t np, float* __restrict__ rho,
                                                  unsigned long long* __restrict__ rho_fx) {
   const int64_t p = gtid();
-  if (p >= np) return;
-  const float4 q = pt[p];
+  const bool live = p < np;
+  const float4 q = live ? pt[p] : make_float4(0.f, 0.f, 0.f, 0.f);
   const SplatCorners s = splat_corners(div_x(q.x, g), div_y(q.y, g), g.nx, g.ny);
-  const float a0 = (1.0f - s.fj), a1 = s.fj;
-  auto add = [&](int c, float t) {
+  __shared__ unsigned long long s_tile[kDensityTile];
+  const Box box = block_box(live, s.i, s.j, s.i1, s.j1);
+  const int bw = box.i1 - box.i0 + 1, bh = box.j1 - box.j0 + 1;
+  bool tiled = bw > 0 && bh > 0 && (int64_t)bw * bh <= kDensityTile;
+  // a position far outside the grid or not a number has weights the fixed point cannot hold:
+  // the float sums take them as they are (block-uniform)
+  if (!FX && tiled)
+    tiled = !__syncthreads_or(live && !(fabsf(s.fi) <= 1.0f && fabsf(s.fj) <= 1.0f));
+  if (!tiled) {
+    if (live)
+      splat_terms2(s, 1.0f, [&](int i, int j, float t) {
+        if (FX)
+          atomicAdd(rho_fx + i + j * g.nx, (unsigned long long)fx_term(t));
+        else
+          unsafeAtomicAdd(&rho[i + j * g.nx], t);
+      });
+    return;
+  }
+  const int area = bw * bh;
+  for (int c = threadIdx.x; c < area; c += kAT) s_tile[c] = 0ull;
+  __syncthreads();
+  if (live)
+    splat_terms2(s, 1.0f, [&](int i, int j, float t) {
+      atomicAdd(s_tile + (i - box.i0) + (j - box.j0) * bw, (unsigned long long)fx_term(t));
+    });
+  __syncthreads();
+  for (int c = threadIdx.x; c < area; c += kAT) {
+    const unsigned long long v = s_tile[c];
+    if (v == 0ull) continue;
+    const int cell = (box.i0 + c % bw) + (box.j0 + c / bw) * g.nx;
     if (FX)
-      atomicAdd(rho_fx + c, (unsigned long long)fx_term(t));
+      atomicAdd(rho_fx + cell, v);
     else
-      unsafeAtomicAdd(&rho[c], t);
-  };
-  add(s.i + s.j * g.nx, (1.0f - s.fi) * a0);
-  add(s.i1 + s.j * g.nx, s.fi * a0);
-  add(s.i + s.j1 * g.nx, (1.0f - s.fi) * a1);
-  add(s.i1 + s.j1 * g.nx, s.fi * a1);
+      unsafeAtomicAdd(&rho[cell], fx_value((long long)v));
+  }
 }
 
 // pbar = (d rho / d X)^T rhobar, zero velocity adjoints.
