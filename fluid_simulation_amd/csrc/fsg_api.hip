@@ -2175,13 +2175,14 @@ int fsg_checkpoint_save(fsg_domain* h, int32_t slot) {
     c.cap = h->np;
   }
   c.np = h->np;
-  if (h->np > 0)
-    HIPCHK(h, hipMemcpyAsync(c.pt, h->pt, (size_t)h->np * sizeof(float4),
-                             hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(c.u[0], UF(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(c.v[0], VF(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(c.u[1], UB(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(c.v[1], VB(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
+  fsg::CopyList list;
+  list.add(c.pt, h->pt, h->np * (int64_t)sizeof(float4));
+  list.add(c.u[0], UF(h), (int64_t)C * 4);
+  list.add(c.v[0], VF(h), (int64_t)C * 4);
+  list.add(c.u[1], UB(h), (int64_t)C * 4);
+  list.add(c.v[1], VB(h), (int64_t)C * 4);
+  launch_copies(h->stream, list);
+  HIPCHK(h, hipGetLastError());
   return FSG_OK;  // stream-ordered: later work on the handle sees the copy
 }
 
@@ -2192,13 +2193,14 @@ int fsg_checkpoint_load(fsg_domain* h, int32_t slot) {
   const size_t C = ncell(h);
   if (int rc = reserve_particles(h, c.np)) return rc;
   h->np = c.np;
-  if (c.np > 0)
-    HIPCHK(h, hipMemcpyAsync(h->pt, c.pt, (size_t)c.np * sizeof(float4),
-                             hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(UF(h), c.u[0], C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(VF(h), c.v[0], C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(UB(h), c.u[1], C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(VB(h), c.v[1], C * 4, hipMemcpyDeviceToDevice, h->stream));
+  fsg::CopyList list;
+  list.add(h->pt, c.pt, c.np * (int64_t)sizeof(float4));
+  list.add(UF(h), c.u[0], (int64_t)C * 4);
+  list.add(VF(h), c.v[0], (int64_t)C * 4);
+  list.add(UB(h), c.u[1], (int64_t)C * 4);
+  list.add(VB(h), c.v[1], (int64_t)C * 4);
+  launch_copies(h->stream, list);
+  HIPCHK(h, hipGetLastError());
   return FSG_OK;  // stream-ordered
 }
 
@@ -2498,8 +2500,10 @@ static int adjoint_step_sl(fsg_domain* h, float dt) {
   AdjState& a = h->adj;
   const int64_t np = h->np;
   const size_t C = ncell(h);
-  HIPCHK(h, hipMemcpyAsync(a.f0u, UF(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(a.f0v, VF(h), C * 4, hipMemcpyDeviceToDevice, h->stream));
+  fsg::CopyList front;
+  front.add(a.f0u, UF(h), (int64_t)C * 4);
+  front.add(a.f0v, VF(h), (int64_t)C * 4);
+  launch_copies(h->stream, front);
   a.taping = true;
   int rc = step_semi_lagrangian(h, dt);
   a.taping = false;
@@ -2509,8 +2513,10 @@ static int adjoint_step_sl(fsg_domain* h, float dt) {
                 "fsg_adjoint_step: no LIQUID cell (the no-fluid step has no adjoint here)");
   const fsg_stats fwd = h->host_stats;
   const float dt_over_density = dt / h->density;
-  HIPCHK(h, hipMemcpyAsync(a.su, a.fu, C * 4, hipMemcpyDeviceToDevice, h->stream));
-  HIPCHK(h, hipMemcpyAsync(a.sv, a.fv, C * 4, hipMemcpyDeviceToDevice, h->stream));
+  fsg::CopyList adj;
+  adj.add(a.su, a.fu, (int64_t)C * 4);
+  adj.add(a.sv, a.fv, (int64_t)C * 4);
+  launch_copies(h->stream, adj);
   timed(h, "adj_advect_grid", [&] {
     launch_adj_advect_grid(h->stream, h->g, a.x0, np, UF(h), VF(h), h->prm.integrator, dt, a.pbar,
                            a.su, a.sv);
@@ -2560,9 +2566,9 @@ int fsg_adjoint_step(fsg_domain* h, int32_t scheme, float dt) {
   AdjState& a = h->adj;
   const int64_t np = h->np;
   const size_t C = ncell(h);
-  if (np > 0)
-    HIPCHK(h, hipMemcpyAsync(a.x0, h->pt, (size_t)np * sizeof(float4), hipMemcpyDeviceToDevice,
-                             h->stream));
+  fsg::CopyList start;
+  start.add(a.x0, h->pt, np * (int64_t)sizeof(float4));
+  launch_copies(h->stream, start);
   if (scheme == FSG_SCHEME_SEMI_LAGRANGIAN) return adjoint_step_sl(h, dt);
   a.taping = true;
   int rc = step_flip_family(h, scheme, dt);

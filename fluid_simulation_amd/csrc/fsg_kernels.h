@@ -58,6 +58,21 @@ struct BatchTables {
 enum { FU_P2G = 1, FU_PREV = 2, FU_GRAVITY = 4, FU_DIRICHLET = 8, FU_EXTINIT = 16,
        FU_CLOSED = 32 };
 
+// Copies between device arrays in one launch: 16-byte aligned, whole 4-byte words.
+struct CopyList {
+  static constexpr int kMost = 6;
+  const void* src[kMost];
+  void* dst[kMost];
+  int64_t bytes[kMost];
+  int n = 0;
+  void add(void* d, const void* s, int64_t b) {
+    if (b <= 0) return;
+    src[n] = s;
+    dst[n] = d;
+    bytes[n++] = b;
+  }
+};
+void launch_copies(hipStream_t s, const CopyList& list);
 void launch_cell_init(hipStream_t s, const Geom& g, uint8_t* label, const uint8_t* solid,
                       float4* acc, int do_labels, int do_acc);
 // The cell set-up of a step: label (if set) := SOLID on the border and where solid is
