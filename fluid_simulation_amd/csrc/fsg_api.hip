@@ -97,6 +97,9 @@ struct BatchInfo {
   int la = 1;
   std::vector<fsg::SceneCoarse> coarse;
   fsg::SceneCoarse* d_coarse = nullptr;
+  int4* d_tscenes = nullptr;    // MgbArgs::tile_scenes
+  uint64_t* d_stage = nullptr;  // SceneCoarseArgs::table
+  int stage_stride = 0;
   uint8_t* d_sinf = nullptr;
   int stride = 0;
   // per-scene CG: 64 x 16 vector tiles inside the scenes, and the scalars (5 S doubles)
@@ -118,8 +121,9 @@ struct BatchInfo {
     a.rz = d_cg;
     a.pq = d_cg + 2 * S;
     a.rr = d_cg + 3 * S;
-    a.bb = d_cg + 4 * S;
+    a.bb = d_cg + 5 * S;
     a.vflag = d_vflag;
+    a.tile_scenes = d_tscenes;
     return a;
   }
   fsg::MgBatchScale scale() const {
@@ -707,6 +711,8 @@ fsg::SceneCoarseArgs scene_coarse_args(const fsg_domain* h) {
   a.omega2 = m.coarse.omega2;
   a.trunc = m.coarse.trunc;
   a.lds = m.coarse_lds;
+  a.table = b.d_stage;
+  a.table_stride = b.stage_stride;
   return a;
 }
 
@@ -752,14 +758,17 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   if (m.clk_span_on && !m.clk_span) alloc_clk_span(h);
   timed(h, "cg_mg_setup", [&] {
     fsg::MgBatchScale bs;
-    if (h->batch) bs = h->batch->scale();
+    if (h->batch) {
+      bs = h->batch->scale();
+      m.mgb = h->batch->cg_args(h->g.nx, h->g.ny);
+    }
     launch_mg_setup(h->stream, h->g, m, h->label, UF(h), VF(h), h->prm.project_mean,
                     h->prm.warm_start != 0 && !h->batch && !adj_rhs, h->sc,
                     h->batch ? &bs : nullptr, adj_rhs, adj_rhs ? nullptr : h->b,
                     adj_rhs ? nullptr : h->n_fluid);
     if (h->batch) {
       launch_mg_scene_setup(h->stream, scene_coarse_args(h));
-      launch_mgb_init(h->stream, h->batch->cg_args(h->g.nx, h->g.ny), h->batch->d_norm, m);
+      launch_mgb_flags(h->stream, m);
     }
   });
   const int max_iter = h->prm.cg_max_iter;
@@ -779,11 +788,11 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
                                           "cg_mg_up4", "cg_mg_up5", "cg_mg_up6", "cg_mg_up7+"};
   // one CG iteration: the V-cycle's kernels, the direction (and the x / residual
   // update where it is not fused into the next iteration's level-0 kernel).  Its head
-  // is its kernels up to and including the stop test (a batch's check kernel; level 0's
+  // is its kernels up to and including the stop test (level 0's
   // down kernel, or levels 0-1 in the fused form; the whole iteration where the
   // hierarchy has no tile level), its tail the rest: once the solve has stopped in
   // iteration q's head, the kernels after it return at once.
-  const int head_levels = h->batch ? 0 : m.fused ? 2 : 1;
+  const int head_levels = m.fused ? 2 : 1;
   const bool whole_head = !h->batch && m.lc < head_levels;
   // the levels with launches of their own; the others (cycle) share one, which in the
   // fused form runs the stop test if it begins with level 1
@@ -791,10 +800,6 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   const int own_levels = cycle ? m.l1 : m.lc;
   const bool cycle_head = m.fused && m.l1 == 1;
   auto enqueue_part = [&](int it, bool head) {
-    if (h->batch && head)
-      timed(h, "cg_mg_check", [&] {
-        launch_mgb_check(h->stream, h->batch->cg_args(h->g.nx, h->g.ny), it, max_iter, tol, h->sc);
-      });
     if (!whole_head)
       for (int l = 0; l < own_levels; ++l)
         if ((l < head_levels) == head)
@@ -818,8 +823,9 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
     for (int l = own_levels - 1; l >= 0; --l)
       timed(h, kUpNames[std::min(l, 7)], [&] { launch_mg_up(h->stream, m, l, it, h->sc); });
     if (h->batch) {
-      const fsg::MgbArgs ba = h->batch->cg_args(h->g.nx, h->g.ny);
-      timed(h, "cg_mg_rz", [&] { launch_mgb_vectors(h->stream, ba, m, it, h->sc, 0); });
+      const fsg::MgbArgs& ba = m.mgb;
+      if (!ba.tile_scenes)  // else with level 0's up kernel
+        timed(h, "cg_mg_rz", [&] { launch_mgb_vectors(h->stream, ba, m, it, h->sc, 0); });
       timed(h, "cg_mg_dir", [&] { launch_mgb_vectors(h->stream, ba, m, it, h->sc, 1); });
       timed(h, "cg_mg_xr", [&] { launch_mgb_vectors(h->stream, ba, m, it, h->sc, 2); });
     } else {
@@ -2000,6 +2006,9 @@ int fsg_batch_create(fsg_domain** out, int32_t n_scenes, const int32_t* nx, cons
     if (c.nx[c.nl - 1] * c.ny[c.nl - 1] > 64) return bail(FSG_E_INVALID, "scene hierarchy");
     c.total = (off + 3) & ~3;
     c.words = mg_stage_words(c.nl, c.nx, c.ny, kCoarseLdsLimit, true);
+    int cells = 0;  // every level from a wavefront on
+    for (int l = 0; l < c.nl; ++l) cells += (c.nx[l] * c.ny[l] + 63) & ~63;
+    b->stage_stride = std::max(b->stage_stride, cells);
     b->stride = std::max(b->stride, c.total);
     b->coarse.push_back(c);
   }
@@ -2010,6 +2019,7 @@ int fsg_batch_create(fsg_domain** out, int32_t n_scenes, const int32_t* nx, cons
   ok &= dalloc(h, &b->d_norm, (size_t)n_scenes) == hipSuccess;
   ok &= dalloc(h, &b->d_inv, (size_t)n_scenes) == hipSuccess;
   ok &= dalloc(h, &b->d_coarse, (size_t)n_scenes) == hipSuccess;
+  ok &= dalloc(h, &b->d_stage, (size_t)n_scenes * b->stage_stride) == hipSuccess;
   ok &= dalloc(h, &b->d_sinf, (size_t)n_scenes * b->stride) == hipSuccess;
   std::vector<int4> vtile;
   std::vector<int2> vend;
@@ -2020,9 +2030,23 @@ int fsg_batch_create(fsg_domain** out, int32_t n_scenes, const int32_t* nx, cons
         vend.push_back(make_int2(ox[s] + nx[s], oy[s] + ny[s]));
       }
   b->n_vtile = (int)vtile.size();
+  const int txs = (W + 31) / 32;
+  std::vector<int4> tscenes((size_t)txs * ((H + 31) / 32), make_int4(-1, -1, -1, -1));
+  bool at_most_four = true;
+  for (int s = 0; s < n_scenes; ++s)
+    for (int ty = oy[s] / 32; ty <= (oy[s] + ny[s] - 1) / 32; ++ty)
+      for (int tx = ox[s] / 32; tx <= (ox[s] + nx[s] - 1) / 32; ++tx) {
+        int4& t = tscenes[(size_t)tx + (size_t)ty * txs];
+        int* const slot = t.x < 0 ? &t.x : t.y < 0 ? &t.y : t.z < 0 ? &t.z : t.w < 0 ? &t.w : nullptr;
+        if (slot)
+          *slot = s;
+        else
+          at_most_four = false;
+      }
+  if (at_most_four) ok &= dalloc(h, &b->d_tscenes, tscenes.size()) == hipSuccess;
   ok &= dalloc(h, &b->d_vtile, vtile.size()) == hipSuccess;
   ok &= dalloc(h, &b->d_vend, vend.size()) == hipSuccess;
-  ok &= dalloc(h, &b->d_cg, (size_t)5 * n_scenes) == hipSuccess;
+  ok &= dalloc(h, &b->d_cg, (size_t)6 * n_scenes) == hipSuccess;
   ok &= dalloc(h, &b->d_vflag, vtile.size()) == hipSuccess;
   if (!ok) return bail(FSG_E_NOMEM, "");
   if (hipMemcpyAsync(b->d_scene, table.data(), sizeof(fsg::BatchScene) * n_scenes,
@@ -2037,6 +2061,9 @@ int fsg_batch_create(fsg_domain** out, int32_t n_scenes, const int32_t* nx, cons
                      hipMemcpyHostToDevice, h->stream) != hipSuccess ||
       hipMemcpyAsync(b->d_vend, vend.data(), sizeof(int2) * vend.size(),
                      hipMemcpyHostToDevice, h->stream) != hipSuccess ||
+      (b->d_tscenes &&
+       hipMemcpyAsync(b->d_tscenes, tscenes.data(), sizeof(int4) * tscenes.size(),
+                      hipMemcpyHostToDevice, h->stream) != hipSuccess) ||
       hipStreamSynchronize(h->stream) != hipSuccess)
     return bail(FSG_E_HIP, "");
   if ((rc = fsg_set_solid_mask(h, b->solid.data())) != FSG_OK) return bail(rc, "");

@@ -322,6 +322,8 @@ struct SceneCoarseArgs {
   float omega = 0.8f, omega2 = 0.8f;
   int trunc = 0;  // as MgCoarseArgs::trunc, on each scene's first level
   size_t lds = 0; // bytes of LDS per scene's stage
+  uint64_t* table = nullptr;  // the stages' words per cell, scene s's at s * table_stride
+  int table_stride = 0;
 };
 
 // Packed batch: per-scene CG scalars (one CG per scene in lock step).
@@ -332,13 +334,17 @@ struct MgbArgs {
   int n_tiles = 0, n_scenes = 0, W = 0, C = 0;  // C: cells of the packed grid
   double* rz = nullptr;  // [2][S] r.z by iteration parity
   double* pq = nullptr;  // [S]
-  double* rr = nullptr;  // [S]
+  double* rr = nullptr;  // [2][S] |r|^2 at the start of an iteration, by its parity
   double* bb = nullptr;  // [S]
   const uint8_t* vflag = nullptr;  // per tile: 1 if it holds an unknown (set each solve)
+  // per 32 x 32 tile of level 0: the scenes that it holds cells of, -1 for none; null where
+  // a tile holds more than four (tiny scenes)
+  const int4* tile_scenes = nullptr;
 };
 
 struct MgHost {
-  bool per_scene = false;  // a batch: stop test and CG scalars per scene (MgbArgs)
+  bool per_scene = false;  // a batch: stop test and CG scalars per scene (mgb)
+  MgbArgs mgb;
   unsigned long long* clk = nullptr;  // k_mg_coarse's own clock: ticks, launches
   bool clk_on = false;
   // level 0's down kernel clock: per recorded launch and block, (start, end) ticks
@@ -419,11 +425,9 @@ void launch_mg_setup(hipStream_t s, const Geom& g, const MgHost& m, const uint8_
                      CgScalars* sc, const MgBatchScale* batch = nullptr,
                      const double* adj_rhs = nullptr, float* rhs = nullptr,
                      int* n_fluid = nullptr);
-// a batch's per-scene CG: init after the setup; the stop test at the start of each
-// iteration; the vector kernels (which: 0 r.z, 1 direction, 2 x / r update)
-void launch_mgb_init(hipStream_t s, const MgbArgs& a, const double* norm, const MgHost& m);
-void launch_mgb_check(hipStream_t s, const MgbArgs& a, int it, int max_iter, double tol,
-                      CgScalars* sc);
+// a batch's per-scene CG: the vector tiles' flags after the setup; the vector kernels
+// (which: 0 r.z, 1 direction, 2 x / r update)
+void launch_mgb_flags(hipStream_t s, const MgHost& m);
 void launch_mgb_vectors(hipStream_t s, const MgbArgs& a, const MgHost& m, int it, CgScalars* sc,
                         int which);
 // removes the plain mean of the FP64 solution over the unknowns (adjoint solves)

@@ -379,7 +379,8 @@ __global__ void __launch_bounds__(kT) k_mg_setup1(int nx, int ny, int project_me
                                                    const double* __restrict__ part_liq,
                                                    int* __restrict__ n_fluid,
                                                    const uint8_t* __restrict__ tflag,
-                                                   int n_tiles) {
+                                                   int n_tiles, const int* __restrict__ sid,
+                                                   const double* __restrict__ factor) {
   __shared__ double sm[4];
   const int C = nx * ny;
   // the live level-0 tiles, where k_mg_setup0t set their flags (else k_mg_tile_flags
@@ -407,6 +408,10 @@ __global__ void __launch_bounds__(kT) k_mg_setup1(int nx, int ny, int project_me
   for (int c = blockIdx.x * kT + threadIdx.x; c < C; c += gridDim.x * kT, w.next()) {
     const uint8_t f = inf[c];
     double bv = b[c];
+    if (sid) {  // a batch: b'[c] *= factor[scene of c]
+      const int s = sid[c];
+      if (s >= 0) b[c] = bv *= factor[s];
+    }
     if (project_mean && is_act(f)) {
       bv -= mean;
       b[c] = bv;
@@ -443,34 +448,39 @@ __global__ void __launch_bounds__(kT) k_mg_setup1(int nx, int ny, int project_me
 }
 
 // Packed batch: |b'_s| over each scene's rectangle, one workgroup per scene (a
-// fixed summation order), and its reciprocal.
+// fixed summation order), its reciprocal, and the scene's |b_s|^2 (1 after the
+// normalisation, 0 for a scene without unknowns) and |r_s|^2 of x0 = 0.  A wavefront takes
+// rows, a lane columns, kNormRows rows' loads in flight: one at a time, with a division
+// for each index, 32 scenes of 64 to 190 cells a side took 14 us (set-up and the
+// normalisation, now folded into k_mg_setup1, together 75 -> 64 us).
+constexpr int kNormRows = 8;
 __global__ void __launch_bounds__(1024) k_mg_scene_norm(const double* __restrict__ b, int pitch,
                                                         const int4* __restrict__ rect,
                                                         double* __restrict__ norm,
-                                                        double* __restrict__ inv) {
+                                                        double* __restrict__ inv, MgbArgs a) {
   __shared__ double sm[16];
   const int4 r = rect[blockIdx.x];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double* const first = b + r.x + (int64_t)r.y * pitch;
   double v[1] = {0.0};
-  for (int q = threadIdx.x; q < r.z * r.w; q += 1024) {
-    const int i = q % r.z, j = q / r.z;
-    const double x = b[(r.x + i) + (int64_t)(r.y + j) * pitch];
-    v[0] += x * x;
-  }
+  for (int j0 = wave; j0 < r.w; j0 += 16 * kNormRows)
+    for (int i = lane; i < r.z; i += 64) {
+      double x[kNormRows];
+#pragma unroll
+      for (int k = 0; k < kNormRows; ++k) {
+        const int j = j0 + 16 * k;
+        const double t = first[i + (int64_t)(j < r.w ? j : j0) * pitch];
+        x[k] = j < r.w ? t : 0.0;
+      }
+#pragma unroll
+      for (int k = 0; k < kNormRows; ++k) v[0] += x[k] * x[k];
+    }
   block_sum<1, 1024>(v, sm);
   if (threadIdx.x == 0) {
     const double n = sqrt(v[0]);
     norm[blockIdx.x] = n;
     inv[blockIdx.x] = n > 0.0 ? 1.0 / n : 0.0;
-  }
-}
-
-// b'[c] *= factor[scene of c]
-__global__ void __launch_bounds__(kT) k_mg_scene_scale(int C, const int* __restrict__ sid,
-                                                        const double* __restrict__ factor,
-                                                        double* __restrict__ b) {
-  for (int c = blockIdx.x * kT + threadIdx.x; c < C; c += gridDim.x * kT) {
-    const int s = sid[c];
-    if (s >= 0) b[c] *= factor[s];
+    a.bb[blockIdx.x] = a.rr[blockIdx.x] = n > 0.0 ? 1.0 : 0.0;
   }
 }
 
@@ -839,13 +849,18 @@ struct MgCheck {
   int n_bb;
   double tol2;
   int max_iter;
-  int external;  // 1: the stop test ran in its own kernel (per-scene CG); read `done` only
+  // a batch (S scenes, a CG each): |r_s|^2 and |b_s|^2, and the sums that this iteration
+  // adds to, cleared with the test
+  int S;
+  const double *rr, *bb;
+  double *rr_next, *pq, *rz;
 };
 
 // Every block takes the same decision from the same partials.  `done` is read by one thread
 // and broadcast, since the writer may set it while other blocks start; either value of it
 // leads to that decision, so it need not be read device-coherent.
-template <int NT>
+// SCENES: the kernel may be a batch's (its code stays out of the others').
+template <int NT, bool SCENES = false>
 __device__ __forceinline__ bool mg_check(const MgCheck& k, int it, bool writer, double* sm) {
   __shared__ int s_done;
   // every load is issued before the first is needed (one memory round trip)
@@ -853,16 +868,40 @@ __device__ __forceinline__ bool mg_check(const MgCheck& k, int it, bool writer, 
   if (threadIdx.x == 0)
     done = __hip_atomic_load(&k.sc->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   double part[1] = {0.0}, bb = 0.0, thr = 0.0;
-  if (!k.external) {
-    bb = it == 0 ? thread_part<NT>(k.part_bb, k.n_bb) : k.sc->rhs_norm2;
-    thr = k.sc->threshold;
-    part[0] = thread_part<NT>(k.part_rr, k.n_rr);
+  if (SCENES && k.S > 0) {
+    // every scene below its own threshold
+    int ok = 1;
+    double worst = 0.0;
+    for (int q = threadIdx.x; q < k.S; q += NT) {
+      const double b = k.bb[q], r = k.rr[q];
+      double t = k.tol2 * b;
+      if (t < DBL_MIN) t = DBL_MIN;
+      if (b > 0.0) {
+        if (!(r < t)) ok = 0;
+        worst = fmax(worst, r / b);
+      }
+    }
+    if (threadIdx.x == 0) s_done = done;
+    const bool stop = __syncthreads_and(ok) != 0 || it >= k.max_iter;
+    if (s_done) return true;
+    if (writer) {
+      for (int q = threadIdx.x; q < k.S; q += NT) k.rr_next[q] = k.pq[q] = k.rz[q] = 0.0;
+      for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_down(worst, off, 64));
+      if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = worst;
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        for (int w = 1; w < NT / 64; ++w) worst = fmax(worst, sm[w]);
+        k.sc->iter = it;
+        k.sc->err = sqrt(worst);
+        if (stop) st_dev(&k.sc->done, 1);
+      }
+    }
+    return stop;
   }
+  bb = it == 0 ? thread_part<NT>(k.part_bb, k.n_bb) : k.sc->rhs_norm2;
+  thr = k.sc->threshold;
+  part[0] = thread_part<NT>(k.part_rr, k.n_rr);
   if (threadIdx.x == 0) s_done = done;
-  if (k.external) {
-    __syncthreads();
-    return s_done != 0;
-  }
   block_sum<1, NT>(part, sm);  // its barriers are behind s_done too
   if (s_done) return true;
   const double rr = part[0];
@@ -1234,7 +1273,7 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
     }
   }
   if (check) {
-    if (mg_check<NT>(chk, it, blockIdx.x == 0, sm)) {
+    if (mg_check<NT, L0 && !XR>(chk, it, blockIdx.x == 0, sm)) {
       clock.end();
       return;
     }
@@ -1361,16 +1400,26 @@ __global__ void __launch_bounds__(NT) k_mg_down(MgLevel f, MgLevel c, float omeg
   }
 }
 
+// A batch's level 0: the scenes (at most four) that a tile holds cells of, their rectangles,
+// and this iteration's r.z per scene, to which the tile's kernel adds (of null: one domain).
+struct MgTileScenes {
+  const int4* of = nullptr;  // -1: none
+  const int4* rect = nullptr;
+  double* rz = nullptr;
+};
+
 // Up: level l+1 -> level l.  A block owns 32 x 32 fine cells, on the window [-S, 32 + S)
 // in strips as k_mg_down: the corrected x = xs + P e there, then S post-sweeps, the last
 // one's tile written to xo.  In LDS: the coarse solution and info around the tile, and x
 // in two buffers.  S = 2 or 3 on level 0, 2 .. kMgMaxSweeps on the levels below (sweep k
 // uses w[k - 1]).  Level 0 also forms the partial of r.z (z = xo) for the next direction.
-template <bool L0, int NT, int S = 2>
+template <bool L0, int NT, int S = 2, bool SCENES = false>
 __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega, float omega2,
                                                const CgScalars* sc, double* __restrict__ part_rz,
                                                int it, const uint8_t* __restrict__ tflag,
-                                               MgSweeps sw, const int* __restrict__ tmap) {
+                                               MgSweeps sw, const int* __restrict__ tmap,
+                                               MgTileScenes scenes) {
+  static_assert(!SCENES || L0, "the scenes' sums belong to level 0");
   static_assert(S >= 2 && S <= kMgMaxSweeps && (!L0 || S <= 3),
                 "level 0 takes two or three sweeps; smaller levels 2 .. kMgMaxSweeps");
   constexpr int W = 32 + 2 * S;
@@ -1379,7 +1428,7 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
   constexpr int WC = UpFrame<S>::WC, CO = UpFrame<S>::CO;
   __shared__ float s_x[2][St::N], s_e[WC * WC];
   __shared__ uint8_t s_cinf[WC * WC];
-  __shared__ double sm[NT / 64];
+  __shared__ double sm[(SCENES ? 4 : 1) * (NT / 64)];
   float wk[kMgMaxSweeps];
   sweep_weights<S>(sw, omega, omega2, wk);
   const int tiles_x = (f.nx + 31) >> 5;
@@ -1450,7 +1499,34 @@ __global__ void __launch_bounds__(NT) k_mg_up(MgLevel f, MgLevel c, float omega,
       f.xo[ts.cell[q]] = v;
       if (L0) rz += (double)rv[q] * (double)v;
     }
-  if (L0) write_part<NT>(rz, part_rz, sm);
+  if constexpr (L0 && !SCENES) write_part<NT>(rz, part_rz, sm);
+  if constexpr (SCENES) {
+    // a batch: r.z of each scene that the tile holds cells of (mostly one)
+    const int4 o = scenes.of[tile];
+    double v[4] = {rz, 0.0, 0.0, 0.0};
+    if (o.y >= 0) {
+      v[0] = 0.0;
+      const int id[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (id[k] < 0) break;
+        const int4 rect = scenes.rect[id[k]];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const int i = ts.gi - rect.x, j = ts.gj + q - rect.y;
+          if (ts.own[q] && i >= 0 && i < rect.z && j >= 0 && j < rect.w)
+            v[k] += (double)rv[q] * (double)(is_act(fv[q]) ? x[q] : 0.f);
+        }
+      }
+    }
+    block_sum<4, NT>(v, sm);
+    if (threadIdx.x == 0) {
+      if (v[0] != 0.0) unsafeAtomicAdd(scenes.rz + o.x, v[0]);
+      if (o.y >= 0 && v[1] != 0.0) unsafeAtomicAdd(scenes.rz + o.y, v[1]);
+      if (o.z >= 0 && v[2] != 0.0) unsafeAtomicAdd(scenes.rz + o.z, v[2]);
+      if (o.w >= 0 && v[3] != 0.0) unsafeAtomicAdd(scenes.rz + o.w, v[3]);
+    }
+  }
 }
 
 // The levels lc .. nlev-1 (each <= 1024 cells) in one workgroup, all in LDS: the
@@ -1725,6 +1801,86 @@ struct StageCell {
   int epos = 0, ebits = 0;
 };
 
+// What a thread keeps of a cell besides its values: pos, epos and ebits, the first cell of the
+// restriction in LDS, the stencil's n (0: no unknown), and which of the eight neighbours are
+// walls (row by row).
+struct StageConst {
+  int pos = 0, epos = 0, rpos = 0, n = 0, ebits = 0, walls = 0;
+};
+// Of cell q of level l; po, fpo: the LDS offsets of level l and of the level above it.
+template <class Lx, class Ly, class Lo>
+__device__ __forceinline__ StageConst stage_const(int nl, Lx&& lx, Ly&& ly, Lo&& lo,
+                                                  const uint8_t* inf, int l, int q, int po,
+                                                  int fpo) {
+  StageConst s;
+  const int nx = lx(l), ny = ly(l), o = lo(l);
+  const bool in = q < nx * ny;
+  int i, j;
+  small_divmod(in ? q : 0, nx, 1.0f / (float)nx, i, j);
+  const uint8_t f = inf[o + (in ? q : 0)];
+  s.pos = po + (j + 1) * (nx + 2) + i + 1;
+  if (l + 1 < nl) {
+    const int cnx = lx(l + 1), cny = ly(l + 1), co = lo(l + 1);
+    const int I = i >> 1, J = j >> 1;
+    const int In = (i & 1) ? I + 1 : I - 1, Jn = (j & 1) ? J + 1 : J - 1;
+    const bool iok = In >= 0 && In < cnx, jok = Jn >= 0 && Jn < cny;
+    const int Ic = iok ? In : I, Jc = jok ? Jn : J;
+    const uint8_t fx = inf[co + Ic + J * cnx], fy = inf[co + I + Jc * cnx];
+    const uint8_t fxy = inf[co + Ic + Jc * cnx];
+    const bool bx = !iok || is_wall(fx), by = !jok || is_wall(fy);
+    const bool bxy = !(iok && jok) || is_wall(fxy);
+    s.epos = po + (nx + 2) * (ny + 3) + (J + 1) * (cnx + 2) + I + 1;
+    s.ebits = (i & 1) | ((j & 1) << 1) | (bx << 2) | (by << 3) | (bxy << 4);
+  }
+  if (l > 0) {
+    s.rpos = fpo + 2 * j * (lx(l - 1) + 2) + 2 * i;
+    int bit = 0;
+#pragma unroll
+    for (int dy = -1; dy <= 1; ++dy)
+#pragma unroll
+      for (int dx = -1; dx <= 1; ++dx) {
+        if (dx == 0 && dy == 0) continue;
+        const int ii = i + dx, jj = j + dy;
+        const bool nin = ii >= 0 && ii < nx && jj >= 0 && jj < ny;
+        const uint8_t fv = inf[o + (nin ? ii + jj * nx : 0)];
+        s.walls |= (!nin || is_wall(fv) ? 1 : 0) << bit++;
+      }
+  }
+  s.n = in && is_act(f) ? f & 7 : 0;
+  return s;
+}
+// The same in one word: 16 bits for each place in LDS, then n, ebits and walls.
+__device__ __forceinline__ uint64_t stage_pack(const StageConst& s) {
+  return (uint64_t)(uint32_t)(s.pos | (s.epos << 16)) |
+         ((uint64_t)(uint32_t)(s.rpos | (s.n << 16) | (s.ebits << 19) | (s.walls << 24)) << 32);
+}
+__device__ __forceinline__ StageConst stage_unpack(uint64_t w) {
+  const uint32_t lo = (uint32_t)w, hi = (uint32_t)(w >> 32);
+  StageConst s;
+  s.pos = lo & 0xFFFF;
+  s.epos = lo >> 16;
+  s.rpos = hi & 0xFFFF;
+  s.n = (hi >> 16) & 7;
+  s.ebits = (hi >> 19) & 31;
+  s.walls = hi >> 24;
+  return s;
+}
+__device__ __forceinline__ void stage_set(StageCell& c, const StageConst& s) {
+  c.pos = s.pos;
+  c.epos = s.epos;
+  c.ebits = s.ebits;
+  c.act = s.n != 0;
+  c.nn = (float)s.n;
+  c.inv = c.act ? inv_nns((uint8_t)s.n) : 0.f;
+}
+// Cells of the levels below the first before level l, each level from a wavefront on.
+template <class Lx, class Ly>
+__device__ __forceinline__ int stage_slot(Lx&& lx, Ly&& ly, int l) {
+  int s0 = 0;
+  for (int k = 1; k < l; ++k) s0 += (lx(k) * ly(k) + 63) & ~63;
+  return s0;
+}
+
 // 2 max(nx, ny) + 8 damped-Jacobi sweeps from zero on the coarsest level, a cell per lane
 // (lane = i + j nx).
 template <int NX>
@@ -1777,48 +1933,31 @@ __device__ __forceinline__ float coarsest_sweeps(float r, float nn, float rn, bo
   return x;
 }
 
-template <int NT, int K, int KB, class Lx, class Ly, class Lo, class Rhs, class Out>
+template <int NT, int K, int KB, bool TABLE, class Lx, class Ly, class Lo, class Rhs, class Out>
 __device__ __forceinline__ void stage_cycle(int nl, Lx&& lx, Ly&& ly, Lo&& lo,
-                                            const uint8_t* inf, float w, float w2, int sweeps,
+                                            const uint8_t* inf, const uint64_t* table, float w, float w2, int sweeps,
                                             float* lds, int words, Rhs&& rhs, Out&& out) {
   float *P0 = lds, *P1 = lds + words;
   for (int q = threadIdx.x; q < 2 * words; q += NT) lds[q] = 0.f;
   StageCell A[K], B[KB];
   float bm[KB][4];  // extra weights of the four children in the restriction
   int rpos[KB], bl[KB];
-  auto set = [&](StageCell& c, int l, int q, int po, int& i, int& j) {
-    const int nx = lx(l), ny = ly(l);
-    c.in = q < nx * ny;
-    small_divmod(c.in ? q : 0, nx, 1.0f / (float)nx, i, j);
-    const uint8_t f = inf[lo(l) + (c.in ? q : 0)];
-    c.act = c.in && is_act(f);
-    c.nn = nns_of(f);
-    c.inv = c.act ? inv_nns(f) : 0.f;
-    c.pos = po + (j + 1) * (nx + 2) + i + 1;
-    if (l + 1 < nl) {
-      const int cnx = lx(l + 1), cny = ly(l + 1), co = lo(l + 1);
-      const int I = i >> 1, J = j >> 1;
-      const int In = (i & 1) ? I + 1 : I - 1, Jn = (j & 1) ? J + 1 : J - 1;
-      const bool iok = In >= 0 && In < cnx, jok = Jn >= 0 && Jn < cny;
-      const int Ic = iok ? In : I, Jc = jok ? Jn : J;
-      const uint8_t fx = inf[co + Ic + J * cnx], fy = inf[co + I + Jc * cnx];
-      const uint8_t fxy = inf[co + Ic + Jc * cnx];
-      const bool bx = !iok || is_wall(fx), by = !jok || is_wall(fy);
-      const bool bxy = !(iok && jok) || is_wall(fxy);
-      c.epos = po + (nx + 2) * (ny + 3) + (J + 1) * (cnx + 2) + I + 1;
-      c.ebits = (i & 1) | ((j & 1) << 1) | (bx << 2) | (by << 3) | (bxy << 4);
-    }
-  };
+  const int n0 = lx(0) * ly(0);
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    int i, j;
-    set(A[k], 0, threadIdx.x + k * NT, 0, i, j);
+    const int q = threadIdx.x + k * NT;
+    if constexpr (TABLE)
+      stage_set(A[k], stage_unpack(q < n0 ? table[q] : 0ull));
+    else
+      stage_set(A[k], stage_const(nl, lx, ly, lo, inf, 0, q, 0, 0));
+    A[k].in = q < n0;
+    if (!A[k].in) A[k].pos = lx(0) + 3;  // of cell (0, 0): read, never written
   }
 #pragma unroll
   for (int b = 0; b < KB; ++b) {
     // the level of this wavefront's cells
     const int slot = __builtin_amdgcn_readfirstlane((int)(threadIdx.x & ~63u) + b * NT);
-    int l = 1, s0 = 0, po = nl > 0 ? (lx(0) + 2) * (ly(0) + 3) : 0, fpo = 0;
+    int l = 1, s0 = 0, po = (lx(0) + 2) * (ly(0) + 3), fpo = 0;
     for (; l < nl; ++l) {
       const int n64 = (lx(l) * ly(l) + 63) & ~63;
       if (slot < s0 + n64) break;
@@ -1829,24 +1968,23 @@ __device__ __forceinline__ void stage_cycle(int nl, Lx&& lx, Ly&& ly, Lo&& lo,
     bl[b] = l < nl ? l : -1;
     rpos[b] = 0;
     if (l < nl) {
-      int i, j;
-      set(B[b], l, slot - s0 + (threadIdx.x & 63), po, i, j);
-      const int nx = lx(l), ny = ly(l), o = lo(l);
-      rpos[b] = fpo + 2 * j * (lx(l - 1) + 2) + 2 * i;
-      uint8_t g[3][3];
-#pragma unroll
-      for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-          const int ii = i + dx - 1, jj = j + dy - 1;
-          const bool in = ii >= 0 && ii < nx && jj >= 0 && jj < ny;
-          const uint8_t fv = inf[o + (in ? ii + jj * nx : 0)];
-          g[dy][dx] = in ? fv : kWall;
-        }
+      const int q = slot - s0 + (int)(threadIdx.x & 63);
+      StageConst sc;
+      if constexpr (TABLE)
+        sc = stage_unpack(table[((n0 + 63) & ~63) + slot + (threadIdx.x & 63)]);
+      else
+        sc = stage_const(nl, lx, ly, lo, inf, l, q, po, fpo);
+      stage_set(B[b], sc);
+      rpos[b] = sc.rpos;
+      const int walls = sc.walls;
+      B[b].in = q < lx(l) * ly(l);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const int dx = (c & 1) ? 2 : 0, dy = (c >> 1) ? 2 : 0;
-        bm[b][c] = moved_weight(g[1][dx], g[dy][1], g[dy][dx]);
+        // neighbours in bits: 0 1 2 / 3 . 4 / 5 6 7
+        const int fx = (c & 1) ? 4 : 3, fy = (c >> 1) ? 6 : 1;
+        const int fxy = (c & 1) + (c >> 1 ? 6 : 1) + ((c & 1) ? 0 : -1);
+        auto wall = [&](int bit) { return (uint8_t)((walls >> bit) & 1 ? kWall : 0); };
+        bm[b][c] = moved_weight(wall(fx), wall(fy), wall(fxy));
       }
     }
   }
@@ -1978,10 +2116,10 @@ __device__ __forceinline__ void coarse_run(const MgCoarseArgs& a, float* lds, in
   const int nl = a.nlev - a.lc, n = a.nx[a.lc] * a.ny[a.lc];
   if (a.words > 0) {
     float r0 = 0.f;
-    stage_cycle<NT, 1, kStageKB>(
+    stage_cycle<NT, 1, kStageKB, false>(
         nl, [&](int l) { return a.nx[a.lc + l]; }, [&](int l) { return a.ny[a.lc + l]; },
-        [&](int l) { return a.off[a.lc + l] - a.off[a.lc]; }, a.inf_all, a.omega, a.omega2,
-        a.sweeps, lds, a.words,
+        [&](int l) { return a.off[a.lc + l] - a.off[a.lc]; }, a.inf_all, nullptr, a.omega,
+        a.omega2, a.sweeps, lds, a.words,
         [&](const bool (&act)[1], float (&r)[1]) {
           rhs(act, r);
           r0 = r[0];
@@ -2099,6 +2237,24 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_scene_setup(SceneCoarseAr
     for (int q = threadIdx.x; q < n; q += kCoarseThreads)
       out[t.off[l] + q] = make_info(slab + t.off[l], nx, t.ny[l], q % nx, q / nx);
   }
+  if (t.words == 0) return;
+  // the stage's words (formed in every cycle they took 2.6 of its 14 us)
+  __threadfence_block();
+  __syncthreads();
+  uint64_t* words = a.table + (size_t)blockIdx.x * a.table_stride;
+  auto lx = [&](int l) { return t.nx[l]; };
+  auto ly = [&](int l) { return t.ny[l]; };
+  auto lo = [&](int l) { return t.off[l]; };
+  const int n0 = t.nx[0] * t.ny[0];
+  int po = 0, fpo = 0;
+  for (int l = 0; l < t.nl; ++l) {
+    const int n = t.nx[l] * t.ny[l], n64 = (n + 63) & ~63;
+    uint64_t* const dst = words + (l == 0 ? 0 : ((n0 + 63) & ~63) + stage_slot(lx, ly, l));
+    for (int q = threadIdx.x; q < n64; q += kCoarseThreads)
+      dst[q] = stage_pack(stage_const(t.nl, lx, ly, lo, out, l, q, po, fpo));
+    fpo = po;
+    po += (t.nx[l] + 2) * (t.ny[l] + 3);
+  }
 }
 
 // One V-cycle of scene `scene`'s own levels.  rhs(act, cell, r):
@@ -2123,9 +2279,10 @@ __device__ __forceinline__ void scene_run(const SceneCoarseArgs& a, int scene, f
     cell[k] = t.cx + i + (t.cy + j) * a.pitch;
   }
   if (t.words > 0 && a.trunc == 0) {
-    stage_cycle<NT, K, kSceneKB>(
-        t.nl, [&](int l) { return t.nx[l]; },
-        [&](int l) { return t.ny[l]; }, [&](int l) { return t.off[l]; }, inf, a.omega, a.omega2, sweeps, lds, t.words,
+    stage_cycle<NT, K, kSceneKB, true>(
+        t.nl, [&](int l) { return t.nx[l]; }, [&](int l) { return t.ny[l]; },
+        [&](int l) { return t.off[l]; }, inf, a.table + (size_t)scene * a.table_stride, a.omega,
+        a.omega2, sweeps, lds, t.words,
         [&](const bool (&act)[K], float (&r)[K]) { rhs(act, cell, r); },
         [&](int k, float x) {
           if (threadIdx.x + k * NT < n) out(cell[k], x);
@@ -2874,52 +3031,6 @@ __device__ __forceinline__ void mgb_add(double v, double* dst, double* sm) {
   if (threadIdx.x == 0 && t[0] != 0.0) unsafeAtomicAdd(dst, t[0]);
 }
 
-// |b'_s|^2 (1 after the per-scene normalisation, 0 for a scene without unknowns) and
-// |r_s|^2 of x0 = 0.
-__global__ void __launch_bounds__(kT) k_mgb_init(MgbArgs a, const double* __restrict__ norm) {
-  for (int s = threadIdx.x; s < a.n_scenes; s += kT) {
-    const double b = norm[s] > 0.0 ? 1.0 : 0.0;
-    a.bb[s] = b;
-    a.rr[s] = b;
-  }
-}
-
-// Stop test of iteration `it` on the scenes' |r_s|^2, then the accumulators of this
-// iteration cleared.  One workgroup.
-__global__ void __launch_bounds__(kT) k_mgb_check(MgbArgs a, int it, int max_iter, double tol2,
-                                                  CgScalars* sc) {
-  __shared__ int s_done;
-  __shared__ double s_w[kT / 64];
-  if (threadIdx.x == 0) s_done = ld_dev(&sc->done);
-  __syncthreads();
-  if (s_done) return;
-  const int S = a.n_scenes;
-  int ok = 1;
-  double worst = 0.0;
-  for (int s = threadIdx.x; s < S; s += kT) {
-    const double bb = a.bb[s], rr = a.rr[s];
-    if (bb > 0.0) {
-      double thr = tol2 * bb;
-      if (thr < DBL_MIN) thr = DBL_MIN;
-      if (!(rr < thr)) ok = 0;
-      worst = fmax(worst, rr / bb);
-    }
-    a.rr[s] = 0.0;
-    a.pq[s] = 0.0;
-    a.rz[(it & 1) * S + s] = 0.0;
-  }
-  const int all_ok = __syncthreads_and(ok);
-  for (int off = 32; off > 0; off >>= 1) worst = fmax(worst, __shfl_down(worst, off, 64));
-  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = worst;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kT / 64; ++w) worst = fmax(worst, s_w[w]);
-    sc->iter = it;
-    sc->err = sqrt(worst);
-    if (all_ok || it >= max_iter) st_dev(&sc->done, 1);
-  }
-}
-
 // The rows k = 0 .. kMgbRows-1 of a thread's column in its tile: cell index (0 for a
 // row outside the scene, in[k] = false) and info byte.  Loads first, then use.
 struct MgbCells {
@@ -2945,7 +3056,8 @@ __device__ __forceinline__ MgbCells mgb_cells(const MgbTile& t, int W,
   return m;
 }
 
-// r_s . z_s.  A block takes kRzTiles consecutive tiles (the list runs scene by scene,
+// r_s . z_s, where level 0's up kernel cannot form it (a tile of more than four scenes; one
+// more launch, 38 us per step of 32 scenes).  A block takes kRzTiles consecutive tiles (the list runs scene by scene,
 // so they mostly share one): their r and z loads are all in flight before the first
 // use, one block sum covers them, and each run of tiles of one scene adds one atomic.
 constexpr int kRzTiles = 4;
@@ -3136,19 +3248,14 @@ __global__ void __launch_bounds__(kT) k_mgb_xr(MgbArgs a, const uint8_t* __restr
     x_new[c] = xn;
     r[c] = rv;
   }
-  mgb_add(acc, &a.rr[t.s], sm);
+  mgb_add(acc, &a.rr[((it + 1) & 1) * a.n_scenes + t.s], sm);
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->spmv = it + 1;
 }
 
-void launch_mgb_init(hipStream_t s, const MgbArgs& a, const double* norm, const MgHost& m) {
-  k_mgb_init<<<1, kT, 0, s>>>(a, norm);
+void launch_mgb_flags(hipStream_t s, const MgHost& m) {
+  const MgbArgs& a = m.mgb;
   if (a.vflag && a.n_tiles > 0)
     k_mgb_flags<<<a.n_tiles, kT, 0, s>>>(a, m.inf[0], const_cast<uint8_t*>(a.vflag));
-}
-
-void launch_mgb_check(hipStream_t s, const MgbArgs& a, int it, int max_iter, double tol,
-                      CgScalars* sc) {
-  k_mgb_check<<<1, kT, 0, s>>>(a, it, max_iter, tol * tol, sc);
 }
 
 // a.vflag is set with the tile table when a batch is packed (k_mgb_rz reads it as given)
@@ -3253,11 +3360,9 @@ void launch_mg_setup(hipStream_t s, const Geom& g, const MgHost& m, const uint8_
     k_mg_setup0<<<nb, kT, 0, s>>>(g, label, uf, vf, m.inf[0], m.b, m.part_sum, m.part_cnt, rhs,
                                   rhs ? m.part_liq : nullptr);
   }
-  if (batch) {
+  if (batch)
     k_mg_scene_norm<<<batch->n_scenes, 1024, 0, s>>>(m.b, g.nx, batch->rect, batch->norm,
-                                                     batch->inv);
-    k_mg_scene_scale<<<nb, kT, 0, s>>>(C, batch->sid, batch->inv, m.b);
-  }
+                                                     batch->inv, m.mgb);
   // x[0] holds the previous solve's solution (k_mg_finish); x[1] is free until the
   // first update of this solve
   if (warm) k_mg_warm<<<nb, kT, 0, s>>>(C, m.inf[0], m.x[0], m.x[1]);
@@ -3269,7 +3374,8 @@ void launch_mg_setup(hipStream_t s, const Geom& g, const MgHost& m, const uint8_
                                   warm ? m.x[1] : nullptr,
                                   m.x[0], m.rl[0], m.part_sum, m.part_cnt, n_part, m.part_bb,
                                   m.part_rr, sc, rhs && !adj_rhs ? m.part_liq : nullptr, n_fluid,
-                                  tiled ? m.tflag : nullptr, n_tiles);
+                                  tiled ? m.tflag : nullptr, n_tiles,
+                                  batch ? batch->sid : nullptr, batch ? batch->inv : nullptr);
   // the levels not formed by k_mg_setup0t, one launch each, down to level l0 - 1
   for (int l = std::max(1, lk + 1); l < std::min(l0, m.nlev); ++l) {
     const int nf = m.nx[l - 1] * m.ny[l - 1], ncl = m.nx[l] * m.ny[l];
@@ -3355,7 +3461,17 @@ MgCheck mg_check_args(const MgHost& m, int it, int max_iter, double tol, CgScala
   // |r|^2: k_mg_setup1's partials (it == 0), else k_mg_xr's or, fused, level 0's down
   // kernel's (one per tile); |b'|^2 from k_mg_setup1
   const int n_rr = (m.fused && it > 0) ? mg_down_blocks(m, 0) : nb;
-  return MgCheck{sc, m.part_rr, n_rr, m.part_bb, nb, tol * tol, max_iter, m.per_scene ? 1 : 0};
+  MgCheck k{sc, m.part_rr, n_rr, m.part_bb, nb, tol * tol, max_iter};
+  if (m.per_scene) {
+    const MgbArgs& a = m.mgb;
+    k.S = a.n_scenes;
+    k.rr = a.rr + (it & 1) * a.n_scenes;
+    k.rr_next = a.rr + ((it + 1) & 1) * a.n_scenes;
+    k.bb = a.bb;
+    k.pq = a.pq;
+    k.rz = a.rz + (it & 1) * a.n_scenes;
+  }
+  return k;
 }
 
 int mg_part_rr_size(const MgHost& m) {
@@ -3554,16 +3670,26 @@ void launch_mg_coarse(hipStream_t s, const MgHost& m, int it, int max_iter, doub
 
 void launch_mg_up(hipStream_t s, const MgHost& m, int l, int it, CgScalars* sc) {
   const int blocks = mg_up_blocks(m.nx[l], m.ny[l]);
-  auto go0 = [&](auto nt) {
+  MgTileScenes scenes;
+  if (m.per_scene && m.mgb.tile_scenes)
+    scenes = MgTileScenes{m.mgb.tile_scenes, m.mgb.rect, m.mgb.rz + (it & 1) * m.mgb.n_scenes};
+  auto go0_of = [&](auto nt, auto of_scenes) {
     constexpr int NT = decltype(nt)::value;
+    constexpr bool B = decltype(of_scenes)::value;
     if (m.level0_sweeps == 3)
-      k_mg_up<true, NT, 3><<<blocks, NT, 0, s>>>(mg_level(m, 0), mg_level(m, 1), m.coarse.omega,
-                                                 m.coarse.omega2, sc, m.part_rz, it, m.tflag,
-                                                 mg_sweeps0(m), m.tmap);
+      k_mg_up<true, NT, 3, B><<<blocks, NT, 0, s>>>(
+          mg_level(m, 0), mg_level(m, 1), m.coarse.omega, m.coarse.omega2, sc, m.part_rz, it,
+          m.tflag, mg_sweeps0(m), m.tmap, scenes);
     else
-      k_mg_up<true, NT><<<blocks, NT, 0, s>>>(mg_level(m, 0), mg_level(m, 1), m.coarse.omega,
-                                              m.coarse.omega2, sc, m.part_rz, it, m.tflag,
-                                              MgSweeps{}, m.tmap);
+      k_mg_up<true, NT, 2, B><<<blocks, NT, 0, s>>>(
+          mg_level(m, 0), mg_level(m, 1), m.coarse.omega, m.coarse.omega2, sc, m.part_rz, it,
+          m.tflag, MgSweeps{}, m.tmap, scenes);
+  };
+  auto go0 = [&](auto nt) {
+    if (scenes.of)
+      go0_of(nt, std::true_type{});
+    else
+      go0_of(nt, std::false_type{});
   };
   if (l == 0 && m.l0_threads == 1024)
     go0(std::integral_constant<int, 1024>{});
@@ -3576,7 +3702,7 @@ void launch_mg_up(hipStream_t s, const MgHost& m, int l, int it, CgScalars* sc) 
       constexpr int S = decltype(ns)::value;
       k_mg_up<false, kTileMany, S><<<blocks, kTileMany, 0, s>>>(
           mg_level(m, l), mg_level(m, l + 1), m.coarse.omega, m.coarse.omega2, sc, nullptr, it,
-          m.tflag_l[l], mg_sweeps(m), nullptr);
+          m.tflag_l[l], mg_sweeps(m), nullptr, MgTileScenes{});
     });
   }
 }
