@@ -149,12 +149,12 @@ def solve_bytes(name, nx, ny, solves):
 # FETCH_SIZE reads 0.5 GiB for its 1 GiB read (factor 2.0), WRITE_SIZE 1 GiB (1.0).
 # traffic = (2.0 * FETCH_SIZE + 1.0 * WRITE_SIZE) * 1024.
 MEASURED_TRAFFIC_1024 = {
-    "cg_mg_down0": (2.0 * 3201.4 + 6303.8) * 1024,
-    "cg_mg_up0": (2.0 * 1828.3 + 1309.8) * 1024,
-    "cg_mg_dir": (2.0 * 1229.6 + 1637.5) * 1024,
-    "particle_scatter": (2.0 * 8065.4 + 18469.3) * 1024,
-    "particle_gather": (2.0 * 10294.5 + 16676.3) * 1024,
-    "face_update": (2.0 * 12821.0 + 28672.2) * 1024,
+    "cg_mg_down0": (2.0 * 3296.1 + 6305.5) * 1024,
+    "cg_mg_up0": (2.0 * 1831.5 + 1312.2) * 1024,
+    "cg_mg_dir": (2.0 * 1270.3 + 1644.5) * 1024,
+    "particle_scatter": (2.0 * 8081.8 + 15745.9) * 1024,
+    "particle_gather": (2.0 * 10291.5 + 16676.3) * 1024,
+    "face_update": (2.0 * 12823.5 + 28672.1) * 1024,
 }
 
 

@@ -788,10 +788,10 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
                                           "cg_mg_up4", "cg_mg_up5", "cg_mg_up6", "cg_mg_up7+"};
   // one CG iteration: the V-cycle's kernels, the direction (and the x / residual
   // update where it is not fused into the next iteration's level-0 kernel).  Its head
-  // is its kernels up to and including the stop test (level 0's
-  // down kernel, or levels 0-1 in the fused form; the whole iteration where the
-  // hierarchy has no tile level), its tail the rest: once the solve has stopped in
-  // iteration q's head, the kernels after it return at once.
+  // is its kernels up to and including the stop test (level 0's down kernel, or levels
+  // 0-1 in the fused form; the whole iteration where the hierarchy has no tile level),
+  // its tail the rest: once the solve has stopped in iteration q's head, the kernels
+  // after it return at once.
   const int head_levels = m.fused ? 2 : 1;
   const bool whole_head = !h->batch && m.lc < head_levels;
   // the levels with launches of their own; the others (cycle) share one, which in the

@@ -357,7 +357,7 @@ int fsg_set_timing(fsg_domain *h, int32_t enable);
    per launch from the device wall clock, free of the launch gaps that HIP events
    around a launch include.  enable = 1: the one-workgroup kernel k_mg_coarse (start
    to end), which runs as its own kernel only where the grid has fewer than two tile
-   levels (elsewhere the last tile level's down kernel runs that stage, and mode 1
+   levels (elsewhere the kernel of the small levels runs that stage, and mode 1
    records no launch); enable = 2: level 0's down kernel (earliest block start to
    latest block end, the first 4096 launches; the span buffer is kept until
    fsg_destroy); 0 stops it.  A nonzero value clears the total, which then covers
