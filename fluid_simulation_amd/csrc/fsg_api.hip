@@ -515,6 +515,7 @@ void classify_and_splat(fsg_domain* h) {
       launch_bucket_order(h->stream, h->g, h->pt, h->np, h->bkt_cnt, h->bkt_off, h->prank,
                           h->psorted, fsg::CellInit{h->label, h->solid, fx ? nullptr : h->acc});
     });
+    if (fsg::bucket_scan_in_fill(h->g)) std::swap(h->bkt_cnt, h->bkt_off);
     src = h->psorted;
   } else {
     timed(h, "cell_init", [&] {
@@ -1006,9 +1007,8 @@ int solve_pressure(fsg_domain* h) {
   if (solver == FSG_SOLVER_MG) return mg_solve(h, -1, nullptr, true);
   timed(h, "pcg_setup", [&] {
     launch_pcg_count(h->stream, h->g, h->label, h->counts);
-    launch_scan_counts(h->stream, pcg_tiles(h->g), h->counts, h->offsets, h->n_fluid);
-    launch_pcg_fill(h->stream, h->g, h->label, h->offsets, h->index_of, h->cell_of, UF(h), VF(h),
-                    h->ap, h->b, h->info);
+    launch_pcg_fill(h->stream, h->g, h->label, h->counts, h->offsets, h->n_fluid, h->index_of,
+                    h->cell_of, UF(h), VF(h), h->ap, h->b, h->info);
   });
   const bool refined = solver == FSG_SOLVER_REFINED, plain = solver == FSG_SOLVER_PLAIN;
   // Launch shape of the one-launch CG: G blocks of 512 threads, kpt x 1024 unknowns per

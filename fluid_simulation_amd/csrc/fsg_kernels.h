@@ -89,11 +89,13 @@ void launch_particle_scatter(hipStream_t s, const Geom& g, const float4* pt, int
                              const BatchTables* batch = nullptr, long long* acc_fx = nullptr);
 void launch_fx_to_float(hipStream_t s, int64_t n, long long* fx, float* out);
 // The splat's bucket order for one domain (np < 2^31, bucket_count(g) <= kMaxBuckets):
-// cnt (zero on entry, zero again on return) and off hold bucket_count(g) ints, rank np
-// ints; sorted receives the np particles grouped by bucket.  ci: the step's cell set-up
+// cnt (zero on entry) and off hold bucket_count(g) ints, rank np ints; sorted receives the
+// np particles grouped by bucket.  On return cnt is zero again, or, with
+// bucket_scan_in_fill(g), off is: the caller swaps the two.  ci: the step's cell set-up
 // (launch_cell_init's work), done by the count kernel as well.
 constexpr int kMaxBuckets = 16384;  // the count kernel's LDS histogram: 64 KiB
 int bucket_count(const Geom& g);
+bool bucket_scan_in_fill(const Geom& g);
 void launch_bucket_order(hipStream_t s, const Geom& g, const float4* pt, int64_t np, int* cnt,
                          int* off, int* rank, float4* sorted, const CellInit& ci = CellInit{});
 // A packed batch: every scene's particles grouped by the 16 x 16-cell buckets of its own
@@ -209,9 +211,10 @@ struct CgParams {
 int pcg_tiles(const Geom& g);
 void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts);
 void launch_scan_counts(hipStream_t s, int nb, const int* counts, int* offsets, int* n_fluid);
-void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
-                     int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
-                     float* rhs, uint8_t* info);
+// counts: launch_pcg_count's; offsets: scratch of as many; n_fluid: their sum (out)
+void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* counts,
+                     int* offsets, int* n_fluid, int* index_of, int* cell_of, const float* uf,
+                     const float* vf, float* b, float* rhs, uint8_t* info);
 
 // plain form (partials: >= 12288 doubles)
 void launch_cg_init(hipStream_t s, int F, const CgParams& cp, const int* cell_of,

@@ -881,7 +881,7 @@ __global__ void __launch_bounds__(256) k_bucket_count(Geom g0, const float4* __r
                                                       int np, int bx0, int nb0,
                                                       int* __restrict__ cnt,
                                                       int* __restrict__ rank, BatchTables tb,
-                                                      CellInit ci) {
+                                                      CellInit ci, int* __restrict__ clear) {
   static_assert(!BATCH || PPT == 1, "a batch block is one particle tile");
   extern __shared__ int s_h[];  // nb ints
   int bx = bx0, nb = nb0, base = 0;
@@ -904,6 +904,8 @@ __global__ void __launch_bounds__(256) k_bucket_count(Geom g0, const float4* __r
       for (int c = blockIdx.x * 256 + threadIdx.x; c < C; c += gridDim.x * 256)
         cell_init_one(g0, ci, c);
     }
+    if (clear)  // the next step's counts
+      for (int e = blockIdx.x * 256 + threadIdx.x; e < nb; e += gridDim.x * 256) clear[e] = 0;
   }
   for (int e = threadIdx.x; e < nb; e += 256) s_h[e] = 0;
   __syncthreads();
@@ -1004,9 +1006,16 @@ __global__ void __launch_bounds__(1024) k_bucket_scan(int* __restrict__ cnt,
 // BATCH: the offsets run over all scenes' buckets in scene order, and the scenes'
 // particle ranges are contiguous in scene order, so every scene's particles land in
 // its own range.
-template <bool BATCH>
+// SCAN (a single domain of at most 256 buckets): off holds the counts, which every block
+// turns into offsets itself, a thread per bucket; k_bucket_scan's launch goes (3.5-4.1 us
+// per step; four steps of 130 x 96 cells 1272 -> 1259 us), and k_bucket_count clears the counts of
+// the step before, which lie in the other of two arrays.  More buckets would take a block
+// more than one pass over the counts, and 1024^2 has 4096.
+constexpr int kFillScanBuckets = 256;
+template <bool BATCH, bool SCAN>
 __global__ void __launch_bounds__(256) k_bucket_fill(Geom g0, const float4* __restrict__ pt,
-                                                     int np, int bx0, const int* __restrict__ off,
+                                                     int np, int bx0, int nb,
+                                                     const int* __restrict__ off,
                                                      const int* __restrict__ rank,
                                                      float4* __restrict__ sorted, BatchTables tb) {
   const PartTile T = part_tile<BATCH>(g0, np, tb);
@@ -1017,9 +1026,27 @@ __global__ void __launch_bounds__(256) k_bucket_fill(Geom g0, const float4* __re
     base = sc.bucket_base;
   }
   const int64_t p = T.p;
+  __shared__ int s_off[SCAN ? kFillScanBuckets : 1], s_w[SCAN ? 4 : 1];
+  if (SCAN) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int v = (int)threadIdx.x < nb ? off[threadIdx.x] : 0;
+    int x = v;  // inclusive scan over the wave
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(x, o, 64);
+      if (lane >= o) x += y;
+    }
+    if (lane == 63) s_w[wave] = x;
+    __syncthreads();
+    int e = x - v;
+    for (int w = 0; w < wave; ++w) e += s_w[w];
+    s_off[threadIdx.x] = e;
+    __syncthreads();
+  }
   if (p >= T.np_end) return;
   const float4 q = pt[p];
-  const int d = off[base + particle_bucket(T.g, q, bx)] + rank[p];
+  const int k = base + particle_bucket(T.g, q, bx);
+  const int d = (SCAN ? s_off[k] : off[k]) + rank[p];
   if (d >= 0 && d < np) sorted[d] = q;
 }
 
@@ -1110,6 +1137,8 @@ int bucket_count(const Geom& g) {
          ((g.ny + (1 << kBucketShift) - 1) >> kBucketShift);
 }
 
+bool bucket_scan_in_fill(const Geom& g) { return bucket_count(g) <= kFillScanBuckets; }
+
 void launch_bucket_order(hipStream_t s, const Geom& g, const float4* pt, int64_t np, int* cnt,
                          int* off, int* rank, float4* sorted, const CellInit& ci) {
   if (np <= 0) return;
@@ -1117,10 +1146,18 @@ void launch_bucket_order(hipStream_t s, const Geom& g, const float4* pt, int64_t
   const int nb = bucket_count(g);
   const int n = (int)np;
   constexpr int kPPT = 4;
+  const bool scan = bucket_scan_in_fill(g);
   k_bucket_count<false, kPPT><<<nblocks((np + kPPT - 1) / kPPT), 256, (size_t)nb * sizeof(int),
-                                s>>>(g, pt, n, bx, nb, cnt, rank, BatchTables{}, ci);
+                                s>>>(g, pt, n, bx, nb, cnt, rank, BatchTables{}, ci,
+                                     scan ? off : nullptr);
+  if (scan) {
+    k_bucket_fill<false, true><<<nblocks(np), 256, 0, s>>>(g, pt, n, bx, nb, cnt, rank, sorted,
+                                                           BatchTables{});
+    return;
+  }
   k_bucket_scan<<<1, 1024, 0, s>>>(cnt, off, nb);
-  k_bucket_fill<false><<<nblocks(np), 256, 0, s>>>(g, pt, n, bx, off, rank, sorted, BatchTables{});
+  k_bucket_fill<false, false><<<nblocks(np), 256, 0, s>>>(g, pt, n, bx, nb, off, rank, sorted,
+                                                          BatchTables{});
 }
 
 void launch_bucket_order_batch(hipStream_t s, const float4* pt, int64_t np, int* cnt, int* off,
@@ -1129,9 +1166,10 @@ void launch_bucket_order_batch(hipStream_t s, const float4* pt, int64_t np, int*
   if (np <= 0 || tb.n_ptile == 0) return;
   const int n = (int)np;
   k_bucket_count<true, 1><<<tb.n_ptile, 256, (size_t)max_scene_buckets * sizeof(int), s>>>(
-      Geom{}, pt, n, 0, 0, cnt, rank, tb, CellInit{});
+      Geom{}, pt, n, 0, 0, cnt, rank, tb, CellInit{}, nullptr);
   k_bucket_scan<<<1, 1024, 0, s>>>(cnt, off, n_buckets);
-  k_bucket_fill<true><<<tb.n_ptile, 256, 0, s>>>(Geom{}, pt, n, 0, off, rank, sorted, tb);
+  k_bucket_fill<true, false><<<tb.n_ptile, 256, 0, s>>>(Geom{}, pt, n, 0, 0, off, rank, sorted,
+                                                        tb);
 }
 void launch_face_update(hipStream_t s, const Geom& g, int flags, float* u, float* v,
                         const float4* acc, float* prev_u, float* prev_v, const uint8_t* label,

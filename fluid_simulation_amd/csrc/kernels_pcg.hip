@@ -220,15 +220,24 @@ __global__ void __launch_bounds__(256) k_pcg_count(Geom g, const uint8_t* __rest
 // Per unknown: its cell, neighbour info (src/FluidSolver.cpp:379-410) and right-hand side
 // b = divVelX + divVelY (:413, MacGrid.h:98-111); per cell: its unknown's index (-1), and
 // b (0) as fsg_get_rhs returns it.
+// A block needs the number of unknowns in the tiles before its own.  With SCAN it sums
+// their counts itself and the last block writes the total; else k_scan_counts has formed
+// the offsets.  Up to kPcgScanTiles tiles (four loads per thread) that costs the kernel
+// less than the scan's launch (3.5 us): with the splat's buckets likewise, four steps of
+// 60 x 40 cells 663 -> 635 us.  More tiles: more passes, for a launch that a solve of that
+// size does not notice.
+constexpr int kPcgScanTiles = 1024;
+template <bool SCAN>
 __global__ void __launch_bounds__(256) k_pcg_fill(Geom g, const uint8_t* __restrict__ label,
                                                   const int* __restrict__ offsets,
+                                                  int* __restrict__ n_fluid,
                                                   int* __restrict__ index_of,
                                                   int* __restrict__ cell_of,
                                                   const float* __restrict__ uf,
                                                   const float* __restrict__ vf,
                                                   float* __restrict__ b, float* __restrict__ rhs,
                                                   uint8_t* __restrict__ info) {
-  __shared__ int s_w[4];
+  __shared__ int s_w[4], s_before[4];
   const int nx = g.nx, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int c[4], n = 0;
   bool in[4], liq[4];
@@ -247,8 +256,17 @@ __global__ void __launch_bounds__(256) k_pcg_fill(Geom g, const uint8_t* __restr
     if (lane >= o) x += y;
   }
   if (lane == 63) s_w[wave] = x;
+  if (SCAN) {
+    int before = 0;
+    for (int q = threadIdx.x; q < (int)blockIdx.x; q += 256) before += offsets[q];
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_down(before, o, 64);
+    if (lane == 0) s_before[wave] = before;
+  }
   __syncthreads();
-  int k = offsets[blockIdx.x] + x - n;
+  int k = SCAN ? s_before[0] + s_before[1] + s_before[2] + s_before[3] : offsets[blockIdx.x];
+  if (SCAN && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1)
+    *n_fluid = k + s_w[0] + s_w[1] + s_w[2] + s_w[3];
+  k += x - n;
   for (int w = 0; w < wave; ++w) k += s_w[w];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -623,11 +641,18 @@ int pcg_tiles(const Geom& g) { return ((g.nx + 31) / 32) * ((g.ny + 31) / 32); }
 void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts) {
   k_pcg_count<<<pcg_tiles(g), 256, 0, s>>>(g, label, counts);
 }
-void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* offsets,
-                     int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
+void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* counts,
+                     int* offsets, int* n_fluid, int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
                      float* rhs, uint8_t* info) {
-  k_pcg_fill<<<pcg_tiles(g), 256, 0, s>>>(g, label, offsets, index_of, cell_of, uf, vf, b, rhs,
-                                          info);
+  const int nb = pcg_tiles(g);
+  if (nb <= kPcgScanTiles) {
+    k_pcg_fill<true><<<nb, 256, 0, s>>>(g, label, counts, n_fluid, index_of, cell_of, uf, vf, b,
+                                        rhs, info);
+    return;
+  }
+  launch_scan_counts(s, nb, counts, offsets, n_fluid);
+  k_pcg_fill<false><<<nb, 256, 0, s>>>(g, label, offsets, n_fluid, index_of, cell_of, uf, vf, b,
+                                       rhs, info);
 }
 
 size_t pcg_lds_bytes(int F, int grid, int nx) {
