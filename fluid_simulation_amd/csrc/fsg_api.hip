@@ -2208,8 +2208,7 @@ int fsg_checkpoint_save(fsg_domain* h, int32_t slot) {
   list.add(c.v[0], VF(h), (int64_t)C * 4);
   list.add(c.u[1], UB(h), (int64_t)C * 4);
   list.add(c.v[1], VB(h), (int64_t)C * 4);
-  launch_copies(h->stream, list);
-  HIPCHK(h, hipGetLastError());
+  HIPCHK(h, launch_copies(h->stream, list));
   return FSG_OK;  // stream-ordered: later work on the handle sees the copy
 }
 
@@ -2226,8 +2225,7 @@ int fsg_checkpoint_load(fsg_domain* h, int32_t slot) {
   list.add(VF(h), c.v[0], (int64_t)C * 4);
   list.add(UB(h), c.u[1], (int64_t)C * 4);
   list.add(VB(h), c.v[1], (int64_t)C * 4);
-  launch_copies(h->stream, list);
-  HIPCHK(h, hipGetLastError());
+  HIPCHK(h, launch_copies(h->stream, list));
   return FSG_OK;  // stream-ordered
 }
 
@@ -2530,7 +2528,7 @@ static int adjoint_step_sl(fsg_domain* h, float dt) {
   fsg::CopyList front;
   front.add(a.f0u, UF(h), (int64_t)C * 4);
   front.add(a.f0v, VF(h), (int64_t)C * 4);
-  launch_copies(h->stream, front);
+  HIPCHK(h, launch_copies(h->stream, front));
   a.taping = true;
   int rc = step_semi_lagrangian(h, dt);
   a.taping = false;
@@ -2543,7 +2541,7 @@ static int adjoint_step_sl(fsg_domain* h, float dt) {
   fsg::CopyList adj;
   adj.add(a.su, a.fu, (int64_t)C * 4);
   adj.add(a.sv, a.fv, (int64_t)C * 4);
-  launch_copies(h->stream, adj);
+  HIPCHK(h, launch_copies(h->stream, adj));
   timed(h, "adj_advect_grid", [&] {
     launch_adj_advect_grid(h->stream, h->g, a.x0, np, UF(h), VF(h), h->prm.integrator, dt, a.pbar,
                            a.su, a.sv);
@@ -2595,7 +2593,7 @@ int fsg_adjoint_step(fsg_domain* h, int32_t scheme, float dt) {
   const size_t C = ncell(h);
   fsg::CopyList start;
   start.add(a.x0, h->pt, np * (int64_t)sizeof(float4));
-  launch_copies(h->stream, start);
+  HIPCHK(h, launch_copies(h->stream, start));
   if (scheme == FSG_SCHEME_SEMI_LAGRANGIAN) return adjoint_step_sl(h, dt);
   a.taping = true;
   int rc = step_flip_family(h, scheme, dt);

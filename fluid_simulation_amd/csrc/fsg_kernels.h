@@ -72,7 +72,8 @@ struct CopyList {
     bytes[n++] = b;
   }
 };
-void launch_copies(hipStream_t s, const CopyList& list);
+// The launch's own result: an error that another call left behind stays where it is.
+hipError_t launch_copies(hipStream_t s, const CopyList& list);
 void launch_cell_init(hipStream_t s, const Geom& g, uint8_t* label, const uint8_t* solid,
                       float4* acc, int do_labels, int do_acc);
 // The cell set-up of a step: label (if set) := SOLID on the border and where solid is

@@ -1057,9 +1057,9 @@ __global__ void __launch_bounds__(256) k_fill_f32(float* __restrict__ a, int64_t
 }
 
 // A saved state's arrays in one launch in place of a runtime copy each: blockIdx.y is the
-// array, a thread moves kCopyU 16-byte words, stored past the L2 (the copy is not read soon,
-// and written through the L2 it took 18 us).  16.6 MB of particles and four grids of 1 MB:
-// 12.6 -> 5.7 us; 0.3 MB and four of 64 KB: 12.6 -> 3.0 us.
+// array, a thread moves kCopyU 16-byte words, stored past the L2 (through it the copy took
+// 18 us).  16.6 MB of particles and four grids of 1 MB: 12.6 -> 5.7 us; 0.3 MB and four of
+// 64 KB: 12.6 -> 3.0 us.
 constexpr int kCopyU = 4;
 __global__ void __launch_bounds__(256) k_copies(CopyList list) {
   typedef float Word __attribute__((ext_vector_type(4)));
@@ -1124,12 +1124,14 @@ void launch_fx_to_float(hipStream_t s, int64_t n, long long* fx, float* out) {
   if (n > 0) k_fx_to_float<<<nblocks(n), 256, 0, s>>>(n, fx, out);
 }
 
-void launch_copies(hipStream_t s, const CopyList& list) {
-  if (list.n == 0) return;
+hipError_t launch_copies(hipStream_t s, const CopyList& list) {
+  if (list.n == 0) return hipSuccess;
   int64_t most = 0;
   for (int k = 0; k < list.n; ++k) most = std::max(most, list.bytes[k]);
   const int64_t per_block = 256 * kCopyU * 16;
-  k_copies<<<dim3((unsigned)((most + per_block - 1) / per_block), list.n), 256, 0, s>>>(list);
+  const dim3 grid((unsigned)((most + per_block - 1) / per_block), list.n);
+  void* args[] = {(void*)&list};
+  return hipLaunchKernel((const void*)k_copies, grid, dim3(256), args, 0, s);
 }
 
 int bucket_count(const Geom& g) {
