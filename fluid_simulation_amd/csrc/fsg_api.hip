@@ -223,8 +223,8 @@ struct fsg_domain {
   int* counts = nullptr;
   int* offsets = nullptr;
   int* n_fluid = nullptr;
-  // the Jacobi-CG forms' unknowns (tile order): index per cell, cell per unknown; b per
-  // cell (every form), and per unknown in ap
+  // the Jacobi-CG forms' unknowns (in tiles, the many-launch form's in rows): index per
+  // cell, cell per unknown; b per cell (every form), and per unknown in ap
   int* index_of = nullptr;
   int* cell_of = nullptr;
   // true: the last pressure solve indexed its unknowns in index_of; false (multigrid
@@ -957,8 +957,13 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
 }
 
 // The three-kernels-per-iteration form of the plain CG, in batches of check_every
-// iterations between stop-test reads: systems that the one-launch form cannot take.
+// iterations between stop-test reads: systems that the one-launch form cannot take.  Its
+// unknowns are in row-major order.
 int plain_many_launches(fsg_domain* h, int F, const CgParams& cp) {
+  timed(h, "pcg_setup", [&] {
+    launch_pcg_rows(h->stream, h->g, h->label, h->counts, h->offsets, h->n_fluid, h->index_of,
+                    h->cell_of, UF(h), VF(h), h->ap, h->b, h->info);
+  });
   timed(h, "cg_init", [&] {
     // b per unknown lies in ap until the first iteration writes it
     launch_cg_init(h->stream, F, cp, h->cell_of, h->info, h->ap, h->r, h->pg0, h->xg, h->partials,
@@ -1005,12 +1010,22 @@ int solve_pressure(fsg_domain* h) {
   // the device); it reads the count back with its stop test.
   h->compacted = solver != FSG_SOLVER_MG;
   if (solver == FSG_SOLVER_MG) return mg_solve(h, -1, nullptr, true);
+  const bool refined = solver == FSG_SOLVER_REFINED, plain = solver == FSG_SOLVER_PLAIN;
+  // The most unknowns that the plain form solves in one launch.  On a grid of more cells the
+  // order of the unknowns (plain_many_launches) is chosen once they are counted.
+  const size_t plain_max = (size_t)4096 * h->max_coop_blocks;
+  const bool count_first = plain && ncell(h) > plain_max;
+  auto fill = [&] {
+    launch_pcg_fill(h->stream, h->g, h->label, h->counts, h->offsets, h->n_fluid, h->index_of,
+                    h->cell_of, UF(h), VF(h), h->ap, h->b, h->info, count_first);
+  };
   timed(h, "pcg_setup", [&] {
     launch_pcg_count(h->stream, h->g, h->label, h->counts);
-    launch_pcg_fill(h->stream, h->g, h->label, h->counts, h->offsets, h->n_fluid, h->index_of,
-                    h->cell_of, UF(h), VF(h), h->ap, h->b, h->info);
+    if (count_first)
+      launch_scan_counts(h->stream, pcg_tiles(h->g), h->counts, h->offsets, h->n_fluid);
+    else
+      fill();
   });
-  const bool refined = solver == FSG_SOLVER_REFINED, plain = solver == FSG_SOLVER_PLAIN;
   // Launch shape of the one-launch CG: G blocks of 512 threads, kpt x 1024 unknowns per
   // block.  One block exchanges nothing and needs no cooperative launch, so it takes
   // every system that fits its registers (1.0-2.6 us per iteration against 4.0-4.4 for
@@ -1026,6 +1041,7 @@ int solve_pressure(fsg_domain* h) {
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->host_stats.n_fluid = F;
     h->last_F = F;
+    if (count_first && (size_t)F <= plain_max) timed(h, "pcg_setup", fill);
     if (F == 0) return FSG_OK;
   }
   // The largest systems: kpt 4 (refined form: 2) on every co-resident block; the

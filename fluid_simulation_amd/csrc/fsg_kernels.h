@@ -212,10 +212,15 @@ struct CgParams {
 int pcg_tiles(const Geom& g);
 void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts);
 void launch_scan_counts(hipStream_t s, int nb, const int* counts, int* offsets, int* n_fluid);
-// counts: launch_pcg_count's; offsets: scratch of as many; n_fluid: their sum (out)
+// counts: launch_pcg_count's; offsets: scratch of as many; n_fluid: their sum (out);
+// scanned: launch_scan_counts has formed the two
 void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* counts,
                      int* offsets, int* n_fluid, int* index_of, int* cell_of, const float* uf,
-                     const float* vf, float* b, float* rhs, uint8_t* info);
+                     const float* vf, float* b, float* rhs, uint8_t* info, bool scanned);
+// The same in row-major order (the many-launch form), count and scan included
+void launch_pcg_rows(hipStream_t s, const Geom& g, const uint8_t* label, int* counts, int* offsets,
+                     int* n_fluid, int* index_of, int* cell_of, const float* uf, const float* vf,
+                     float* b, float* rhs, uint8_t* info);
 
 // plain form (partials: >= 12288 doubles)
 void launch_cg_init(hipStream_t s, int F, const CgParams& cp, const int* cell_of,

@@ -4,7 +4,7 @@
 // (kernels_pcg.hip) holds in registers (about 2^20), and for a plain solve whose
 // co-resident launch was refused or gave up a wait.
 //
-// Unknowns are the LIQUID cells in the order of kernels_pcg.hip's set-up.  The operator
+// Unknowns are the LIQUID cells in row-major order (kernels_pcg.hip's set-up).  The operator
 // is applied matrix-free: one info byte per unknown holds the four LIQUID-neighbour bits
 // and the count of non-SOLID neighbours, so A's row is diag_tab[count] at the centre and
 // off = 1/dx^2 at each LIQUID neighbour; x and p are cell grids.

@@ -194,7 +194,18 @@ __device__ __forceinline__ bool grid_sum(PcgNet& net, double (&v)[NV], PcgShared
 // patch's rim (320 links for 4 full tiles), where a range of the row-major order has a
 // full row of the grid above and below it (2044 at 1024 columns); the halo is read
 // through device-coherent loads in every iteration (62 blocks: 5.5 -> 5.0 us each).
+// ROWS: row-major order, a "tile" being 1024 cells in a row: the many-launch form's, whose
+// kernels walk the unknowns through the cell grids and are bound by the lines that a wave
+// touches (2048^2 box, 4.2 million unknowns: 67.9 us per iteration in rows, 74.1 in tiles;
+// 3000^2, 4.6 million in no simple shape: 76.9 and 88.9).
+template <bool ROWS>
 __device__ __forceinline__ bool tile_cell(const Geom& g, int tile, int t, int& i, int& j) {
+  if (ROWS) {
+    const int c = tile * 1024 + t;
+    j = c / g.nx;
+    i = c - j * g.nx;
+    return j < g.ny;
+  }
   const int tiles_x = (g.nx + 31) >> 5;
   i = (tile % tiles_x) * 32 + (t & 31);
   j = (tile / tiles_x) * 32 + (t >> 5);
@@ -202,6 +213,7 @@ __device__ __forceinline__ bool tile_cell(const Geom& g, int tile, int t, int& i
 }
 
 // LIQUID cells per tile (thread t: the four cells 4 t .. 4 t + 3 of the tile).
+template <bool ROWS>
 __global__ void __launch_bounds__(256) k_pcg_count(Geom g, const uint8_t* __restrict__ label,
                                                    int* __restrict__ counts) {
   __shared__ int s_w[4];
@@ -209,7 +221,7 @@ __global__ void __launch_bounds__(256) k_pcg_count(Geom g, const uint8_t* __rest
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     int i, j;
-    if (tile_cell(g, blockIdx.x, 4 * threadIdx.x + e, i, j)) n += label[i + j * g.nx] == kLiquid;
+    if (tile_cell<ROWS>(g, blockIdx.x, 4 * threadIdx.x + e, i, j)) n += label[i + j * g.nx] == kLiquid;
   }
   for (int off = 32; off > 0; off >>= 1) n += __shfl_down(n, off, 64);
   if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = n;
@@ -227,7 +239,7 @@ __global__ void __launch_bounds__(256) k_pcg_count(Geom g, const uint8_t* __rest
 // 60 x 40 cells 663 -> 635 us.  More tiles: more passes, for a launch that a solve of that
 // size does not notice.
 constexpr int kPcgScanTiles = 1024;
-template <bool SCAN>
+template <bool SCAN, bool ROWS>
 __global__ void __launch_bounds__(256) k_pcg_fill(Geom g, const uint8_t* __restrict__ label,
                                                   const int* __restrict__ offsets,
                                                   int* __restrict__ n_fluid,
@@ -244,7 +256,7 @@ __global__ void __launch_bounds__(256) k_pcg_fill(Geom g, const uint8_t* __restr
   int ci[4], cj[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    in[e] = tile_cell(g, blockIdx.x, 4 * threadIdx.x + e, ci[e], cj[e]);
+    in[e] = tile_cell<ROWS>(g, blockIdx.x, 4 * threadIdx.x + e, ci[e], cj[e]);
     c[e] = in[e] ? ci[e] + cj[e] * nx : 0;
     liq[e] = in[e] && label[c[e]] == kLiquid;
     n += liq[e];
@@ -639,20 +651,29 @@ __global__ void __launch_bounds__(kPcgThreads) k_pcg_one(PersistentArgs a) {
 
 int pcg_tiles(const Geom& g) { return ((g.nx + 31) / 32) * ((g.ny + 31) / 32); }
 void launch_pcg_count(hipStream_t s, const Geom& g, const uint8_t* label, int* counts) {
-  k_pcg_count<<<pcg_tiles(g), 256, 0, s>>>(g, label, counts);
+  k_pcg_count<false><<<pcg_tiles(g), 256, 0, s>>>(g, label, counts);
 }
 void launch_pcg_fill(hipStream_t s, const Geom& g, const uint8_t* label, const int* counts,
-                     int* offsets, int* n_fluid, int* index_of, int* cell_of, const float* uf, const float* vf, float* b,
-                     float* rhs, uint8_t* info) {
+                     int* offsets, int* n_fluid, int* index_of, int* cell_of, const float* uf,
+                     const float* vf, float* b, float* rhs, uint8_t* info, bool scanned) {
   const int nb = pcg_tiles(g);
-  if (nb <= kPcgScanTiles) {
-    k_pcg_fill<true><<<nb, 256, 0, s>>>(g, label, counts, n_fluid, index_of, cell_of, uf, vf, b,
-                                        rhs, info);
+  if (nb <= kPcgScanTiles && !scanned) {
+    k_pcg_fill<true, false><<<nb, 256, 0, s>>>(g, label, counts, n_fluid, index_of, cell_of, uf,
+                                               vf, b, rhs, info);
     return;
   }
+  if (!scanned) launch_scan_counts(s, nb, counts, offsets, n_fluid);
+  k_pcg_fill<false, false><<<nb, 256, 0, s>>>(g, label, offsets, n_fluid, index_of, cell_of, uf,
+                                              vf, b, rhs, info);
+}
+void launch_pcg_rows(hipStream_t s, const Geom& g, const uint8_t* label, int* counts, int* offsets,
+                     int* n_fluid, int* index_of, int* cell_of, const float* uf, const float* vf,
+                     float* b, float* rhs, uint8_t* info) {
+  const int nb = (g.nx * g.ny + 1023) / 1024;  // at most pcg_tiles(g)
+  k_pcg_count<true><<<nb, 256, 0, s>>>(g, label, counts);
   launch_scan_counts(s, nb, counts, offsets, n_fluid);
-  k_pcg_fill<false><<<nb, 256, 0, s>>>(g, label, offsets, n_fluid, index_of, cell_of, uf, vf, b,
-                                       rhs, info);
+  k_pcg_fill<false, true><<<nb, 256, 0, s>>>(g, label, offsets, n_fluid, index_of, cell_of, uf, vf,
+                                             b, rhs, info);
 }
 
 size_t pcg_lds_bytes(int F, int grid, int nx) {

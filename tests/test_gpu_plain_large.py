@@ -1,0 +1,42 @@
+"""The plain form on grids of more cells than one launch takes unknowns, where the order of
+the unknowns is chosen by their number: none, one block's, several blocks', and more than one
+launch takes."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from fluid_simulation_amd import fsg
+
+from test_gpu_pcg import _cg, _system
+
+pytestmark = pytest.mark.gpu
+
+NX, NY = 1300, 1000
+
+
+@pytest.mark.parametrize("n", [0, 700, 33000, 1 << 20, (1 << 20) + 1])
+def test_truncated_iterate(n):
+    """After 20 iterations, as test_gpu_pcg's: 1e-4 against FP64."""
+    lab, u, v = _system(NX, NY, n, 5)
+    liq = lab == fsg.LIQUID
+    d = fsg.Domain(NX, NY, NX, NY, 0.01, 0.05)
+    d.set_params(solver=fsg.SOLVER_PLAIN, cg_tol=1e-6, cg_max_iter=20)
+    # a solve of another system before it: nothing of it may be left
+    other, _, _ = _system(NX, NY, 40000, 6)
+    d.set_labels(other)
+    d.set_velocity(v, u)
+    d.run_phase("PRESSURE", 0.01)
+    d.set_labels(lab)
+    d.set_velocity(u, v)
+    d.run_phase("PRESSURE", 0.01)
+    st, b, p = d.stats(), d.rhs(), d.pressure()
+    assert st.n_fluid == n == int(liq.sum())
+    assert np.array_equal(d.fluid_indices()[liq], np.arange(n))
+    assert (d.fluid_indices()[~liq] == -1).all()
+    div = (np.append(u, np.zeros((NY, 1), np.float32), 1)[:, 1:] - u) + \
+        (np.append(v, np.zeros((1, NX), np.float32), 0)[1:] - v)
+    assert np.array_equal(b, np.where(liq, div, np.float32(0)))
+    want = _cg(lab, b, 20, 1e-6) if n else np.zeros((NY, NX))
+    assert np.abs(p - want).max() <= 1e-4 * np.abs(want).max()
+    d.close()
