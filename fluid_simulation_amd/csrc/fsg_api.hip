@@ -241,9 +241,11 @@ struct fsg_domain {
   double* partials = nullptr;
   unsigned* bar = nullptr;  // [1]: a one-launch CG solve abandoned a wait
   CgScalars* sc = nullptr;
-  bool last_dev = false;    // the last solve's statistics are in sc (a one-launch CG form)
-  bool dev_totals = false;  // sc holds totals of such solves (since the last reset)
-  HostScalars* hsc = nullptr;  // pinned host memory: the solve loop's readback
+  HostScalars* hsc = nullptr;  // pinned host memory: the solves' scalars (read_scalars)
+  // A one-launch CG solve leaves its statistics in sc and adds to the totals there: what of
+  // them the host has not read, and the totals as it read them last.
+  bool last_unread = false, totals_unread = false;
+  int64_t dev_unknown_iterations = 0, dev_solves = 0;
   // pinned host memory between the device and the caller's arrays (copy_out), allocated by
   // the first large copy: a ring of chunks, an event each
   char* stage = nullptr;
@@ -269,7 +271,8 @@ struct fsg_domain {
   int mg_last_iters_adj = 0;  // and of the last adjoint solve (a different system)
   int mg_prev_iters = 0;      // the same for the solves before those
   int mg_prev_iters_adj = 0;
-  // host-side statistics of the plain solver
+  // the last solve's statistics (but see last_unread), the totals of the solves that add
+  // theirs on the host
   fsg_stats host_stats{};
   std::string err;
   Timer timer;
@@ -731,6 +734,21 @@ void alloc_clk_span(fsg_domain* h) {
     m.clk_span_cap = kSpanLaunches;
 }
 
+// sc (into hs, and its totals) and, if asked for, n_fluid and bar[1], once the stream's work
+// so far is done.
+int read_scalars(fsg_domain* h, bool n_fluid, bool abort, CgScalars& hs) {
+  if (!h->hsc)
+    HIPCHK(h, hipHostMalloc((void**)&h->hsc, sizeof(HostScalars), hipHostMallocCoherent));
+  launch_read_scalars(h->stream, h->sc, n_fluid ? h->n_fluid : nullptr,
+                      abort ? h->bar + 1 : nullptr, h->hsc);
+  HIPCHK(h, hipStreamSynchronize(h->stream));
+  memcpy(&hs, &h->hsc->sc, sizeof(hs));
+  h->dev_unknown_iterations = (int64_t)hs.total_unknown_iters;
+  h->dev_solves = hs.total_solves;
+  h->totals_unread = false;
+  return FSG_OK;
+}
+
 // F < 0: the number of unknowns is still on the device (h->n_fluid); it is read back
 // with the stop-test copy, so the solve costs no extra host round trip.
 // defer_finish: the caller's pressure update does the finish (MgFinishFuse) where it can
@@ -873,11 +891,7 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
     return FSG_OK;
   };
   auto read_back = [&]() -> int {
-    if (!h->hsc)
-      HIPCHK(h, hipHostMalloc((void**)&h->hsc, sizeof(HostScalars), hipHostMallocCoherent));
-    launch_read_scalars(h->stream, h->sc, F < 0 ? h->n_fluid : nullptr, h->hsc);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    memcpy(&hs, &h->hsc->sc, sizeof(hs));
+    if (int rc = read_scalars(h, F < 0, false, hs)) return rc;
     if (F < 0) F = h->hsc->n_fluid;
     if (hs.stuck) return fail(h, FSG_E_HIP, "multigrid solver: a wait on the device ran out");
     return FSG_OK;
@@ -994,13 +1008,15 @@ int plain_many_launches(fsg_domain* h, int F, const CgParams& cp) {
   h->host_stats.cg_error = hs.err;
   h->host_stats.total_unknown_iterations += (int64_t)F * hs.spmv;
   h->host_stats.total_solves += 1;
-  h->last_dev = false;
+  h->dev_unknown_iterations = (int64_t)hs.total_unknown_iters;
+  h->dev_solves = hs.total_solves;
+  h->totals_unread = false;
   return FSG_OK;
 }
 
 int solve_pressure(fsg_domain* h) {
   h->mg_solved = false;
-  h->last_dev = false;
+  h->last_unread = false;
   h->host_stats.cg_iterations = 0;
   h->host_stats.cg_error = 0.0;
   h->host_stats.refine_sweeps = 0;
@@ -1103,25 +1119,27 @@ int solve_pressure(fsg_domain* h) {
         [&] { e = launch_pcg(h->stream, a, grid, kpt); });
   h->last_grid = grid;
   h->last_kpt = kpt;
-  h->last_dev = h->dev_totals = true;
   if (plain && grid > 1) {
     // a cooperative launch that was refused, or gave up a wait, is solved again the way
     // that needs no co-resident blocks
-    unsigned gave_up = 0;
-    if (e == hipSuccess) {
-      HIPCHK(h, hipMemcpyAsync(&gave_up, h->bar + 1, sizeof(gave_up), hipMemcpyDeviceToHost,
-                               h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-    } else {
+    CgScalars hs{};
+    bool gave_up = e != hipSuccess;
+    if (gave_up) {
       (void)hipGetLastError();
+    } else {
+      if (int rc = read_scalars(h, false, true, hs)) return rc;
+      gave_up = h->hsc->abort != 0;
     }
-    if (e != hipSuccess || gave_up) {
+    if (gave_up) {
       launch_fill(h->stream, reinterpret_cast<float*>(h->bar), 4, 0.f);
       return plain_many_launches(h, F, a.cp);
     }
+    h->host_stats.cg_iterations = hs.iter;
+    h->host_stats.cg_error = hs.err;
     return FSG_OK;
   }
   HIPCHK(h, e);
+  h->last_unread = h->totals_unread = true;
   return FSG_OK;
 }
 
@@ -1438,15 +1456,15 @@ int fsg_get_geometry(const fsg_domain* h, int32_t* nx, int32_t* ny, float* dx, f
   return FSG_OK;
 }
 
-// The persistent solver raises bar[1] when a block abandons a grid-barrier wait
-// (bounded spin); every block then leaves the kernel and the solution is invalid.
+// A one-launch solve raises bar[1] when a block abandons a wait (bounded spin); every block
+// then leaves the kernel and the solution is invalid.
+static const char kSolverAbortMsg[] =
+    "persistent pressure solver abandoned a wait: results are invalid";
 static int check_solver_abort(fsg_domain* h) {
   unsigned flag = 0;
   HIPCHK(h, hipMemcpyAsync(&flag, h->bar + 1, sizeof(flag), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
-  if (flag)
-    return fail(h, FSG_E_HIP,
-                "persistent pressure solver abandoned a grid-barrier wait: results are invalid");
+  if (flag) return fail(h, FSG_E_HIP, kSolverAbortMsg);
   return FSG_OK;
 }
 
@@ -1828,34 +1846,32 @@ int fsg_get_reject_flags(fsg_domain* h, uint8_t* flags) {
   return copy_out(h, {{flags, h->reject, (size_t)h->np}});
 }
 
+// Reads what the host has not seen of the one-launch solves' statistics.
+static int pull_stats(fsg_domain* h) {
+  if (!h->last_unread && !h->totals_unread) return FSG_OK;
+  CgScalars hs{};
+  if (int rc = read_scalars(h, true, true, hs)) return rc;
+  if (h->last_unread) {
+    if (h->hsc->abort) return fail(h, FSG_E_HIP, kSolverAbortMsg);
+    h->host_stats.n_fluid = h->hsc->n_fluid;
+    h->host_stats.cg_iterations = hs.iter;
+    h->host_stats.cg_error = hs.err;
+    h->host_stats.refine_sweeps = hs.refine_sweeps;
+  }
+  h->last_unread = false;
+  return FSG_OK;
+}
+
 int fsg_get_stats(fsg_domain* h, fsg_stats* s) {
   if (!h || !s) return FSG_E_INVALID;
-  // the multigrid form and the many-launch plain form keep their statistics on the host
-  // (read with their stop tests): no device access, no synchronisation
-  const bool one_launch =
-      h->prm.solver == FSG_SOLVER_PERSISTENT || h->prm.solver == FSG_SOLVER_REFINED;
-  if (!one_launch && !h->last_dev && !h->dev_totals) {
-    *s = h->host_stats;
-    return FSG_OK;
-  }
-  if (int rc = check_solver_abort(h)) return rc;
-  CgScalars hs{};
-  int F = 0;
-  HIPCHK(h, hipMemcpyAsync(&hs, h->sc, sizeof(hs), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipMemcpyAsync(&F, h->n_fluid, sizeof(int), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  if (one_launch)
-    memset(s, 0, sizeof(*s));
-  else
-    *s = h->host_stats;
-  if (one_launch || h->last_dev) {
-    s->n_fluid = F;
-    s->cg_iterations = hs.iter;
-    s->cg_error = hs.err;
-    s->refine_sweeps = hs.refine_sweeps;
-  }
-  s->total_unknown_iterations = (int64_t)hs.total_unknown_iters + h->host_stats.total_unknown_iterations;
-  s->total_solves = hs.total_solves + h->host_stats.total_solves;
+  // no device access and no synchronisation unless the last solve was one that the host has
+  // not waited for (the persistent and refined forms, the plain form's one-block solves)
+  if (int rc = pull_stats(h)) return rc;
+  *s = h->host_stats;
+  if (h->prm.solver == FSG_SOLVER_PERSISTENT || h->prm.solver == FSG_SOLVER_REFINED)
+    s->mg_live_tiles = 0;
+  s->total_unknown_iterations += h->dev_unknown_iterations;
+  s->total_solves += h->dev_solves;
   return FSG_OK;
 }
 
@@ -1871,7 +1887,8 @@ int fsg_reset_stats(fsg_domain* h) {
   HIPCHK(h, hipStreamSynchronize(h->stream));
   h->host_stats.total_unknown_iterations = 0;
   h->host_stats.total_solves = 0;
-  h->dev_totals = false;
+  h->dev_unknown_iterations = h->dev_solves = 0;
+  h->totals_unread = false;
   return FSG_OK;
 }
 
@@ -2341,6 +2358,7 @@ int fsg_autotune(fsg_domain* h, int32_t scheme, float dt, int32_t steps, fsg_tun
             for (int nt : {256, 512}) cands.push_back({ls[0], ls[1], co, fu, gi, so, nt});
   TuneState saved;
   if (int rc = tune_save(h, saved)) return rc;
+  (void)pull_stats(h);  // an abandoned solve has no statistics to keep
   const fsg_stats stats0 = h->host_stats;
   const int last0 = h->mg_last_iters, prev0 = h->mg_prev_iters;
   HIPCHK(h, hipStreamSynchronize(h->stream));

@@ -186,16 +186,16 @@ struct CgScalars {
   int pad_;
 };
 
-// The scalars a solve's host loop reads back after each batch of iterations, written by
+// The scalars that the host reads back after a batch of iterations or a solve, written by
 // one small kernel into pinned host memory (one launch instead of two device-to-host
-// copies).  n_fluid is -1 when not asked for.
+// copies).  n_fluid is -1 and abort 0 when not asked for.
 struct HostScalars {
   CgScalars sc;
   int n_fluid;
-  int pad;
+  unsigned abort;
 };
 void launch_read_scalars(hipStream_t s, const CgScalars* sc, const int* n_fluid,
-                         HostScalars* out);
+                         const unsigned* abort, HostScalars* out);
 
 struct CgParams {
   int max_iter;

@@ -3771,17 +3771,19 @@ void launch_mg_remove_mean(hipStream_t s, const MgHost& m) {
 
 __global__ void __launch_bounds__(64) k_read_scalars(const CgScalars* __restrict__ sc,
                                                     const int* __restrict__ n_fluid,
+                                                    const unsigned* __restrict__ abort,
                                                     HostScalars* __restrict__ out) {
   constexpr int kW = (int)(sizeof(CgScalars) / 4);
-  static_assert(sizeof(CgScalars) % 4 == 0 && kW < 64, "one word per lane");
+  static_assert(sizeof(CgScalars) % 4 == 0 && kW <= 62, "one word per lane");
   const int t = threadIdx.x;
   if (t < kW) reinterpret_cast<int*>(&out->sc)[t] = reinterpret_cast<const int*>(sc)[t];
+  if (t == 62) out->abort = abort ? *abort : 0u;
   if (t == 63) out->n_fluid = n_fluid ? *n_fluid : -1;
   __threadfence_system();
 }
 void launch_read_scalars(hipStream_t s, const CgScalars* sc, const int* n_fluid,
-                         HostScalars* out) {
-  k_read_scalars<<<1, 64, 0, s>>>(sc, n_fluid, out);
+                         const unsigned* abort, HostScalars* out) {
+  k_read_scalars<<<1, 64, 0, s>>>(sc, n_fluid, abort, out);
 }
 
 void launch_mg_finish(hipStream_t s, const MgHost& m, int project_mean, CgScalars* sc,
