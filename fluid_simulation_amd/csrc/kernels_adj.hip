@@ -15,6 +15,8 @@
 // The buffer a step starts with as its front is overwritten before it is read (the
 // extension init writes every back face), so only the back buffer and the particles
 // carry adjoints between steps.
+#include <type_traits>
+
 #include "fsg_kernels.h"
 
 namespace fsg {
@@ -446,10 +448,11 @@ __global__ void __launch_bounds__(kAT) k_adj_p2g(Geom g, const float4* __restric
 // y / dy) with Grid::addToValueInterpolated's weights.
 // FX: the terms are added as 64-bit fixed-point integers (fx_term) into rho_fx, so
 // the density does not depend on the order of the atomics (fsg_params.deterministic).
-// The terms go to an LDS copy of the block's footprint where that fits (as the splat's; four
-// terms in [0, 1] per particle, so 256 particles' sums are far from the fixed point's range),
-// then one atomic per touched cell: 1,040,000 particles near their storage order on 512^2
-// cells 177 -> 18.6 us, fixed-point sums.
+// The terms go to an LDS copy of the block's footprint where that fits (as the splat's), then
+// one atomic per touched cell: 1,040,000 particles near their storage order on 512^2 cells
+// 177 -> 18.6 us, fixed-point sums.  The float form sums in FP64 there: any position's terms,
+// and weights down to 2^-46, which 2^-40 fixed point loses (13.0 us in fixed point, 13.3 in
+// FP64; with every cell holding 40 particles 14.2 and 16.2).
 constexpr int kDensityTile = 2048;
 template <bool FX>
 __global__ void __launch_bounds__(kAT) k_density(Geom g, const float4* __restrict__ pt,
@@ -459,14 +462,11 @@ __global__ void __launch_bounds__(kAT) k_density(Geom g, const float4* __restric
   const bool live = p < np;
   const float4 q = live ? pt[p] : make_float4(0.f, 0.f, 0.f, 0.f);
   const SplatCorners s = splat_corners(div_x(q.x, g), div_y(q.y, g), g.nx, g.ny);
-  __shared__ unsigned long long s_tile[kDensityTile];
+  using Sum = std::conditional_t<FX, unsigned long long, double>;
+  __shared__ Sum s_tile[kDensityTile];
   const Box box = block_box(live, s.i, s.j, s.i1, s.j1);
   const int bw = box.i1 - box.i0 + 1, bh = box.j1 - box.j0 + 1;
-  bool tiled = bw > 0 && bh > 0 && (int64_t)bw * bh <= kDensityTile;
-  // a position far outside the grid or not a number has weights the fixed point cannot hold:
-  // the float sums take them as they are (block-uniform)
-  if (!FX && tiled)
-    tiled = !__syncthreads_or(live && !(fabsf(s.fi) <= 1.0f && fabsf(s.fj) <= 1.0f));
+  const bool tiled = bw > 0 && bh > 0 && (int64_t)bw * bh <= kDensityTile;
   if (!tiled) {
     if (live)
       splat_terms2(s, 1.0f, [&](int i, int j, float t) {
@@ -478,21 +478,25 @@ __global__ void __launch_bounds__(kAT) k_density(Geom g, const float4* __restric
     return;
   }
   const int area = bw * bh;
-  for (int c = threadIdx.x; c < area; c += kAT) s_tile[c] = 0ull;
+  for (int c = threadIdx.x; c < area; c += kAT) s_tile[c] = Sum(0);
   __syncthreads();
   if (live)
     splat_terms2(s, 1.0f, [&](int i, int j, float t) {
-      atomicAdd(s_tile + (i - box.i0) + (j - box.j0) * bw, (unsigned long long)fx_term(t));
+      Sum* const dst = s_tile + (i - box.i0) + (j - box.j0) * bw;
+      if constexpr (FX)
+        atomicAdd(dst, (Sum)fx_term(t));
+      else
+        __hip_atomic_fetch_add(dst, (Sum)t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     });
   __syncthreads();
   for (int c = threadIdx.x; c < area; c += kAT) {
-    const unsigned long long v = s_tile[c];
-    if (v == 0ull) continue;
+    const Sum v = s_tile[c];
+    if (v == Sum(0)) continue;
     const int cell = (box.i0 + c % bw) + (box.j0 + c / bw) * g.nx;
-    if (FX)
+    if constexpr (FX)
       atomicAdd(rho_fx + cell, v);
     else
-      unsafeAtomicAdd(&rho[cell], fx_value((long long)v));
+      unsafeAtomicAdd(&rho[cell], (float)v);
   }
 }
 
