@@ -2618,7 +2618,7 @@ __global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk,
   extern __shared__ float lds[];
   __shared__ double sm[kCycNT / 64];
   __shared__ unsigned long long s_ticket;
-  __shared__ int s_stop;
+  __shared__ int s_done, s_stop;  // a finished solve; the stop test's result (stopped)
   // the counter: the launch's number and the next task.  Every workgroup draws one; the one
   // with the last task sets the counter for the next launch.
   unsigned long long ticket = 0;
@@ -2629,14 +2629,14 @@ __global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk,
     done = __hip_atomic_load(&chk.sc->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   if (threadIdx.x == 0) {
     s_ticket = ticket;
-    s_stop = done;
+    s_done = done;
   }
   __syncthreads();
   const unsigned task = __builtin_amdgcn_readfirstlane((unsigned)s_ticket);
   const unsigned launch = __builtin_amdgcn_readfirstlane((unsigned)(s_ticket >> 32));
   if (task == a.n_tasks - 1 && threadIdx.x == 0)
     st_dev(a.ticket, (unsigned long long)(launch + 1) << 32);
-  if (s_stop) return;
+  if (s_done) return;
   const unsigned tag = launch + 1;  // the words start out as zero
   if (task == 0) {  // the stop test, for all
     if (check) {
