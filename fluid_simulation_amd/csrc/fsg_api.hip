@@ -254,6 +254,7 @@ struct fsg_domain {
   int max_coop_blocks = 0;  // co-resident 1024-thread blocks of the persistent solver
   size_t pcg_lds_max = 0;   // dynamic LDS the persistent solver may use per block
   int last_F = 0, last_grid = 0, last_kpt = 0;
+  int spin_max = 0;         // fsg_test_spin_max, 0: the solvers' own
   // multigrid form: hierarchy allocated on first use; iterations of the last solve
   MgHost mg{};
   BatchInfo* batch = nullptr;  // packed batch of scenes (fsg_batch_create), else null
@@ -771,6 +772,7 @@ int mg_solve(fsg_domain* h, int F, const double* adj_rhs = nullptr, bool defer_f
   m.l0_threads = h->prm.mg_tile_threads;
   m.level_sweeps = h->prm.mg_level_sweeps;
   m.level0_sweeps = h->prm.mg_level0_sweeps;
+  m.cyc.spin_max = h->spin_max > 0 ? h->spin_max : kMgSpins;
   m.tmap = h->prm.mg_spread_tiles ? m.tmap_buf : nullptr;
   m.clk_on = h->kclock == 1;
   m.clk_span_on = h->kclock == 2;
@@ -1106,6 +1108,7 @@ int solve_pressure(fsg_domain* h) {
   a.x64 = h->x64;
   a.slots = reinterpret_cast<uint64_t*>(h->partials);
   a.abort = h->bar + 1;
+  a.spin_max = (unsigned)(h->spin_max > 0 ? h->spin_max : kPcgSpins);
   a.sc = h->sc;
   a.refined = refined;
   a.cp = make_cg_params(h, refined ? (float)h->prm.refine_inner_tol : (float)h->prm.cg_tol);
@@ -1465,6 +1468,15 @@ static int check_solver_abort(fsg_domain* h) {
   HIPCHK(h, hipMemcpyAsync(&flag, h->bar + 1, sizeof(flag), hipMemcpyDeviceToHost, h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
   if (flag) return fail(h, FSG_E_HIP, kSolverAbortMsg);
+  return FSG_OK;
+}
+
+// For tests of what follows a wait between workgroups that runs out (not in fsg.h): the polls
+// after which the pressure solvers give one up, 0 for their own bound.
+int fsg_test_spin_max(fsg_domain* h, int32_t polls) {
+  if (!h || polls < 0) return FSG_E_INVALID;
+  h->spin_max = polls;
+  h->mg_graphs.clear();  // the captured launches hold it
   return FSG_OK;
 }
 

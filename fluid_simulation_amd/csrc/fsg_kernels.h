@@ -235,6 +235,8 @@ void launch_cg_iteration(hipStream_t s, int F, int nx, int it, const CgParams& c
 constexpr int kPcgOneUnknowns = 8192;  // the most unknowns that one block solves (FP32 form)
 constexpr int kPcgOneRefined = 4096;   // and in the refined form
 constexpr int kPcgMaxBlocks = 256;     // blocks of a solve: four waves read their sums
+// a wait of seconds between workgroups is treated as a fault
+constexpr int kPcgSpins = 1 << 22, kMgSpins = 1 << 20;
 struct PersistentArgs {
   int nx;
   int F_actual;          // unknowns of this solve, or a bound of them (sizes the launch)
@@ -248,6 +250,7 @@ struct PersistentArgs {
   double* x64;           // F_actual doubles: FP64 solution exchange (refined form)
   uint64_t* slots;       // pcg_slot_words(grid): the blocks' partial sums, tagged
   unsigned* abort;       // set when a block gave up waiting
+  unsigned spin_max;     // polls after which it does
   CgScalars* sc;
   CgParams cp;
   int refined;
@@ -307,6 +310,7 @@ struct MgCycleArgs {
   unsigned long long* ticket = nullptr;  // the launch's number (high half), the next task
   unsigned* flag = nullptr;              // the stop test's result (twice the launch + 0 or 1)
   unsigned* hint = nullptr;              // per task: the launch in which it last finished
+  int spin_max = kMgSpins;               // polls after which a task gives up a wait
   MgCycleLevel lv[kMgMaxLevels];
 };
 

@@ -2376,10 +2376,13 @@ __global__ void __launch_bounds__(kCoarseThreads) k_mg_scene_coarse(SceneCoarseA
 // two steps ahead of it in the chain with one thread, so that the idle tasks' polls do not
 // crowd out the others' loads.
 //
-// Waits are bounded all the same (kSpinMax polls of about a microsecond): one that runs out
-// marks the solve as failed instead of keeping the device busy for good.
+// Waits are bounded all the same (MgCycleArgs::spin_max polls of about a microsecond): one
+// that runs out marks the solve as failed instead of keeping the device busy for good.
 constexpr int kCycNT = 1024;
-constexpr int kSpinMax = 1 << 20;
+struct CycleWait {
+  int* stuck;
+  int most;  // polls
+};
 
 __device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
   return ((unsigned long long)tag << 32) | __float_as_uint(v);
@@ -2392,7 +2395,7 @@ __device__ __forceinline__ float untag(unsigned long long w) {
 // (Without need p[k] is still read: it points to any word.)
 template <int N>
 __device__ __forceinline__ void wait_tagged(const unsigned long long* const (&p)[N],
-                                            const bool (&need)[N], unsigned tag, int* stuck,
+                                            const bool (&need)[N], unsigned tag, const CycleWait& wait,
                                             float (&v)[N]) {
   unsigned long long w[N];
   for (int n = 0;; ++n) {
@@ -2402,8 +2405,8 @@ __device__ __forceinline__ void wait_tagged(const unsigned long long* const (&p)
 #pragma unroll
     for (int k = 0; k < N; ++k) ok &= !need[k] || (unsigned)(w[k] >> 32) == tag;
     if (ok) break;
-    if (n == kSpinMax) {
-      st_dev(stuck, 1);
+    if (n >= wait.most) {
+      st_dev(wait.stuck, 1);
       break;
     }
     __builtin_amdgcn_s_sleep(1);
@@ -2418,11 +2421,11 @@ __device__ __forceinline__ void wait_tagged(const unsigned long long* const (&p)
 constexpr int kHintPitch = 32;
 constexpr int kFlags = 32;  // copies of the stop test's result, a line each
 __device__ __forceinline__ void wait_hint(const unsigned* hint, int task, unsigned tag,
-                                          int* stuck) {
+                                          const CycleWait& wait) {
   if (threadIdx.x == 0)
     for (int n = 0; ld_dev(hint + task * kHintPitch) != tag; ++n) {
-      if (n == kSpinMax) {
-        st_dev(stuck, 1);
+      if (n >= wait.most) {
+        st_dev(wait.stuck, 1);
         break;
       }
       __builtin_amdgcn_s_sleep(4);
@@ -2432,7 +2435,7 @@ __device__ __forceinline__ void wait_hint(const unsigned* hint, int task, unsign
 
 template <int S, class Stopped>
 __device__ __forceinline__ void cycle_down(const MgCycleArgs& a, int k, int tile, unsigned tag,
-                                           const float (&wk)[kMgMaxSweeps], int* stuck,
+                                           const float (&wk)[kMgMaxSweeps], const CycleWait& wait,
                                            float* lds, Stopped&& stopped) {
   constexpr int NT = kCycNT, W = 34 + 2 * S, WC = kDownWC;
   using St = Strip<W, NT>;
@@ -2471,7 +2474,7 @@ __device__ __forceinline__ void cycle_down(const MgCycleArgs& a, int k, int tile
   if (k > 0) {
     if (k >= 2) {
       const MgCycleLevel g = a.lv[k - 2];
-      wait_hint(a.hint, g.down0 + 4 * bx + 4 * by * g.tiles_x, tag, stuck);
+      wait_hint(a.hint, g.down0 + 4 * bx + 4 * by * g.tiles_x, tag, wait);
     }
     const unsigned long long* p[R];
     bool need[R];
@@ -2480,7 +2483,7 @@ __device__ __forceinline__ void cycle_down(const MgCycleArgs& a, int k, int tile
       p[q] = f.tr + ts.cell[q];
       need[q] = is_act(fv[q]);
     }
-    wait_tagged<R>(p, need, tag, stuck, rv);
+    wait_tagged<R>(p, need, tag, wait, rv);
   }
   if (threadIdx.x < WC * WC) s_cinf[threadIdx.x] = cv;
   down_core<NT, S>(ts, fv, rv, wk, s_x0, s_x1, s_cinf, bx, by, c.nx, c.ny,
@@ -2491,7 +2494,7 @@ __device__ __forceinline__ void cycle_down(const MgCycleArgs& a, int k, int tile
 
 template <int S, class Stopped>
 __device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, unsigned tag,
-                                         int it, const float (&wk)[kMgMaxSweeps], int* stuck,
+                                         int it, const float (&wk)[kMgMaxSweeps], const CycleWait& wait,
                                          float* lds, Stopped&& stopped) {
   constexpr int NT = kCycNT, W = 32 + 2 * S, WC = UpFrame<S>::WC, CO = UpFrame<S>::CO;
   using St = Strip<W, NT>;
@@ -2531,7 +2534,7 @@ __device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, 
   }
   // the level's own values on the way down once the tile's task is done (its neighbours'
   // follow soon), then the coarse result
-  wait_hint(a.hint, f.down0 + tile, tag, stuck);
+  wait_hint(a.hint, f.down0 + tile, tag, wait);
   {
     const unsigned long long* p[2 * R];
     bool need[2 * R];
@@ -2543,7 +2546,7 @@ __device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, 
       p[R + q] = k == 0 ? p[q] : f.tr + ts.cell[q];
       need[R + q] = need[q];
     }
-    wait_tagged<2 * R>(p, need, tag, stuck, v);
+    wait_tagged<2 * R>(p, need, tag, wait, v);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       x[q] = v[q];
@@ -2552,16 +2555,16 @@ __device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, 
   }
   if (k + 2 < a.nl) {
     const MgCycleLevel g = a.lv[k + 2];
-    wait_hint(a.hint, g.up0 + (bx >> 2) + (by >> 2) * g.tiles_x, tag, stuck);
+    wait_hint(a.hint, g.up0 + (bx >> 2) + (by >> 2) * g.tiles_x, tag, wait);
   } else {
     const int sh = a.nl - 1 - k;
     const MgCycleLevel g = a.lv[a.nl - 1];
-    wait_hint(a.hint, g.down0 + (bx >> sh) + (by >> sh) * g.tiles_x, tag, stuck);
+    wait_hint(a.hint, g.down0 + (bx >> sh) + (by >> sh) * g.tiles_x, tag, wait);
   }
   const unsigned long long* const pe[1] = {c.te + ce};
   const bool ne[1] = {is_act(cv)};
   float ev[1];
-  wait_tagged<1>(pe, ne, tag, stuck, ev);
+  wait_tagged<1>(pe, ne, tag, wait, ev);
   if (threadIdx.x < WC * WC) {
     s_e[threadIdx.x] = ev[0];
     s_cinf[threadIdx.x] = cv;
@@ -2582,20 +2585,20 @@ __device__ __forceinline__ void cycle_up(const MgCycleArgs& a, int k, int tile, 
 // The one-workgroup stage of one domain, and of scene `s` of a batch (the cells of its
 // rectangle of the packed level, cells outside every rectangle hold no unknown).
 __device__ __forceinline__ void cycle_coarse(const MgCoarseArgs& a, const MgCycleLevel& f,
-                                             unsigned tag, int* stuck, float* lds) {
+                                             unsigned tag, const CycleWait& wait, float* lds) {
   __shared__ int s_lv[3 * kMgMaxLevels];
   const int n = f.nx * f.ny;
   coarse_run<kCycNT>(
       a, lds, s_lv,
       [&](const bool (&act)[1], float (&r)[1]) {
         const unsigned long long* const p[1] = {f.tr + (threadIdx.x < n ? threadIdx.x : 0)};
-        wait_tagged<1>(p, act, tag, stuck, r);
+        wait_tagged<1>(p, act, tag, wait, r);
       },
       [&](float, float x) { st_dev(f.te + threadIdx.x, tagged(x, tag)); });
 }
 
 __device__ __forceinline__ void cycle_scene(const SceneCoarseArgs& a, const MgCycleLevel& f,
-                                            int scene, unsigned tag, int* stuck, float* lds) {
+                                            int scene, unsigned tag, const CycleWait& wait, float* lds) {
   static_assert(kCycNT == kCoarseThreads, "the stage's workgroup");
   scene_run(
       a, scene, lds,
@@ -2603,7 +2606,7 @@ __device__ __forceinline__ void cycle_scene(const SceneCoarseArgs& a, const MgCy
         const unsigned long long* p[kSceneK];
 #pragma unroll
         for (int k = 0; k < kSceneK; ++k) p[k] = f.tr + cell[k];
-        wait_tagged<kSceneK>(p, act, tag, stuck, r);
+        wait_tagged<kSceneK>(p, act, tag, wait, r);
       },
       [&](int cell, float x) { st_dev(f.te + cell, tagged(x, tag)); });
 }
@@ -2645,7 +2648,7 @@ __global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk,
     }
     return;
   }
-  int* const stuck = &chk.sc->stuck;
+  const CycleWait wait{&chk.sc->stuck, a.spin_max};
   // (a task calls it when its first loads are under way, all threads alike)
   auto stopped = [&]() __attribute__((always_inline)) {
     if (!check) return false;
@@ -2653,8 +2656,8 @@ __global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk,
       const unsigned* const flag = a.flag + (task % kFlags) * kHintPitch;
       unsigned w = ld_dev(flag);
       for (int n = 0; (w >> 1) != (tag & 0x7fffffffu); w = ld_dev(flag)) {
-        if (++n == kSpinMax) {
-          st_dev(stuck, 1);
+        if (++n > wait.most) {
+          st_dev(wait.stuck, 1);
           break;
         }
         __builtin_amdgcn_s_sleep(1);
@@ -2669,17 +2672,17 @@ __global__ void __launch_bounds__(kCycNT) k_mg_cycle(MgCycleArgs a, MgCheck chk,
   if (task < a.coarse0) {
     int k = 0;
     while (k + 1 < a.nl && task >= a.lv[k + 1].down0) ++k;
-    cycle_down<S>(a, k, (int)(task - a.lv[k].down0), tag, wk, stuck, lds, stopped);
+    cycle_down<S>(a, k, (int)(task - a.lv[k].down0), tag, wk, wait, lds, stopped);
   } else if (task < a.up0) {
     if (stopped()) return;
     if constexpr (BATCH)
-      cycle_scene(sa, a.lv[a.nl], (int)(task - a.coarse0), tag, stuck, lds);
+      cycle_scene(sa, a.lv[a.nl], (int)(task - a.coarse0), tag, wait, lds);
     else
-      cycle_coarse(ca, a.lv[a.nl], tag, stuck, lds);
+      cycle_coarse(ca, a.lv[a.nl], tag, wait, lds);
   } else {
     int k = a.nl - 1;
     while (k > 0 && task >= a.lv[k - 1].up0) --k;
-    cycle_up<S>(a, k, (int)(task - a.lv[k].up0), tag, it, wk, stuck, lds, stopped);
+    cycle_up<S>(a, k, (int)(task - a.lv[k].up0), tag, it, wk, wait, lds, stopped);
   }
   if (threadIdx.x == 0) st_dev(a.hint + task * kHintPitch, tag);
 }

@@ -57,7 +57,6 @@ namespace fsg {
 namespace {
 
 constexpr int kPcgThreads = 512;
-constexpr unsigned kSpinLimit = 1u << 22;  // seconds of waiting: treated as a fault
 constexpr int kSlotWords = 4;              // 64-bit words per block and sum: 2 doubles
 
 // Sum over the first 8 lanes of each 16-lane row, in lane 7 of the row.
@@ -87,7 +86,8 @@ struct PcgNet {
   uint64_t* slots;  // [2][G][kSlotWords]
   uint64_t* z;      // one word per unknown: z of the unknowns in some block's halo
   unsigned* abort;
-  uint32_t epoch;   // sums so far; the tag of the last one
+  unsigned spin_max;  // polls of a wait, at most
+  uint32_t epoch;     // sums so far; the tag of the last one
 };
 
 struct PcgShared {
@@ -100,7 +100,7 @@ struct PcgShared {
 // Polls a thread's N words until each carries the tag (at(q): word q, null for none);
 // false when the wait was abandoned.  All loads of a round are in flight together.
 template <int N, typename At>
-__device__ __forceinline__ bool poll(At&& at, uint32_t tag, uint64_t (&w)[N], unsigned* abort) {
+__device__ __forceinline__ bool poll(At&& at, uint32_t tag, uint64_t (&w)[N], const PcgNet& net) {
   for (unsigned spins = 0;; ++spins) {
     bool good = true;
 #pragma unroll
@@ -111,11 +111,11 @@ __device__ __forceinline__ bool poll(At&& at, uint32_t tag, uint64_t (&w)[N], un
 #pragma unroll
     for (int q = 0; q < N; ++q) good &= tag_of(w[q]) == tag;
     if (good) return true;
-    if (spins > kSpinLimit) {
-      st_dev(abort, 1u);
+    if (spins >= net.spin_max) {
+      st_dev(net.abort, 1u);
       return false;
     }
-    if ((spins & 255u) == 255u && ld_dev(abort)) return false;
+    if ((spins & 255u) == 255u && ld_dev(net.abort)) return false;
   }
 }
 
@@ -165,7 +165,7 @@ __device__ __forceinline__ bool grid_sum(PcgNet& net, double (&v)[NV], PcgShared
       const int b = wave * 64 + lane;
       uint64_t w[2 * NV];
       good = poll([&](int q) { return b < G ? set + (size_t)b * kSlotWords + q : nullptr; }, e, w,
-                  net.abort);
+                  net);
       double t[NV];
 #pragma unroll
       for (int q = 0; q < NV; ++q)
@@ -399,7 +399,7 @@ __device__ __forceinline__ void pcg_solve(const PersistentArgs& a, int F, float*
   }
   __syncthreads();
   const int nh = ONE ? 0 : sh.n_halo;
-  PcgNet net{a.slots, a.zx, a.abort, 0u};
+  PcgNet net{a.slots, a.zx, a.abort, a.spin_max, 0u};
   auto idle = [](int, int) { return true; };
   // z of the halo, published for sum e: four words of a thread in flight at once
   auto stage_halo = [&](int w, int nw) {
@@ -412,7 +412,7 @@ __device__ __forceinline__ void pcg_solve(const PersistentArgs& a, int F, float*
         return t < nh ? net.z + lhq[t] : nullptr;
       };
       uint64_t v[U];
-      good &= poll(at, net.epoch, v, net.abort);
+      good &= poll(at, net.epoch, v, net);
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (t0 + u * n < nh) lzh[t0 + u * n] = __uint_as_float((uint32_t)v[u]);
