@@ -251,8 +251,8 @@ struct fsg_domain {
   char* stage = nullptr;
   hipEvent_t stage_ev[kStageSlots] = {};
   bool mg_finish_pending = false;  // the next pressure update finishes the MG solve
-  int max_coop_blocks = 0;  // co-resident 1024-thread blocks of the persistent solver
-  size_t pcg_lds_max = 0;   // dynamic LDS the persistent solver may use per block
+  int max_coop_blocks = 0;  // co-resident blocks of a one-launch solve, at most
+  size_t pcg_lds_max = 0;   // dynamic LDS that such a block may use
   int last_F = 0, last_grid = 0, last_kpt = 0;
   int spin_max = 0;         // fsg_test_spin_max, 0: the solvers' own
   // multigrid form: hierarchy allocated on first use; iterations of the last solve
@@ -1062,9 +1062,8 @@ int solve_pressure(fsg_domain* h) {
     if (count_first && (size_t)F <= plain_max) timed(h, "pcg_setup", fill);
     if (F == 0) return FSG_OK;
   }
-  // The largest systems: kpt 4 (refined form: 2) on every co-resident block; the
-  // persistent and refined forms also refuse grids whose rows would not leave a block's
-  // unknowns room in an LDS window of the row-major order (pcg_lds_bytes).
+  // The largest systems: 4096 unknowns per co-resident block (the refined form is held to
+  // 2048); the persistent and refined forms also refuse very wide grids (pcg_row_window).
   const int gmax = h->max_coop_blocks;
   const int kfix = plain ? 0 : h->prm.pcg_kpt;
   auto blocks = [&](int k) {
@@ -1076,7 +1075,7 @@ int solve_pressure(fsg_domain* h) {
   for (int k : {1, 2, 4}) {
     if (fits || (kfix > 0 && k != kfix) || (refined && k == 4)) continue;
     fits = blocks(k) <= gmax &&
-           (plain || pcg_lds_bytes(F, std::max(blocks(k), 1), h->g.nx) <= h->pcg_lds_max);
+           (plain || pcg_row_window(F, std::max(blocks(k), 1), h->g.nx) <= h->pcg_lds_max);
   }
   // More than one block: the fewest, since a sum costs what the blocks poll of each other
   // (plain form at 1024^2, 251,000 unknowns: 5.0 / 5.9 / 7.7 us per iteration at kpt
@@ -1089,6 +1088,7 @@ int solve_pressure(fsg_domain* h) {
     kpt = kfix > 0 ? kfix : 4;
     grid = std::max(blocks(kpt), 2);
   }
+  if (grid > 1 && pcg_lds_bytes(F, grid, kpt) > h->pcg_lds_max) kpt = 0;
   if (kpt == 0) {
     if (plain) return plain_many_launches(h, F, make_cg_params(h, (float)h->prm.cg_tol));
     return fail(h, FSG_E_INVALID,

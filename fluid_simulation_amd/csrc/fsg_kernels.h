@@ -261,7 +261,12 @@ struct PersistentArgs {
   int min_iter;          // the solve runs only with cp.max_iter >= min_iter (plain form:
                          // 1, it takes no iteration at max_iter 0; else 0)
 };
-size_t pcg_lds_bytes(int F, int grid, int nx);
+size_t pcg_lds_bytes(int F, int grid, int kpt);  // dynamic LDS per block of launch_pcg
+// What the persistent and refined forms are held to: three windows of a block's unknowns in
+// row-major order, a grid row on either side.  The kernel has no such windows; the bound is
+// that of the systems these forms have always taken (nx up to about 6400), so that a caller
+// who falls back on the refusal meets it where it was.
+size_t pcg_row_window(int F, int grid, int nx);
 size_t pcg_slot_words(int grid);
 // kpt: 1024-unknown units per block.  grid 1: an ordinary launch, F_actual (kpt is not
 // used) at most kPcgOneUnknowns or kPcgOneRefined; more blocks: kpt 1, 2 or 4, a

@@ -676,9 +676,17 @@ void launch_pcg_rows(hipStream_t s, const Geom& g, const uint8_t* label, int* co
                                              b, rhs, info);
 }
 
-size_t pcg_lds_bytes(int F, int grid, int nx) {
+size_t pcg_row_window(int F, int grid, int nx) {
   const int per = (F + grid - 1) / grid;
   return (size_t)3 * (per + 2 * nx) * sizeof(float);
+}
+size_t pcg_lds_bytes(int F, int grid, int kpt) {
+  if (grid == 1) {
+    int cap = kPcgThreads;  // the kernel's unknowns per thread x threads for any number up to F
+    while (cap < F) cap *= 2;
+    return (size_t)(cap + 1) * sizeof(float);
+  }
+  return (size_t)(1 + 1024 * kpt + 3 * pcg_halo_cap((F + grid - 1) / grid)) * sizeof(float);
 }
 size_t pcg_slot_words(int grid) { return (size_t)2 * grid * kSlotWords; }
 
@@ -693,17 +701,14 @@ hipError_t launch_pcg(hipStream_t s, const PersistentArgs& a, int grid, int kpt)
   void* args[] = {(void*)&a};
   const bool ref = a.refined != 0;
   const void* f = nullptr;
+  const size_t lds = pcg_lds_bytes(a.F_actual, grid, kpt);
   if (grid == 1) {
-    int cap = kPcgThreads;  // the kernel's KPT x threads for any F <= F_actual
-    while (cap < a.F_actual) cap *= 2;
-    const size_t lds = (size_t)(cap + 1) * sizeof(float);
     if (a.F_actual > (ref ? kPcgOneRefined : kPcgOneUnknowns)) return hipErrorInvalidValue;
     f = ref ? (const void*)k_pcg_one<8, true> : (const void*)k_pcg_one<16, false>;
     return hipLaunchKernel(f, dim3(1), dim3(kPcgThreads), args, lds, s);
   }
   const int per = (a.F_actual + grid - 1) / grid;
   if (per > 1024 * kpt) return hipErrorInvalidValue;
-  const size_t lds = (size_t)(1 + 1024 * kpt + 3 * pcg_halo_cap(per)) * sizeof(float);
   const int n_slots = (int)pcg_slot_words(grid);
   const int64_t n = std::max<int64_t>(a.F_actual, n_slots);
   k_pcg_clear<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(a.zx, a.F_actual, a.slots, n_slots,

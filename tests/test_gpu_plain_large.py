@@ -40,3 +40,25 @@ def test_truncated_iterate(n):
     want = _cg(lab, b, 20, 1e-6) if n else np.zeros((NY, NX))
     assert np.abs(p - want).max() <= 1e-4 * np.abs(want).max()
     d.close()
+
+
+@pytest.mark.parametrize("nx", [6000, 9000])
+def test_wide_grids(nx):
+    """The plain form takes a wide grid in one launch; the persistent and refined forms refuse
+    the wider one, and solve again afterwards."""
+    ny, n = 20, 30000
+    lab, u, v = _system(nx, ny, n, 9)
+    d = fsg.Domain(nx, ny, nx, ny, 0.01, 0.05)
+    d.set_labels(lab)
+    for solver in (fsg.SOLVER_PERSISTENT, fsg.SOLVER_REFINED, fsg.SOLVER_PLAIN):
+        d.set_params(solver=solver, cg_tol=1e-12, cg_max_iter=20, refine_max_outer=1)
+        d.set_velocity(u, v)
+        if nx == 9000 and solver != fsg.SOLVER_PLAIN:
+            with pytest.raises(fsg.FsgError, match="too large"):
+                d.run_phase("PRESSURE", 0.01)
+            continue
+        d.run_phase("PRESSURE", 0.01)
+        assert d.stats().n_fluid == n
+        want = _cg(lab, d.rhs(), 20, 1e-12)
+        assert np.abs(d.pressure() - want).max() <= 1e-4 * np.abs(want).max()
+    d.close()
