@@ -102,7 +102,7 @@ struct BatchInfo {
   int stage_stride = 0;
   uint8_t* d_sinf = nullptr;
   int stride = 0;
-  // per-scene CG: 64 x 16 vector tiles inside the scenes, and the scalars (5 S doubles)
+  // per-scene CG: 64 x 16 vector tiles inside the scenes, and the scalars (6 S doubles)
   int4* d_vtile = nullptr;
   int2* d_vend = nullptr;  // per vector tile: its scene's column and row ends
   int n_vtile = 0;
@@ -236,7 +236,7 @@ struct fsg_domain {
   float* ap = nullptr;
   float* xg = nullptr;
   float* pg0 = nullptr;
-  float* exch = nullptr;    // 3 C floats: the one-launch CG's tagged words (2 C of them)
+  uint64_t* exch = nullptr; // C words: z across the one-launch CG's blocks, tagged
   double* x64 = nullptr;
   double* partials = nullptr;
   unsigned* bar = nullptr;  // [1]: a one-launch CG solve abandoned a wait
@@ -1104,7 +1104,7 @@ int solve_pressure(fsg_domain* h) {
   a.index_of = h->index_of;
   a.b = h->ap;
   a.xg = h->xg;
-  a.zx = reinterpret_cast<uint64_t*>(h->exch);
+  a.zx = h->exch;
   a.x64 = h->x64;
   a.slots = reinterpret_cast<uint64_t*>(h->partials);
   a.abort = h->bar + 1;
@@ -1336,7 +1336,7 @@ int fsg_create(fsg_domain** out, int32_t nx, int32_t ny, float length_x, float l
   ok &= dalloc(h, &h->ap, C) == hipSuccess;
   ok &= dalloc(h, &h->xg, C) == hipSuccess;
   ok &= dalloc(h, &h->pg0, C) == hipSuccess;
-  ok &= dalloc(h, &h->exch, 3 * C) == hipSuccess;
+  ok &= dalloc(h, &h->exch, C) == hipSuccess;
   ok &= dalloc(h, &h->x64, C) == hipSuccess;
   ok &= dalloc(h, &h->partials, (size_t)4 * 4096) == hipSuccess;
   ok &= dalloc(h, &h->bar, 16) == hipSuccess;

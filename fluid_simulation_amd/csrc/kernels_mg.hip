@@ -56,11 +56,13 @@ namespace fsg {
 
 namespace {
 
-constexpr int kT = 256;         // threads of the vector kernels and the level-0 tiles
+constexpr int kT = 256;         // threads of the vector kernels, and of a level-0 tile at 256
 // The tile levels below 0 of more tiles than this have a launch each (in either direction),
 // the others share k_mg_cycle: a task costs a draw of 12 ns from one counter and its polls,
 // so a level of 256 tiles is as fast by itself (1024^2: 661 us per step with the line at 64
-// tiles, 672 at 256; 2048^2: 1013, 1027 and, at 1024, 1108 us).
+// tiles, 672 at 256; 2048^2: 1013, 1027 and, at 1024, 1108 us; batches of 32 scenes of
+// 64 .. 190 cells a side: 754 at 64 and 742 at 512, of 256 scenes of 64 .. 512: 10,600,
+// 10,630 and, at 4096, 11,140).
 constexpr int kCycleTiles = 64;
 constexpr int kTileMany = 512;  // threads per tile of the former
 constexpr uint8_t kAct = kMgUnknown;  // info bit: the cell is an unknown
@@ -3567,7 +3569,7 @@ void launch_mg_down(hipStream_t s, MgHost& m, int l, int it, int max_iter, doubl
   // the stop test: level 0's kernel, or level 1's in the fused form (level 0 forms
   // the residual it tests)
   const int check = l == (m.fused ? 1 : 0) ? 1 : 0;
-  // level 0: m.l0_threads per tile (256 by default: many tiles); the others: few_tiles
+  // level 0: m.l0_threads per tile; the others: kTileMany
   if (l == 0) {
     // fused form: iteration it - 1's update, the buffers k_mg_xr would use then
     const MgXr xr = m.fused ? MgXr{m.x[(it + 1) & 1], m.x[it & 1], m.p[it & 1], m.b, m.part_pq,
