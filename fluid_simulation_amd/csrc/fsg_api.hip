@@ -394,7 +394,13 @@ int copy_out(fsg_domain* h, const HostCopy (&list)[N]) {
   bool through[N], any = false;
   for (size_t k = 0; k < N; ++k) {
     const HostCopy& c = list[k];
-    through[k] = c.host && staged(h, c);
+    // arrays that share memory with another of the call are written one after the other
+    bool apart = true;
+    for (size_t q = 0; q < N; ++q)
+      apart &= q == k || !list[q].host ||
+               (uintptr_t)list[q].host + list[q].bytes <= (uintptr_t)c.host ||
+               (uintptr_t)c.host + c.bytes <= (uintptr_t)list[q].host;
+    through[k] = c.host && apart && staged(h, c);
     if (through[k])
       any = true;
     else if (c.host && c.bytes > 0)
